@@ -23,6 +23,7 @@
 #include "ladder_common.hpp"
 #include "ladder_tune.hpp"
 #include "tri_solve.hpp"
+#include "zmma.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -79,6 +80,8 @@ __device__ __forceinline__ S to_storage(double2 x) {
 template <typename S, bool NT>
 __global__ void __launch_bounds__(256) blk_assemble_kernel(LadderArgs a, BlockedState<S> st, int item0, int nbatch) {
   const int b0 = blockIdx.y * ASM_QG;
+  if (a.nitems) nbatch = min(nbatch, *a.nitems - item0);
+  if (b0 >= nbatch) return;
   const int ng = min(ASM_QG, nbatch - b0);
   const int n = st.n, ncol = st.ncol, nv = a.nv, T = a.T;
   const int i0 = blockIdx.x * ASM_ROWS, r1 = min(n, i0 + ASM_ROWS);
@@ -96,7 +99,7 @@ __global__ void __launch_bounds__(256) blk_assemble_kernel(LadderArgs a, Blocked
   int wk[ASM_QG], qk[ASM_QG];
 #pragma unroll
   for (int k = 0; k < ASM_QG; ++k) {
-    const int item = item0 + b0 + min(k, ng - 1);
+    const int item = ladder_item(a, item0 + b0 + min(k, ng - 1));
     const int q = item % a.nq, w = (item / a.nq) % a.nw, chan = item / (a.nq * a.nw);
     Gk[k] = ladder_matrix_ptr(a, chan, w, q);
     Uk[k] = a.dense ? nullptr : a.u_r + chan * T * T;
@@ -280,6 +283,7 @@ __device__ __forceinline__ void panel_columns(S (&P)[RPT][NB], unsigned& done, P
 template <typename S, int NB, int RPT, int MAXTH>
 __global__ void __launch_bounds__(MAXTH) blk_panel_kernel(BlockedState<S> st, int p0, int slot) {
   const int b = blockIdx.x;
+  if (ladder_idle(st.src, st.item0 + b)) return;
   const int n = st.n, ld = st.ld;
   const int TH = blockDim.x;
   const int tid = threadIdx.x;
@@ -400,6 +404,7 @@ __global__ void __launch_bounds__(64) blk_rows_kernel(BlockedState<S> st, int p0
                                                       int l_hi, int flags, int ntile_a, int ntile, int nprob) {
   int b, tile;
   if (!xcd_tile(blockIdx.x, nprob, ntile, b, tile)) return;
+  if (ladder_idle(st.src, st.item0 + b)) return;
   const int n = st.n, ld = st.ld;
   S* W = st.W + static_cast<size_t>(b) * n * ld;
   const int nbw = (n - p0 < NB) ? n - p0 : NB;
@@ -546,6 +551,7 @@ __global__ void __launch_bounds__(256) blk_gemm_kernel(BlockedState<S> st, GemmR
   constexpr int TM = 16 * RI;
   int b, t;
   if (!xcd_tile(blockIdx.x, nprob, g.tiles_r * g.tiles_c, b, t)) return;
+  if (ladder_idle(st.src, st.item0 + b)) return;
   const int tr = t / g.tiles_c, tcl = t - (t / g.tiles_c) * g.tiles_c;
   const int ld = st.ld;
   S* W = st.W + static_cast<size_t>(b) * st.n * ld;
@@ -605,6 +611,89 @@ __global__ void __launch_bounds__(256) blk_gemm_kernel(BlockedState<S> st, GemmR
   }
 }
 
+// The complex128 update on the FP64 matrix cores (zmma.hpp): (32 MI) x 64 tiles, each wavefront
+// MI x 2 blocks of 16 x 16. The accumulators start from C and the A operand is staged negated. Rows
+// and columns past the edge are clamped (their results are not stored). Bound by the C tiles and panels
+// from HBM at a depth of 64. The whole factorisation at n = 720 (5642 problems) takes 199 ms with chunks of 8
+// (three workgroups per CU), 262 ms with chunks of 16 (two), and took 240 ms with 4x4-per-thread
+// vector-FMA tiles; at n = 120 (68442 problems) 34.4 against 38.3 ms.
+template <int MI, bool FUSED = false>
+__global__ void __launch_bounds__(256, MI == 2 ? 3 : 2) blk_gemm_f64_kernel(BlockedState<double2> st, GemmRange g, int nprob) {
+  constexpr int TM = 32 * MI, KC = 8;
+  int b, t;
+  if (!xcd_tile(blockIdx.x, nprob, g.tiles_r * g.tiles_c, b, t)) return;
+  if (ladder_idle(st.src, st.item0 + b)) return;
+  const int tr = t / g.tiles_c, tcl = t - (t / g.tiles_c) * g.tiles_c;
+  const int ld = st.ld;
+  double2* W = st.W + static_cast<size_t>(b) * st.n * ld;
+  const int rt = g.r0 + tr * TM, ct = g.c0 + tcl * 64;
+  __shared__ double2 s_a[TM][KC + 1];
+  __shared__ double2 s_b[KC][65];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = 16 * MI * (wave >> 1), wn = 32 * (wave & 1);
+  constexpr int LA = TM / 32;
+  const int ar = tid / KC, ak = tid % KC, bk = tid / 64, bc = tid % 64;
+  const double2* A[LA];
+#pragma unroll
+  for (int u = 0; u < LA; ++u) A[u] = W + static_cast<size_t>(min(rt + ar + 32 * u, g.r1 - 1)) * ld + g.k0 + ak;
+  const double2* B = W + static_cast<size_t>(g.k0 + bk) * ld + min(ct + bc, g.c1 - 1);
+  double2 ra[LA], rb[2];
+  auto load = [&](int kc) {
+    if (kc + KC <= g.kw) {
+#pragma unroll
+      for (int u = 0; u < LA; ++u) ra[u] = A[u][kc];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) rb[u] = B[static_cast<size_t>(kc + 4 * u) * ld];
+    } else {
+#pragma unroll
+      for (int u = 0; u < LA; ++u) ra[u] = kc + ak < g.kw ? A[u][kc] : make_double2(0.0, 0.0);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        rb[u] = kc + bk + 4 * u < g.kw ? B[static_cast<size_t>(kc + 4 * u) * ld] : make_double2(0.0, 0.0);
+    }
+  };
+  load(0);
+  ZmmaAcc<MI, 2> acc;
+  LadderSrc src{};
+  if constexpr (FUSED) src = ladder_src(st.src, st.item0 + b);
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const int r = min(rt + wm + 16 * i + zmma_row(lane, r4), g.r1 - 1);
+        const int c = min(ct + wn + 16 * j + (lane & 15), g.c1 - 1);
+        double2 x;
+        if constexpr (FUSED)
+          x = gemm_c_at<double2>(st, W, g, b, r, c, src, nullptr);
+        else
+          x = W[static_cast<size_t>(r) * ld + c];
+        acc.re[i][j][r4] = x.x;
+        acc.im[i][j][r4] = x.y;
+      }
+  for (int kc = 0; kc < g.kw; kc += KC) {
+#pragma unroll
+    for (int u = 0; u < LA; ++u) s_a[ar + 32 * u][ak] = make_double2(-ra[u].x, -ra[u].y);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) s_b[bk + 4 * u][bc] = rb[u];
+    __syncthreads();
+    if (kc + KC < g.kw) load(kc + KC);
+    zmma_chunk<MI, 2, TM, 64, KC>(acc, s_a, s_b, wm, wn, lane);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const int r = rt + wm + 16 * i + zmma_row(lane, r4), c = ct + wn + 16 * j + (lane & 15);
+        if (r < g.r1 && c < g.c1)
+          W[static_cast<size_t>(r) * ld + c] = make_double2(acc.re[i][j][r4], acc.im[i][j][r4]);
+      }
+}
+
 // Same update on the FP32 matrix cores: each wavefront owns a 32x32 quarter of the tile as
 // 2x2 blocks of 16x16, and a complex product becomes two real MFMA chains over the
 // interleaved k index (re/im): C_re -= [a_re, -a_im] . [b_re; b_im],
@@ -616,6 +705,7 @@ __global__ void __launch_bounds__(256) blk_gemm_mfma_kernel(BlockedState<float2>
   typedef float V4 __attribute__((ext_vector_type(4)));
   int b, t;
   if (!xcd_tile(blockIdx.x, nprob, g.tiles_r * g.tiles_c, b, t)) return;
+  if (ladder_idle(st.src, st.item0 + b)) return;
   const int tr = t / g.tiles_c, tcl = t - (t / g.tiles_c) * g.tiles_c;
   const int ld = st.ld;
   float2* W = st.W + static_cast<size_t>(b) * st.n * ld;
@@ -725,6 +815,7 @@ __global__ void __launch_bounds__(256) blk_gemm_bf16x3_kernel(BlockedState<float
   constexpr int KR = 2 * KC + 8;  // bf16 per staged row (interleaved re/im, padded)
   int b, t;
   if (!xcd_tile(blockIdx.x, nprob, g.tiles_r * g.tiles_c, b, t)) return;
+  if (ladder_idle(st.src, st.item0 + b)) return;
   const int tr = t / g.tiles_c, tcl = t - (t / g.tiles_c) * g.tiles_c;
   const int ld = st.ld;
   float2* W = st.W + static_cast<size_t>(b) * st.n * ld;
@@ -923,24 +1014,21 @@ __global__ void __launch_bounds__(256) blk_gemm_bf16x3_kernel(BlockedState<float
     }
 }
 
-__global__ void blk_info_kernel(const int* __restrict__ st_info, int32_t* __restrict__ info, int item0, int nitems) {
+__global__ void blk_info_kernel(LadderArgs a, const int* __restrict__ st_info, int item0, int nitems) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < nitems) info[item0 + b] = st_info[b];
+  if (b < nitems && !ladder_idle(a, item0 + b)) a.info[ladder_item(a, item0 + b)] = st_info[b];
 }
 
-int blocked_copy_info(const int* st_info, int32_t* info, int item0, int nitems, hipStream_t stream) {
-  if (!info) return 0;
-  hipLaunchKernelGGL(blk_info_kernel, dim3(ceil_div(nitems, 256)), dim3(256), 0, stream, st_info, info, item0, nitems);
+int blocked_copy_info(const LadderArgs& a, const int* st_info, int item0, int nitems, hipStream_t stream) {
+  if (!a.info) return 0;
+  hipLaunchKernelGGL(blk_info_kernel, dim3(ceil_div(nitems, 256)), dim3(256), 0, stream, a, st_info, item0, nitems);
   DGAMI_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
 // ---------------------------------------------------------------------------
 // Complex64 trailing updates run on the FP32 matrix cores; DGAMI_BLOCKED_GEMM=vector selects
-// the vector-FMA tile kernel instead (for comparisons). Complex128 updates always use the
-// vector-FMA kernel: the FP64 MFMA (v_mfma_f64_16x16x4_f64) returned wrong products on
-// gfx950 when the compiler rewrote its source registers right after issue, which source
-// code cannot prevent.
+// the vector-FMA tile kernel instead (for comparisons). Complex128 updates run on the FP64 matrix cores.
 // The first outer block takes over the assembly of its trailing rows unless DGAMI_LADDER_FUSE=0.
 static bool ladder_fuse_enabled() {
   const char* v = getenv("DGAMI_LADDER_FUSE");
@@ -982,8 +1070,8 @@ struct BlockedSteps {
     if (r1 <= r0 || c1 <= c0 || kw <= 0) return 0;
     int mode = BLK_GEMM_VECTOR;
     if constexpr (std::is_same<S, float2>::value) mode = use_vector_gemm() ? BLK_GEMM_VECTOR : st.gemm_mode;
-    // update tiles are 64 x 64; complex128 variants with tall_tiles use 128 x 64 (8 rows per
-    // thread) for updates of more than 96 rows. Measured at n = 720 (5642 problems) the 64-row
+    // update tiles are 64 x 64; complex128 variants with tall_tiles use 128 x 64 for updates of more
+    // than 96 rows. Measured at n = 720 (5642 problems) the 64-row
     // tiles are 8% faster over the whole factorisation (more workgroups per CU), and at n = 120
     // a 128-row tile over the short updates is mostly empty.
     constexpr bool c128 = std::is_same<S, double2>::value;
@@ -999,14 +1087,14 @@ struct BlockedSteps {
       if constexpr (c128) {
         if (tall) {
           if (fused)
-            hipLaunchKernelGGL((blk_gemm_kernel<S, 16, 8, true>), gd, dim3(256), 0, stream, st, g, nb);
+            hipLaunchKernelGGL((blk_gemm_f64_kernel<4, true>), gd, dim3(256), 0, stream, st, g, nb);
           else
-            hipLaunchKernelGGL((blk_gemm_kernel<S, 16, 8>), gd, dim3(256), 0, stream, st, g, nb);
+            hipLaunchKernelGGL((blk_gemm_f64_kernel<4>), gd, dim3(256), 0, stream, st, g, nb);
         } else {
           if (fused)
-            hipLaunchKernelGGL((blk_gemm_kernel<S, 16, 4, true>), gd, dim3(256), 0, stream, st, g, nb);
+            hipLaunchKernelGGL((blk_gemm_f64_kernel<2, true>), gd, dim3(256), 0, stream, st, g, nb);
           else
-            hipLaunchKernelGGL((blk_gemm_kernel<S, 16, 4>), gd, dim3(256), 0, stream, st, g, nb);
+            hipLaunchKernelGGL((blk_gemm_f64_kernel<2>), gd, dim3(256), 0, stream, st, g, nb);
         }
       } else {
         if (fused)
@@ -1204,12 +1292,14 @@ int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream) {
     if (rc) return rc;
     // back substitution on the carried right-hand sides, x / beta straight to the output
     TriFactors<double2> f{L.st.W, L.tri, L.st.dinv, n, ld, nblk};
+    f.nitems = a.nitems;
+    f.item0 = static_cast<int>(item0);
     rc = tri_diag_inverse(f, nb, false, L.s);
     if (rc) return rc;
     TriVec<double2> y{L.st.W + n, static_cast<size_t>(n) * ld, ld};
     rc = tri_backward(f, nb, a.T, y, TriVec<double2>{nullptr, 0, 0}, &a, static_cast<int>(item0), L.s);
     if (rc) return rc;
-    rc = blocked_copy_info(L.st.info, a.info, static_cast<int>(item0), nb, L.s);
+    rc = blocked_copy_info(a, L.st.info, static_cast<int>(item0), nb, L.s);
     if (rc) return rc;
   }
   for (int l = 1; l < nl; ++l) {

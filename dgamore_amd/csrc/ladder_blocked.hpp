@@ -12,7 +12,7 @@ constexpr int BLK_MAX_N = 1536;                     // largest compound size of 
 constexpr int BLK_MAP_STRIDE = 3 * BLK_MAX_NB + 1;  // ints of one problem's interchange map
 constexpr int BLK_PANELS = 8;                       // most register panels per outer block (trailing-update depth)
 
-// Trailing-update kernels of the complex64 factorisation (complex128 always uses vector FMA).
+// Trailing-update kernels of the complex64 factorisation (complex128 uses the FP64 matrix cores).
 enum BlockedGemm { BLK_GEMM_VECTOR = 0, BLK_GEMM_F32_MFMA = 1, BLK_GEMM_BF16X3 = 2 };
 
 template <typename S>
@@ -91,7 +91,7 @@ int blocked_gemm_fp64(BlockedState<double2>& st, int nb, int r0, int r1, int c0,
 int blocked_gemm_c64(BlockedState<float2>& st, int nb, int r0, int r1, int c0, int c1, int k0, int kw,
                      hipStream_t stream);
 
-// info[item0 + b] = first zero pivot of problem b of the batch (no-op for info == nullptr).
-int blocked_copy_info(const int* st_info, int32_t* info, int item0, int nitems, hipStream_t stream);
+// a.info of work index item0 + b = first zero pivot of problem b of the batch (no-op without info).
+int blocked_copy_info(const LadderArgs& a, const int* st_info, int item0, int nitems, hipStream_t stream);
 
 }  // namespace dgami

@@ -41,8 +41,10 @@ template <int NW, int RS, int CS>
 __global__ void __launch_bounds__(NW * 64) ladder_col_kernel(LadderArgs a) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const int q = blockIdx.x % a.nq;
-  const int rest = blockIdx.x / a.nq;
+  if (ladder_idle(a, blockIdx.x)) return;
+  const int item = ladder_item(a, blockIdx.x);
+  const int q = item % a.nq;
+  const int rest = item / a.nq;
   const int w = rest % a.nw;
   const int chan = rest / a.nw;
   const int n = a.n, T = a.T, ncol = n + T;

@@ -23,7 +23,15 @@ struct LadderArgs {
   // CHI0INV / VERTEX right-hand sides restricted to the columns (c, v') with v' in
   // [rhs_vlo, rhs_vlo + rhs_w) for every orbital pair c (rhs_w = 0: every column)
   int rhs_vlo = 0, rhs_w = 0;
+  // LU of a subset: work index k < *nitems stands for problem items[k]; kernels launched for more
+  // problems than the device count return at once (null: every problem, k itself)
+  const int* items = nullptr;
+  const int* nitems = nullptr;
 };
+
+// Problem of work index k, and whether k lies beyond the subset.
+__device__ __forceinline__ int ladder_item(const LadderArgs& a, int k) { return a.items ? a.items[k] : k; }
+__device__ __forceinline__ bool ladder_idle(const LadderArgs& a, int k) { return a.nitems && k >= *a.nitems; }
 
 // Compound column of right-hand side r (CHI0INV / VERTEX modes).
 __device__ __forceinline__ int ladder_rhs_col(const LadderArgs& a, int r) {
@@ -104,7 +112,8 @@ struct LadderSrc {
   int w, q;
 };
 
-__device__ __forceinline__ LadderSrc ladder_src(const LadderArgs& a, int item) {
+__device__ __forceinline__ LadderSrc ladder_src(const LadderArgs& a, int k) {
+  const int item = ladder_item(a, k);
   const int q = item % a.nq, w = (item / a.nq) % a.nw, chan = item / (a.nq * a.nw);
   LadderSrc s;
   s.G = ladder_matrix_ptr(a, chan, w, q);

@@ -25,6 +25,7 @@ __device__ __forceinline__ float2 cone<float2>() {
 template <typename S>
 __global__ void __launch_bounds__(64) tri_diag_inverse_kernel(TriFactors<S> f, int need_lower) {
   const int kb = blockIdx.x, b = blockIdx.y;
+  if (f.nitems && f.item0 + b >= *f.nitems) return;
   const int c0 = kb * TRI_B;
   const int cb = min(TRI_B, f.n - c0);
   const int tid = threadIdx.x;
@@ -94,6 +95,7 @@ __device__ __forceinline__ void tri_sweep_body(const TriFactors<S>& f, const Tri
                                                const LadderArgs& la, int item0) {
   const int b = blockIdx.x;
   if (f.skip && f.skip[b] != 0) return;
+  if (f.nitems && f.item0 + b >= *f.nitems) return;
   const int tid = threadIdx.x;
   const int n = f.n;
   __shared__ S s_d[TRI_B][TRI_B + 1];
@@ -172,7 +174,7 @@ __device__ __forceinline__ void tri_sweep_body(const TriFactors<S>& f, const Tri
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       if constexpr (TO_LADDER) {
-        const int item = item0 + b;
+        const int item = ladder_item(la, item0 + b);
         const int q = item % la.nq, w = (item / la.nq) % la.nw, chan = item / (la.nq * la.nw);
         la.out[ladder_out_index(la, chan, w, q, r, t)] = cscale(to_c128(yr[m][t]), la.inv_beta);
       } else {

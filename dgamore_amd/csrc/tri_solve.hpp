@@ -24,6 +24,8 @@ struct TriFactors {
   const double2* dinv; // [batch][n] inverse pivots (diagonal of U^-1)
   int n, ld, nblk;
   const int* skip = nullptr;  // [batch] or null: the sweeps leave problems with skip[b] != 0 untouched
+  const int* nitems = nullptr;  // device count or null: problems item0 + b >= *nitems are left out
+  int item0 = 0;
 };
 
 // Right-hand-side block [batch][n][T] addressed with a row stride (elements) and an item stride.

@@ -335,7 +335,7 @@ static int vertex_solve_t(LadderArgs a, int what, const VertexArgs& o_in, int ge
 #undef DGAMI_VTX_FULL
     }
     DGAMI_HIP_CHECK(hipGetLastError());
-    rc = blocked_copy_info(st.info, a.info, static_cast<int>(item0), nb, stream);
+    rc = blocked_copy_info(a, st.info, static_cast<int>(item0), nb, stream);
     if (rc) return rc;
   }
   for (int l = 1; l < nl; ++l) {

@@ -16,56 +16,72 @@ struct ZgemmArgs {
   long long sa, sb, sc;  // batch strides
   double2 alpha, beta;
   const int* active = nullptr;  // [batch] or null: batch entries with active[b] == 0 are skipped
+  const int* tile_active = nullptr;  // [batch][column tiles] or null: tiles of ZG_TN columns with 0 are skipped
 };
 
-constexpr int ZG_TM = 64, ZG_TN = 64, ZG_TK = 16;
-static_assert(ZG_TM * ZG_TK == 4 * 256 && ZG_TK * ZG_TN == 4 * 256, "four operand elements per thread");
+constexpr int ZG_TM = 64, ZG_TN = 64, ZG_TK = 8;
+static_assert(ZG_TM * ZG_TK == 2 * 256 && ZG_TK * ZG_TN == 2 * 256, "two operand elements per thread");
 
 // grid: xcd_grid(batch, tiles_m * tiles_n); block 256 (all tiles of one batch entry on one XCD). Each
-// wavefront owns a 32 x 32 quarter of the tile. Bound by the FP64 matrix cores (zmma.hpp): the
-// refinement's residual products 4.90 -> 3.85 ms, the double-counting product 2.5 -> 2.0 ms.
-static __global__ void __launch_bounds__(256) zgemm_kernel(ZgemmArgs g, int batch, int tiles_n, int tiles_m) {
+// wavefront owns a 32 x 32 quarter of the tile. Bound by the FP64 matrix cores (zmma.hpp). Rows and
+// columns past the edge are clamped, not predicated (their results are not stored; a per-load
+// predicate cost 8%), and only the last k-chunk zeroes its tail. Measured on 62 products of 768 x 832
+// x 768: chunks of 8 at three workgroups per CU 3.76 ms (64.8 TF/s), of 16 3.84, of 32 3.93; the
+// vector-FMA tile ran at 32 TF/s.
+// THREE: complex products from three real ones, (re, im) = (t1 - t2, t3 - t1 - t2) with t1 = re re,
+// t2 = im im, t3 = (re + im)(re + im): a quarter fewer matrix instructions (3.12 ms), with an error
+// bounded by |A| |B| instead of per part (for the products of an iteration whose residual is formed
+// apart). Chunks of 16 left it one workgroup per CU (4.22 ms).
+template <bool THREE>
+static __global__ void __launch_bounds__(256, THREE ? 2 : 3) zgemm_kernel(ZgemmArgs g, int batch, int tiles_n, int tiles_m) {
   int b, t;
   if (!xcd_tile(blockIdx.x, batch, tiles_m * tiles_n, b, t)) return;
   if (g.active && g.active[b] == 0) return;
-  const double2* A = g.A + b * g.sa;
-  const double2* B = g.B + b * g.sb;
-  double2* C = g.C + b * g.sc;
   const int tm = t / tiles_n, tn = t - (t / tiles_n) * tiles_n;
+  if (g.tile_active && g.tile_active[b * tiles_n + tn] == 0) return;
   const int m0 = tm * ZG_TM, n0 = tn * ZG_TN;
   __shared__ double2 s_a[ZG_TM][ZG_TK + 1];
   __shared__ double2 s_b[ZG_TK][ZG_TN + 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = 32 * (wave >> 1), wn = 32 * (wave & 1);
-  ZmmaAcc<2, 2> acc;
-  zmma_zero(acc);
-  // the next k-tile's operands are loaded into registers while the current one is used
-  double2 ra[4], rb[4];
-  auto load = [&](int k0) {
+  // thread: element (ar + 32 u, ak) of the A chunk and (bk + 4 u, bc) of the B chunk
+  const int ar = tid / ZG_TK, ak = tid % ZG_TK, bk = tid / ZG_TN, bc = tid % ZG_TN;
+  const double2* A[2];
+  const double2* B = g.B + b * g.sb + static_cast<size_t>(bk) * g.ldb + min(n0 + bc, g.N - 1);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e = tid + 256 * u;
-      const int r = e / ZG_TK, s = e % ZG_TK;
-      ra[u] = (m0 + r < g.M && k0 + s < g.K) ? A[static_cast<size_t>(m0 + r) * g.lda + k0 + s]
-                                              : make_double2(0.0, 0.0);
-      const int s2 = e / ZG_TN, c = e % ZG_TN;
-      rb[u] = (k0 + s2 < g.K && n0 + c < g.N) ? B[static_cast<size_t>(k0 + s2) * g.ldb + n0 + c]
-                                               : make_double2(0.0, 0.0);
+  for (int u = 0; u < 2; ++u) A[u] = g.A + b * g.sa + static_cast<size_t>(min(m0 + ar + 32 * u, g.M - 1)) * g.lda + ak;
+  ZmmaAcc<2, 2, THREE> acc;
+  zmma_zero(acc);
+  // the next k-chunk's operands are loaded into registers while the current one is used
+  double2 ra[2], rb[2];
+  auto load = [&](int k0) {
+    if (k0 + ZG_TK <= g.K) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        ra[u] = A[u][k0];
+        rb[u] = B[static_cast<size_t>(k0 + 4 * u) * g.ldb];
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        ra[u] = k0 + ak < g.K ? A[u][k0] : make_double2(0.0, 0.0);
+        rb[u] = k0 + bk + 4 * u < g.K ? B[static_cast<size_t>(k0 + 4 * u) * g.ldb] : make_double2(0.0, 0.0);
+      }
     }
   };
   load(0);
   for (int k0 = 0; k0 < g.K; k0 += ZG_TK) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e = tid + 256 * u;
-      s_a[e / ZG_TK][e % ZG_TK] = ra[u];
-      s_b[e / ZG_TN][e % ZG_TN] = rb[u];
+    for (int u = 0; u < 2; ++u) {
+      s_a[ar + 32 * u][ak] = ra[u];
+      s_b[bk + 4 * u][bc] = rb[u];
     }
     __syncthreads();
     if (k0 + ZG_TK < g.K) load(k0 + ZG_TK);
     zmma_chunk<2, 2, ZG_TM, ZG_TN, ZG_TK>(acc, s_a, s_b, wm, wn, lane);
     __syncthreads();
   }
+  double2* C = g.C + b * g.sc;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -75,18 +91,19 @@ static __global__ void __launch_bounds__(256) zgemm_kernel(ZgemmArgs g, int batc
         const int r = m0 + wm + 16 * i + zmma_row(lane, r4), c = n0 + wn + 16 * j + (lane & 15);
         if (r >= g.M || c >= g.N) continue;
         double2* e = C + static_cast<size_t>(r) * g.ldc + c;
-        double2 val = cmul(g.alpha, make_double2(acc.re[i][j][r4], acc.im[i][j][r4]));
+        double2 val = cmul(g.alpha, zmma_value(acc, i, j, r4));
         if (g.beta.x != 0.0 || g.beta.y != 0.0) val = cfma(val, g.beta, *e);
         *e = val;
       }
 }
 
+template <bool THREE = false>
 inline int launch_zgemm(const ZgemmArgs& g, int batch, hipStream_t stream) {
   if (g.M <= 0 || g.N <= 0 || batch <= 0) return 0;
   const int tn = ceil_div(g.N, ZG_TN), tm = ceil_div(g.M, ZG_TM);
   const size_t grid = xcd_grid(batch, static_cast<size_t>(tn) * tm);
   DGAMI_ARG_CHECK(grid < (size_t(1) << 31), "zgemm: grid too large");
-  hipLaunchKernelGGL(zgemm_kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, g, batch, tn, tm);
+  hipLaunchKernelGGL((zgemm_kernel<THREE>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, g, batch, tn, tm);
   DGAMI_HIP_CHECK(hipGetLastError());
   return 0;
 }
