@@ -9,6 +9,7 @@
 #include "dgami_internal.hpp"
 #include "dgami_launch.hpp"
 #include "ladder_common.hpp"
+#include "ladder_shared.hpp"
 #include "ladder_tune.hpp"
 
 namespace dgami {
@@ -44,6 +45,7 @@ int ladder_solve_fp64(const LadderArgs& a, hipStream_t stream) {
     const int v = ladder_col_variant(a.n, a.T);
     if (v >= 0) return ladder_col_launch(v, a, stream);
   }
+  if (f.empty() && ladder_shared_applies(a)) return ladder_solve_shared(a, stream);
   if (f.empty()) {
     const int tuned = ladder_tuned_kernel(a.n, a.T, DGAMI_PLAIN_FP64);
     if (tuned >= 0) {

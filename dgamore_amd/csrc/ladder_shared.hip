@@ -1,0 +1,711 @@
+// Ladder sums through the part of the matrix that the q-points of a (channel, w) group share.
+//
+// A(q) = chi0^-1(q) delta_vv' + (Gamma - U_r - V_r(q)) / beta^2. Gamma, by far the largest part, is
+// the same for every q of a group, and chi0^-1(q) differs little from its mean over q. With
+//   A0 = mean_q A(q),   D(q) = A(q) - A0   (blocks of nb^2 x nb^2 on the v = v' diagonal, and a
+//                                           rank-nb^2 term of V_r(q) - mean V_r),
+// and P = A0^-1 formed once per group, P A(q) = 1 + P D(q) is close to 1 (spectral radius of P D(q)
+// 0.01 ... 0.8 on the synthetic models of 1 to 3 orbitals, beta = 5 ... 40, U = 2 ... 8), and every
+// column of every q is solved by GMRES on it. One iteration of all q and right-hand sides of a
+// group is one n x n by n x (nq nb^2) product on the matrix cores plus one pass over the Krylov
+// basis, where the LU factors an own n x n matrix for every q: at n = 720 and 91 q-points 15
+// products of 3.4 GF per group against 91 factorisations of 1.0 GF that stream 47.8 GB.
+//
+// Each cycle runs up to SH_M iterations from the residual of the current X, B - A0 X - D(q) X, formed
+// in FP64 from A0 and D(q) themselves, so the error of P only slows the convergence down; X ends as
+// an LU solution with a step of iterative refinement does. Every column has its own Hessenberg matrix and
+// status on the device; tiles of 64 columns (SH_TN) without an active column are skipped by the
+// products and the basis kernels, and no value is read by the host, so a call can be captured.
+// Problems with a column that does not converge (a singular or nearly singular A(q), a NaN) are
+// collected on the device and solved by the LU with partial pivoting, whose info they report.
+#include <algorithm>
+#include <cstdlib>
+#include <string>
+#include <type_traits>
+
+#include "dgami.h"
+#include "dgami_internal.hpp"
+#include "dgami_launch.hpp"
+#include "ladder_common.hpp"
+#include "ladder_shared.hpp"
+#include "zgemm.hpp"
+
+namespace dgami {
+
+int ladder_col_variant(int n, int nrhs);
+int ladder_col_launch(int variant, const LadderArgs& a, hipStream_t stream);
+int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream);
+
+constexpr int SH_M = 10;           // Krylov vectors of a cycle
+constexpr int SH_TN = ZG_TN;       // columns of a workgroup, and of a tile of the products
+constexpr int SH_WAVES = 4;        // wavefronts of a workgroup, which share the rows of its columns
+constexpr int SH_ROT = SH_M * (SH_M + 1) / 2;
+
+// A cycle stops a column at a residual of SH_CYCLE_TOL of its start (below that the error of P
+// decides); the column is done when its residual is below SH_DONE_TOL of |X|.
+constexpr int SH_CYCLES = 4;
+constexpr double SH_CYCLE_TOL = 1e-10;
+constexpr double SH_DONE_TOL = 2e-16;
+// A cycle that leaves more than this of its residual is stagnating.
+constexpr double SH_STAGNATION = 0.3;
+
+enum SharedState { SH_RUN = 0, SH_DONE = 1, SH_FAIL = 2 };
+
+struct SharedArgs {
+  LadderArgs a;
+  int group0, groups;     // groups of this batch
+  int N, ntile;           // columns (q, t) of a group, tiles of SH_TN columns
+  size_t cols;            // columns of the batch
+  const double2* P;       // [groups][n][n]
+  const double2* dd;      // D(q): [nw][T*T][nv][nq]
+  const double2* dv;      // (V_r(q) - mean V_r) / beta^2: [nchan][nq][T*T], or null
+  const double2* z0;      // P B [groups][n][T]
+  double2* V;             // [SH_M + 1][groups][n][N] Krylov basis
+  double2* u;             // operand of the products [groups][n][N]
+  double2* g;             // their result
+  double2* X;             // solution
+  double2* sums;          // [groups][T][N] sums over v of the vector D(q) is applied to (with dv)
+  // per column, column fastest
+  double* rc;             // [SH_M] rotations
+  double2* rs;
+  double2* R;             // [SH_ROT] triangular factor, column j at j (j + 1) / 2
+  double2* gv;            // [SH_M + 1] rotated residual
+  double* beta0;
+  double* target;
+  double* xnorm;
+  int* kdim;              // vectors of the current cycle
+  int* state;             // SharedState
+  int* live;              // 1 while the column iterates in the current cycle
+  int* tile_run;          // [groups][ntile] 1 while the tile has a running column
+  int* tile_live;         // [groups][ntile] 1 while the tile has a column iterating in this cycle
+};
+
+// ---------------------------------------------------------------------------
+// D(q) = chi0^-1(q) - mean over q and the mean, one wavefront per (w, block, v).
+__global__ void __launch_bounds__(256) shared_mean_kernel(const double2* __restrict__ ci, double2* __restrict__ mean,
+                                                          double2* __restrict__ dd, int rows, int nq) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= rows) return;
+  const double2* src = ci + static_cast<size_t>(row) * nq;
+  double2 s = make_double2(0.0, 0.0);
+  for (int q = lane; q < nq; q += 64) s = cadd(s, src[q]);
+  for (int o = 32; o > 0; o >>= 1) s = cadd(s, make_double2(__shfl_xor(s.x, o), __shfl_xor(s.y, o)));
+  s = cscale(s, 1.0 / nq);
+  for (int q = lane; q < nq; q += 64) dd[static_cast<size_t>(row) * nq + q] = csub(src[q], s);
+  if (lane == 0) mean[row] = s;
+}
+
+// The same for V_r [nchan][nq][T*T]: one wavefront per (chan, block); dv is scaled by 1 / beta^2.
+__global__ void __launch_bounds__(64) shared_vmean_kernel(LadderArgs a, double2* __restrict__ mean,
+                                                          double2* __restrict__ dv) {
+  const int TT = a.T * a.T, chan = blockIdx.x / TT, e = blockIdx.x - chan * TT, lane = threadIdx.x;
+  const double2* src = a.v_r + static_cast<size_t>(chan) * a.nq * TT + e;
+  double2 s = make_double2(0.0, 0.0);
+  for (int q = lane; q < a.nq; q += 64) s = cadd(s, src[static_cast<size_t>(q) * TT]);
+  for (int o = 32; o > 0; o >>= 1) s = cadd(s, make_double2(__shfl_xor(s.x, o), __shfl_xor(s.y, o)));
+  s = cscale(s, 1.0 / a.nq);
+  double2* dst = dv + static_cast<size_t>(chan) * a.nq * TT + e;
+  for (int q = lane; q < a.nq; q += 64)
+    dst[static_cast<size_t>(q) * TT] = cscale(csub(src[static_cast<size_t>(q) * TT], s), a.inv_beta2);
+  if (lane == 0) mean[blockIdx.x] = s;
+}
+
+// A0 of the groups [g0, g0 + groups): grid (ceil(n*n/256), groups).
+__global__ void __launch_bounds__(256) shared_matrix_kernel(LadderArgs a, const double2* __restrict__ mean,
+                                                            const double2* __restrict__ vmean,
+                                                            double2* __restrict__ A0, int g0) {
+  const size_t nn = static_cast<size_t>(a.n) * a.n;
+  const size_t e = blockIdx.x * static_cast<size_t>(256) + threadIdx.x;
+  if (e >= nn) return;
+  const int grp = g0 + blockIdx.y, chan = grp / a.nw, w = grp - chan * a.nw;
+  const int i = static_cast<int>(e / a.n), j = static_cast<int>(e - static_cast<size_t>(i) * a.n);
+  const int ri = i / a.nv, vi = i - ri * a.nv, cj = j / a.nv, vj = j - cj * a.nv;
+  double2 uv = a.u_r[chan * a.T * a.T + ri * a.T + cj];
+  if (vmean) uv = cadd(uv, vmean[chan * a.T * a.T + ri * a.T + cj]);
+  double2 x = cscale(csub(a.gamma[grp * nn + e], uv), a.inv_beta2);
+  if (vi == vj) x = cadd(x, mean[(static_cast<size_t>(w) * a.T * a.T + ri * a.T + cj) * a.nv + vi]);
+  A0[blockIdx.y * nn + e] = x;
+}
+
+// z0 = P B: sums of P over the frequencies of every orbital pair. One wavefront per (group, row).
+__global__ void __launch_bounds__(256) shared_rhs_kernel(const double2* __restrict__ P, double2* __restrict__ z0, int rows,
+                                                         int n, int T, int nv) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= rows) return;
+  for (int t = 0; t < T; ++t) {
+    const double2* src = P + static_cast<size_t>(row) * n + t * nv;
+    double2 s = make_double2(0.0, 0.0);
+    for (int v = lane; v < nv; v += 64) s = cadd(s, src[v]);
+    for (int o = 32; o > 0; o >>= 1) s = cadd(s, make_double2(__shfl_xor(s.x, o), __shfl_xor(s.y, o)));
+    if (lane == 0) z0[static_cast<size_t>(row) * T + t] = s;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Workgroups of the kernels below: one tile of SH_TN columns of one group; thread (wave, lane) owns
+// column `lane` of the tile and the rows i = wave + SH_WAVES k, so that a row of the tile is one 1 KiB
+// run. They are bound by the reads of the basis.
+struct SharedTile {
+  int grp, e, q, t, wave, lane;  // batch-local group, column (clamped), its q and right-hand side
+  bool in;
+  size_t base, col;              // offset of the column in a [groups][n][N] vector, column of the batch
+};
+
+__device__ __forceinline__ SharedTile shared_tile(const SharedArgs& s) {
+  SharedTile x;
+  x.grp = blockIdx.x / s.ntile;
+  const int tile = blockIdx.x - x.grp * s.ntile;
+  x.lane = threadIdx.x & 63;
+  x.wave = threadIdx.x >> 6;
+  const int e = tile * SH_TN + x.lane;
+  x.in = e < s.N;
+  x.e = x.in ? e : s.N - 1;
+  x.q = x.e / s.a.T;
+  x.t = x.e - x.q * s.a.T;
+  x.base = static_cast<size_t>(x.grp) * s.a.n * s.N + x.e;
+  x.col = static_cast<size_t>(x.grp) * s.N + x.e;
+  return x;
+}
+
+// Sum over the wavefronts of a workgroup of one value per column.
+__device__ __forceinline__ double2 wave_sum(double2 (&sh)[SH_WAVES][SH_TN], double2 v, const SharedTile& x) {
+  __syncthreads();
+  sh[x.wave][x.lane] = v;
+  __syncthreads();
+  double2 r = sh[0][x.lane];
+#pragma unroll
+  for (int k = 1; k < SH_WAVES; ++k) r = cadd(r, sh[k][x.lane]);
+  return r;
+}
+
+// D(q) of a column's frequency-diagonal part for nb = 1 (row i = v).
+__device__ __forceinline__ const double2* shared_diag(const SharedArgs& s, const SharedTile& x) {
+  const int w = (s.group0 + x.grp) % s.a.nw;
+  return s.dd + static_cast<size_t>(w) * s.a.n * s.a.nq + x.q;
+}
+
+// Start of a cycle: b = z0 (first) or P r (in s.g); V_0 = b / |b| and the column's state. DIAG
+// (one orbital, no V_r): u = D(q) V_0 here too.
+template <bool DIAG>
+__global__ void __launch_bounds__(256) shared_start_kernel(SharedArgs s, int first) {
+  const int tile_id = blockIdx.x;
+  if (!first && s.tile_run[tile_id] == 0) return;
+  __shared__ double2 sh[SH_WAVES][SH_TN];
+  const SharedTile x = shared_tile(s);
+  const int n = s.a.n;
+  const double2* b = first ? s.z0 + static_cast<size_t>(x.grp) * n * s.a.T + x.t : s.g + x.base;
+  const size_t stride = first ? s.a.T : s.N;
+  double nrm = 0.0;
+#pragma unroll 4
+  for (int i = x.wave; i < n; i += SH_WAVES) {
+    const double2 y = b[i * stride];
+    nrm = fma(y.x, y.x, fma(y.y, y.y, nrm));
+  }
+  nrm = sqrt(wave_sum(sh, make_double2(nrm, 0.0), x).x);
+  const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
+  const double2* dd = shared_diag(s, x);
+#pragma unroll 4
+  for (int i = x.wave; i < n; i += SH_WAVES) {
+    const double2 v = cscale(b[i * stride], inv);
+    const size_t o = x.base + static_cast<size_t>(i) * s.N;
+    if (x.in) s.V[o] = v;
+    if constexpr (DIAG) {
+      if (x.in) s.u[o] = cmul(dd[static_cast<size_t>(i) * s.a.nq], v);
+    }
+  }
+  if (x.wave == 0) {
+    int st = first ? SH_RUN : s.state[x.col];
+    const double xn = first ? nrm : s.xnorm[x.col];
+    if (!(nrm <= 1e300)) st = SH_FAIL;  // infinite or NaN
+    if (st == SH_RUN && nrm <= SH_DONE_TOL * xn) st = SH_DONE;
+    const int live = x.in && st == SH_RUN;
+    if (x.in) {
+      s.state[x.col] = st;
+      s.live[x.col] = live;
+      s.beta0[x.col] = nrm;
+      s.target[x.col] = fmax(SH_CYCLE_TOL * nrm, SH_DONE_TOL * xn);
+      s.kdim[x.col] = 0;
+      s.gv[x.col] = make_double2(nrm, 0.0);
+    }
+    const unsigned long long any = __ballot(live);
+    if (x.lane == 0) s.tile_live[tile_id] = any != 0;
+  }
+}
+
+// Iteration k: w = P u (in s.g) is orthogonalised against V_0 .. V_k (KC = k + 1 rounded up to even;
+// the pointer of an index beyond k is that of V_k and its coefficient 0), V_(k+1) is written (with
+// DIAG u = D(q) V_(k+1) too), and the column's Hessenberg matrix (1 + P D(q) projected) and
+// residual are updated. |w - projection| comes from |w|^2 - sum |h|^2: w = P D(q) V_k itself is
+// orthogonalised, not V_k + w, so little cancels, and V and the Hessenberg matrix stay consistent.
+template <bool DIAG, int KC>
+__global__ void __launch_bounds__(256) shared_step_kernel(SharedArgs s, int k) {
+  const int tile_id = blockIdx.x;
+  if (s.tile_live[tile_id] == 0) return;
+  __shared__ double2 sh[SH_WAVES][SH_TN];
+  const SharedTile x = shared_tile(s);
+  const int n = s.a.n, N = s.N;
+  const size_t vec = static_cast<size_t>(s.groups) * n * N;
+  const double2* Vp[KC];
+#pragma unroll
+  for (int j = 0; j < KC; ++j) Vp[j] = s.V + static_cast<size_t>(j <= k ? j : k) * vec + x.base;
+  const double2* w = s.g + x.base;
+  double2 h[KC];
+#pragma unroll
+  for (int j = 0; j < KC; ++j) h[j] = make_double2(0.0, 0.0);
+  double nrm = 0.0;
+#pragma unroll 2
+  for (int i = x.wave; i < n; i += SH_WAVES) {
+    const size_t o = static_cast<size_t>(i) * N;
+    const double2 y = w[o];
+    double2 p[KC];
+#pragma unroll
+    for (int j = 0; j < KC; ++j) p[j] = Vp[j][o];
+    nrm = fma(y.x, y.x, fma(y.y, y.y, nrm));
+#pragma unroll
+    for (int j = 0; j < KC; ++j) h[j] = cfma(h[j], cconj(p[j]), y);
+  }
+  nrm = wave_sum(sh, make_double2(nrm, 0.0), x).x;
+  double left = nrm;
+#pragma unroll
+  for (int j = 0; j < KC; ++j) {
+    h[j] = wave_sum(sh, h[j], x);
+    if (j > k) h[j] = make_double2(0.0, 0.0);
+    left -= h[j].x * h[j].x + h[j].y * h[j].y;
+  }
+  const double hn = sqrt(fmax(left, 0.0));
+  const double inv = hn > 1e-150 ? 1.0 / hn : 0.0;
+  const double2* dd = shared_diag(s, x);
+  double2* Vn = s.V + static_cast<size_t>(k + 1) * vec + x.base;
+  double2* un = s.u + x.base;
+#pragma unroll 2
+  for (int i = x.wave; i < n; i += SH_WAVES) {
+    const size_t o = static_cast<size_t>(i) * N;
+    double2 y = w[o];
+    double2 p[KC];
+#pragma unroll
+    for (int j = 0; j < KC; ++j) p[j] = Vp[j][o];
+#pragma unroll
+    for (int j = 0; j < KC; ++j) y = cfms(y, h[j], p[j]);
+    y = cscale(y, inv);
+    if (x.in) Vn[o] = y;
+    if constexpr (DIAG) {
+      if (x.in) un[o] = cmul(dd[static_cast<size_t>(i) * s.a.nq], y);
+    }
+  }
+  if (x.wave == 0) {
+    int live = x.in && s.live[x.col];
+    if (live) {
+      const size_t cols = s.cols, col = x.col;
+#pragma unroll
+      for (int j = 0; j < KC; ++j)
+        if (j == k) h[j].x += 1.0;
+#pragma unroll
+      for (int j = 0; j + 1 < KC; ++j) {
+        if (j < k) {
+          const double c = s.rc[j * cols + col];
+          const double2 sn = s.rs[j * cols + col];
+          const double2 t = cfma(cscale(h[j], c), sn, h[j + 1]);
+          h[j + 1] = cfms(cscale(h[j + 1], c), cconj(sn), h[j]);
+          h[j] = t;
+        }
+      }
+      double2 hk = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int j = 0; j < KC; ++j)
+        if (j == k) hk = h[j];
+      const double ah = hypot(hk.x, hk.y), r = hypot(ah, hn);
+      const double c = r > 0.0 ? ah / r : 1.0;
+      const double2 ph = ah > 0.0 ? cscale(hk, 1.0 / ah) : make_double2(1.0, 0.0);
+      const double2 sn = cscale(ph, r > 0.0 ? hn / r : 0.0);
+      s.rc[k * cols + col] = c;
+      s.rs[k * cols + col] = sn;
+      const size_t rk = static_cast<size_t>(k) * (k + 1) / 2;
+#pragma unroll
+      for (int j = 0; j < KC; ++j)
+        if (j < k) s.R[(rk + j) * cols + col] = h[j];
+      s.R[(rk + k) * cols + col] = cscale(ph, r);
+      const double2 gk = s.gv[k * cols + col];
+      s.gv[k * cols + col] = cscale(gk, c);
+      const double2 gn = cmul(make_double2(-sn.x, sn.y), gk);
+      s.gv[(k + 1) * cols + col] = gn;
+      s.kdim[col] = k + 1;
+      const double res = hypot(gn.x, gn.y);
+      // converged, broken down, or not a number: the column waits for the end of the cycle
+      live = res > s.target[col] && hn > 0.0 && k + 1 < SH_M;
+      s.live[col] = live;
+    }
+    const unsigned long long any = __ballot(live);
+    if (x.lane == 0) s.tile_live[tile_id] = any != 0;
+  }
+}
+
+// End of a cycle: X (+)= sum_j y_j V_j with the y of the column's triangular factor, and its state.
+__global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs s, int cycle, int last) {
+  const int tile_id = blockIdx.x;
+  if (cycle > 0 && s.tile_run[tile_id] == 0) return;
+  __shared__ double2 sh[SH_WAVES][SH_TN];
+  __shared__ int s_kmax;
+  const SharedTile x = shared_tile(s);
+  const int n = s.a.n, N = s.N;
+  const size_t vec = static_cast<size_t>(s.groups) * n * N, cols = s.cols, col = x.col;
+  const bool run = s.state[col] == SH_RUN;
+  const int kd = run ? s.kdim[col] : 0;
+  double2 y[SH_M];
+#pragma unroll
+  for (int j = SH_M - 1; j >= 0; --j) {
+    y[j] = make_double2(0.0, 0.0);
+    if (j < kd) {
+      double2 r = s.gv[j * cols + col];
+#pragma unroll
+      for (int l = j + 1; l < SH_M; ++l)
+        if (l < kd) r = cfms(r, s.R[(static_cast<size_t>(l) * (l + 1) / 2 + j) * cols + col], y[l]);
+      y[j] = cmul(r, cinv(s.R[(static_cast<size_t>(j) * (j + 1) / 2 + j) * cols + col]));
+    }
+  }
+  if (x.wave == 0) {
+    int km = kd;
+    for (int o = 32; o > 0; o >>= 1) km = max(km, __shfl_xor(km, o));
+    if (x.lane == 0) s_kmax = km;
+  }
+  __syncthreads();
+  const int kmax = s_kmax;
+  double nrm = 0.0;
+  auto pass = [&](auto kc_tag) {
+    constexpr int KC = decltype(kc_tag)::value;
+#pragma unroll 2
+    for (int i = x.wave; i < n; i += SH_WAVES) {
+      const size_t o = x.base + static_cast<size_t>(i) * N;
+      double2 p[KC];
+#pragma unroll
+      for (int j = 0; j < KC; ++j) p[j] = s.V[static_cast<size_t>(j < kmax ? j : 0) * vec + o];
+      double2 acc = cycle > 0 ? s.X[o] : make_double2(0.0, 0.0);
+#pragma unroll
+      for (int j = 0; j < KC; ++j)
+        if (j < kd) acc = cfma(acc, y[j], p[j]);
+      nrm = fma(acc.x, acc.x, fma(acc.y, acc.y, nrm));
+      if (x.in) s.X[o] = acc;
+    }
+  };
+  switch ((kmax + 1) / 2) {
+    case 0:
+    case 1: pass(std::integral_constant<int, 2>{}); break;
+    case 2: pass(std::integral_constant<int, 4>{}); break;
+    case 3: pass(std::integral_constant<int, 6>{}); break;
+    case 4: pass(std::integral_constant<int, 8>{}); break;
+    default: pass(std::integral_constant<int, SH_M>{}); break;
+  }
+  const double xn = sqrt(wave_sum(sh, make_double2(nrm, 0.0), x).x);
+  if (x.wave == 0) {
+    int st = s.state[col];
+    if (run) {
+      const double2 g = s.gv[static_cast<size_t>(kd) * cols + col];
+      const double res = hypot(g.x, g.y), b0 = s.beta0[col];
+      if (!(xn <= 1e300) || !(res <= 1e300))
+        st = SH_FAIL;
+      else if (cycle > 0 && res <= 2.0 * SH_DONE_TOL * xn)
+        st = SH_DONE;  // the residual it started from was formed from A itself
+      else if (last || !(res <= SH_STAGNATION * b0))
+        st = SH_FAIL;
+    }
+    if (x.in) {
+      s.state[col] = st;
+      s.xnorm[col] = xn;
+    }
+    const unsigned long long any = __ballot(x.in && st == SH_RUN);
+    if (x.lane == 0) s.tile_run[tile_id] = any != 0;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Sums over v of every orbital pair's rows of v ([groups][T][N], for the V_r term). One workgroup per tile.
+template <int T>
+__global__ void __launch_bounds__(256) shared_sums_kernel(SharedArgs s, const double2* __restrict__ v,
+                                                          const int* __restrict__ tiles) {
+  if (tiles[blockIdx.x] == 0) return;
+  __shared__ double2 sh[SH_WAVES][SH_TN];
+  const SharedTile x = shared_tile(s);
+  const int nv = s.a.nv, N = s.N;
+  for (int c = 0; c < T; ++c) {
+    double2 sv = make_double2(0.0, 0.0);
+    for (int vi = x.wave; vi < nv; vi += SH_WAVES) sv = cadd(sv, v[x.base + static_cast<size_t>(c * nv + vi) * N]);
+    sv = wave_sum(sh, sv, x);
+    if (x.in && x.wave == 0) s.sums[(static_cast<size_t>(x.grp) * T + c) * N + x.e] = sv;
+  }
+}
+
+// u = D(q) v, or (RESIDUAL) u = B - A0 v - D(q) v with A0 v in s.g. grid (tiles, ceil(nv / 4)), one
+// frequency per wavefront. The blocks of the tile's q-points are staged in LDS, coalesced over q; read
+// by every column from global memory they made this step 5 times slower than its traffic.
+template <int T, bool RESIDUAL>
+__global__ void __launch_bounds__(256) shared_apply_kernel(SharedArgs s, const double2* __restrict__ v,
+                                                           const int* __restrict__ tiles) {
+  if (tiles[blockIdx.x] == 0) return;
+  constexpr int QT = (63 + T - 1) / T + 1;  // most q-points of a tile
+  __shared__ double2 s_d[SH_WAVES][T * T][QT];
+  const SharedTile x = shared_tile(s);
+  const int nv = s.a.nv, nq = s.a.nq, N = s.N;
+  const int vi = blockIdx.y * SH_WAVES + x.wave;
+  const int g = s.group0 + x.grp, w = g % s.a.nw, chan = g / s.a.nw;
+  const int q0 = (blockIdx.x - x.grp * s.ntile) * SH_TN / T;
+  double2 y[T];
+  if (vi < nv) {
+    const double2* dd = s.dd + (static_cast<size_t>(w) * T * T * nv + vi) * nq;
+    for (int e = x.lane; e < T * T * QT; e += 64) {
+      const int blk = e / QT, qq = e - blk * QT;
+      if (q0 + qq < nq) s_d[x.wave][blk][qq] = dd[static_cast<size_t>(blk) * nv * nq + q0 + qq];
+    }
+#pragma unroll
+    for (int c = 0; c < T; ++c) y[c] = v[x.base + static_cast<size_t>(c * nv + vi) * N];
+  }
+  __syncthreads();
+  if (vi >= nv || !x.in) return;
+  const int qq = x.q - q0;
+#pragma unroll
+  for (int r = 0; r < T; ++r) {
+    double2 acc = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int c = 0; c < T; ++c) acc = cfma(acc, s_d[x.wave][r * T + c][qq], y[c]);
+    if (s.dv) {
+      const double2* dv = s.dv + (static_cast<size_t>(chan) * nq + x.q) * T * T + r * T;
+      for (int c = 0; c < T; ++c) acc = cfms(acc, dv[c], s.sums[(static_cast<size_t>(x.grp) * T + c) * N + x.e]);
+    }
+    const size_t o = x.base + static_cast<size_t>(r * nv + vi) * N;
+    if constexpr (RESIDUAL) acc = csub(make_double2(r == x.t ? 1.0 : 0.0, 0.0), cadd(s.g[o], acc));
+    s.u[o] = acc;
+  }
+}
+
+// out = X / beta, q fastest. grid (n, groups).
+__global__ void __launch_bounds__(256) shared_output_kernel(SharedArgs s) {
+  const LadderArgs& a = s.a;
+  const int i = blockIdx.x, grp = blockIdx.y;
+  const double2* X = s.X + (static_cast<size_t>(grp) * a.n + i) * s.N;
+  const int g = s.group0 + grp, w = g % a.nw, chan = g / a.nw;
+  for (int e = threadIdx.x; e < s.N; e += 256) {
+    const int t = e / a.nq, q = e - t * a.nq;
+    a.out[ladder_out_index(a, chan, w, q, i, t)] = cscale(X[q * a.T + t], a.inv_beta);
+  }
+}
+
+// info 0 for the converged problems of the batch; the others are appended to the list (in item
+// order, so the LU sees the same list on every run). One workgroup.
+__global__ void __launch_bounds__(1024) shared_collect_kernel(SharedArgs s, int* __restrict__ list, int* __restrict__ count,
+                                                              int clear) {
+  __shared__ int s_cnt[16];
+  const int items = s.groups * s.a.nq, T = s.a.T;
+  int base = clear ? 0 : *count;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int i0 = 0; i0 < items; i0 += 1024) {
+    const int i = i0 + threadIdx.x;
+    bool bad = false;
+    if (i < items) {
+      for (int t = 0; t < T; ++t) bad |= s.state[static_cast<size_t>(i) * T + t] != SH_DONE;
+      if (!bad && s.a.info) s.a.info[static_cast<size_t>(s.group0) * s.a.nq + i] = 0;
+    }
+    const unsigned long long m = __ballot(bad);
+    __syncthreads();
+    if (lane == 0) s_cnt[wave] = __popcll(m);
+    __syncthreads();
+    int off = base, tot = 0;
+    for (int k = 0; k < 16; ++k) {
+      if (k < wave) off += s_cnt[k];
+      tot += s_cnt[k];
+    }
+    if (bad) list[off + __popcll(m & ((1ull << lane) - 1))] = s.group0 * s.a.nq + i;
+    base += tot;
+  }
+  if (threadIdx.x == 0) *count = base;
+}
+
+// ---------------------------------------------------------------------------
+template <bool DIAG>
+static int shared_step(const SharedArgs& s, int k, hipStream_t stream) {
+  const dim3 gd(static_cast<unsigned>(s.groups) * s.ntile), bd(256);
+  switch (k / 2) {
+    case 0: hipLaunchKernelGGL((shared_step_kernel<DIAG, 2>), gd, bd, 0, stream, s, k); break;
+    case 1: hipLaunchKernelGGL((shared_step_kernel<DIAG, 4>), gd, bd, 0, stream, s, k); break;
+    case 2: hipLaunchKernelGGL((shared_step_kernel<DIAG, 6>), gd, bd, 0, stream, s, k); break;
+    case 3: hipLaunchKernelGGL((shared_step_kernel<DIAG, 8>), gd, bd, 0, stream, s, k); break;
+    default: hipLaunchKernelGGL((shared_step_kernel<DIAG, SH_M>), gd, bd, 0, stream, s, k); break;
+  }
+  DGAMI_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+// u = D(q) v, or u = B - A v with A0 v in s.g.
+template <int T>
+static int shared_apply(const SharedArgs& s, const double2* v, bool residual, const int* tiles, hipStream_t stream) {
+  const unsigned nt = static_cast<unsigned>(s.groups) * s.ntile;
+  if (s.dv) {
+    hipLaunchKernelGGL((shared_sums_kernel<T>), dim3(nt), dim3(256), 0, stream, s, v, tiles);
+    DGAMI_HIP_CHECK(hipGetLastError());
+  }
+  const dim3 gd(nt, ceil_div(s.a.nv, SH_WAVES)), bd(256);
+  if (residual)
+    hipLaunchKernelGGL((shared_apply_kernel<T, true>), gd, bd, 0, stream, s, v, tiles);
+  else
+    hipLaunchKernelGGL((shared_apply_kernel<T, false>), gd, bd, 0, stream, s, v, tiles);
+  DGAMI_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+// C = A B of every group's n x n matrix, tiles without work left out.
+static int shared_product(const SharedArgs& s, const double2* A, const double2* B, const int* tiles, bool three,
+                          hipStream_t stream) {
+  ZgemmArgs g;
+  g.A = A;
+  g.B = B;
+  g.C = s.g;
+  g.M = g.K = g.lda = s.a.n;
+  g.N = g.ldb = g.ldc = s.N;
+  g.sa = static_cast<long long>(s.a.n) * s.a.n;
+  g.sb = g.sc = static_cast<long long>(s.a.n) * s.N;
+  g.alpha = make_double2(1.0, 0.0);
+  g.beta = make_double2(0.0, 0.0);
+  g.tile_active = tiles;
+  return three ? launch_zgemm<true>(g, s.groups, stream) : launch_zgemm<false>(g, s.groups, stream);
+}
+
+template <int T>
+static int shared_solve(SharedArgs& s, const double2* A0, hipStream_t stream) {
+  const dim3 gd(static_cast<unsigned>(s.groups) * s.ntile), bd(256);
+  const bool diag = T == 1 && !s.dv;
+  const size_t vec = static_cast<size_t>(s.groups) * s.a.n * s.N;
+  int rc = 0;
+#define DGAMI_STEP(x) \
+  if ((rc = (x)) != 0) return rc
+  for (int cycle = 0; cycle < SH_CYCLES; ++cycle) {
+    if (cycle > 0) {
+      DGAMI_STEP(shared_product(s, A0, s.X, s.tile_run, false, stream));
+      DGAMI_STEP(shared_apply<T>(s, s.X, true, s.tile_run, stream));
+      DGAMI_STEP(shared_product(s, s.P, s.u, s.tile_run, true, stream));
+    }
+    if (diag)
+      hipLaunchKernelGGL((shared_start_kernel<true>), gd, bd, 0, stream, s, cycle == 0 ? 1 : 0);
+    else
+      hipLaunchKernelGGL((shared_start_kernel<false>), gd, bd, 0, stream, s, cycle == 0 ? 1 : 0);
+    DGAMI_HIP_CHECK(hipGetLastError());
+    for (int k = 0; k < SH_M; ++k) {
+      if (!diag) DGAMI_STEP(shared_apply<T>(s, s.V + k * vec, false, s.tile_live, stream));
+      DGAMI_STEP(shared_product(s, s.P, s.u, s.tile_live, true, stream));
+      DGAMI_STEP(diag ? shared_step<true>(s, k, stream) : shared_step<false>(s, k, stream));
+    }
+    hipLaunchKernelGGL(shared_update_kernel, gd, bd, 0, stream, s, cycle, cycle == SH_CYCLES - 1 ? 1 : 0);
+    DGAMI_HIP_CHECK(hipGetLastError());
+  }
+#undef DGAMI_STEP
+  return 0;
+}
+
+bool ladder_shared_applies(const LadderArgs& a) {
+  if (a.dense || a.rhs_mode != LADDER_RHS_INDICATOR || a.items) return false;
+  if (a.T != 1 && a.T != 4 && a.T != 9 && a.T != 16) return false;
+  if (a.n <= SHARED_MIN_N || a.n > 1536 || a.nq < SHARED_MIN_NQ) return false;
+  const char* v = getenv("DGAMI_LADDER_SHARED");
+  return !(v && std::string(v) == "0");
+}
+
+int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
+  const int n = a.n, T = a.T, nq = a.nq, TT = T * T;
+  const size_t G = static_cast<size_t>(a.nchan) * a.nw, nn = static_cast<size_t>(n) * n;
+  const int N = nq * T, ntile = static_cast<int>(ceil_div(N, SH_TN));
+  const size_t items = G * nq;
+  // groups per batch: basis, operands and iterate of at most 24 GiB
+  const size_t vec1 = static_cast<size_t>(n) * N * sizeof(double2);
+  size_t gb = (size_t(24) << 30) / (vec1 * (SH_M + 4) + 2 * nn * sizeof(double2));
+  gb = std::max<size_t>(1, std::min(gb, G));
+  gb = std::min<size_t>(gb, 65535);
+  const size_t cols = gb * N;
+
+  const size_t rows = static_cast<size_t>(a.nw) * TT * a.nv;
+  const size_t vsz = a.v_r ? static_cast<size_t>(a.nchan) * TT : 0, dvsz = vsz * nq;
+  const size_t szc = rows + rows * nq + vsz + dvsz + gb * nn * 2 + gb * n * T;
+  double2* m = static_cast<double2*>(workspace(WS_SHARED, szc * sizeof(double2)));
+  const size_t vecs = gb * static_cast<size_t>(n) * N;
+  const size_t sumsz = a.v_r ? gb * T * N : 0;
+  double2* vp = static_cast<double2*>(workspace(WS_SHARED_VEC, (vecs * (SH_M + 4) + sumsz) * sizeof(double2)));
+  const size_t per_col = sizeof(double2) * (SH_M + SH_ROT + SH_M + 1) + sizeof(double) * (SH_M + 3) + 3 * sizeof(int);
+  char* st = static_cast<char*>(
+      workspace(WS_SHARED_STATE, cols * per_col + (2 * gb * ntile + items + gb + 64) * sizeof(int)));
+  if (!m || !vp || !st) return -2;
+
+  SharedArgs s{};
+  s.a = a;
+  double2* mean = m;
+  double2* dd = mean + rows;
+  double2* vmean = dd + rows * nq;
+  double2* dv = vmean + vsz;
+  double2* A0 = dv + dvsz;
+  double2* P = A0 + gb * nn;
+  double2* z0 = P + gb * nn;
+  s.dd = dd;
+  s.dv = a.v_r ? dv : nullptr;
+  s.P = P;
+  s.z0 = z0;
+  s.N = N;
+  s.ntile = ntile;
+  s.rs = reinterpret_cast<double2*>(st);
+  s.R = s.rs + SH_M * cols;
+  s.gv = s.R + SH_ROT * cols;
+  s.rc = reinterpret_cast<double*>(s.gv + (SH_M + 1) * cols);
+  s.beta0 = s.rc + SH_M * cols;
+  s.target = s.beta0 + cols;
+  s.xnorm = s.target + cols;
+  s.kdim = reinterpret_cast<int*>(s.xnorm + cols);
+  s.state = s.kdim + cols;
+  s.live = s.state + cols;
+  s.tile_run = s.live + cols;
+  s.tile_live = s.tile_run + gb * ntile;
+  int* list = s.tile_live + gb * ntile;
+  int* count = list + items;
+  int* pinfo = count + 1;  // [gb] of the inversions; a singular mean matrix shows in the columns
+
+  hipLaunchKernelGGL(shared_mean_kernel, dim3(ceil_div(rows, 4)), dim3(256), 0, stream, a.chi0_inv, mean, dd,
+                     static_cast<int>(rows), nq);
+  DGAMI_HIP_CHECK(hipGetLastError());
+  if (a.v_r) {
+    hipLaunchKernelGGL(shared_vmean_kernel, dim3(static_cast<unsigned>(vsz)), dim3(64), 0, stream, a, vmean, dv);
+    DGAMI_HIP_CHECK(hipGetLastError());
+  }
+  for (size_t g0 = 0; g0 < G; g0 += gb) {
+    const int ng = static_cast<int>(std::min(gb, G - g0));
+    s.group0 = static_cast<int>(g0);
+    s.groups = ng;
+    s.cols = static_cast<size_t>(ng) * N;
+    const size_t used = static_cast<size_t>(ng) * n * N;
+    s.V = vp;
+    s.u = s.V + used * (SH_M + 1);
+    s.g = s.u + used;
+    s.X = s.g + used;
+    s.sums = s.X + used;
+    hipLaunchKernelGGL(shared_matrix_kernel, dim3(ceil_div(nn, 256), ng), dim3(256), 0, stream, a, mean,
+                       a.v_r ? vmean : nullptr, A0, s.group0);
+    DGAMI_HIP_CHECK(hipGetLastError());
+    int rc = dgami_invert_dense(ng, n, reinterpret_cast<const dgami_c128*>(A0), reinterpret_cast<dgami_c128*>(P), pinfo,
+                                stream);
+    if (rc) return rc;
+    hipLaunchKernelGGL(shared_rhs_kernel, dim3(ceil_div(static_cast<size_t>(ng) * n, 4)), dim3(256), 0, stream, P, z0,
+                       ng * n, n, T, a.nv);
+    DGAMI_HIP_CHECK(hipGetLastError());
+    switch (T) {
+      case 1: rc = shared_solve<1>(s, A0, stream); break;
+      case 4: rc = shared_solve<4>(s, A0, stream); break;
+      case 9: rc = shared_solve<9>(s, A0, stream); break;
+      default: rc = shared_solve<16>(s, A0, stream); break;
+    }
+    if (rc) return rc;
+    hipLaunchKernelGGL(shared_output_kernel, dim3(n, ng), dim3(256), 0, stream, s);
+    DGAMI_HIP_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(shared_collect_kernel, dim3(1), dim3(1024), 0, stream, s, list, count, g0 == 0 ? 1 : 0);
+    DGAMI_HIP_CHECK(hipGetLastError());
+  }
+  // the problems that did not converge, by the LU: its kernels are launched for every problem and
+  // return at once beyond the device count
+  LadderArgs f = a;
+  f.items = list;
+  f.nitems = count;
+  const int v = ladder_col_variant(n, T);
+  return v >= 0 ? ladder_col_launch(v, f, stream) : ladder_blocked_fp64(f, -1, stream);
+}
+
+}  // namespace dgami
