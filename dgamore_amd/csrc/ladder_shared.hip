@@ -36,30 +36,12 @@ int ladder_col_variant(int n, int nrhs);
 int ladder_col_launch(int variant, const LadderArgs& a, hipStream_t stream);
 int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream);
 
-constexpr int SH_M = 10;           // Krylov vectors of a cycle
 constexpr int SH_TN = ZG_TN;       // columns of a workgroup, and of a tile of the products
 constexpr int SH_WAVES = 4;        // wavefronts of a workgroup, which share the rows of its columns
-constexpr int SH_ROT = SH_M * (SH_M + 1) / 2;
 
-// A cycle stops a column at a residual of SH_CYCLE_TOL of its start (below that the error of P
-// decides); the column is done when its residual is below SH_DONE_TOL of |X|.
-constexpr int SH_CYCLES = 4;
-constexpr double SH_CYCLE_TOL = 1e-10;
-constexpr double SH_DONE_TOL = 2e-16;
-// A cycle that leaves more than this of its residual is stagnating.
-constexpr double SH_STAGNATION = 0.3;
-
-enum SharedState { SH_RUN = 0, SH_DONE = 1, SH_FAIL = 2 };
-
-struct SharedArgs {
-  LadderArgs a;
-  int group0, groups;     // groups of this batch
-  int N, ntile;           // columns (q, t) of a group, tiles of SH_TN columns
+struct SharedArgs : SharedGroups {
+  int ntile;              // tiles of SH_TN columns
   size_t cols;            // columns of the batch
-  const double2* P;       // [groups][n][n]
-  const double2* dd;      // D(q): [nw][T*T][nv][nq]
-  const double2* dv;      // (V_r(q) - mean V_r) / beta^2: [nchan][nq][T*T], or null
-  const double2* z0;      // P B [groups][n][T]
   double2* V;             // [SH_M + 1][groups][n][N] Krylov basis
   double2* u;             // operand of the products [groups][n][N]
   double2* g;             // their result
@@ -74,7 +56,6 @@ struct SharedArgs {
   double* target;
   double* xnorm;
   int* kdim;              // vectors of the current cycle
-  int* state;             // SharedState
   int* live;              // 1 while the column iterates in the current cycle
   int* tile_run;          // [groups][ntile] 1 while the tile has a running column
   int* tile_live;         // [groups][ntile] 1 while the tile has a column iterating in this cycle
@@ -489,7 +470,7 @@ __global__ void __launch_bounds__(256) shared_output_kernel(SharedArgs s) {
 
 // info 0 for the converged problems of the batch; the others are appended to the list (in item
 // order, so the LU sees the same list on every run). One workgroup.
-__global__ void __launch_bounds__(1024) shared_collect_kernel(SharedArgs s, int* __restrict__ list, int* __restrict__ count,
+__global__ void __launch_bounds__(1024) shared_collect_kernel(SharedGroups s, int* __restrict__ list, int* __restrict__ count,
                                                               int clear) {
   __shared__ int s_cnt[16];
   const int items = s.groups * s.a.nq, T = s.a.T;
@@ -605,46 +586,28 @@ bool ladder_shared_applies(const LadderArgs& a) {
   return !(v && std::string(v) == "0");
 }
 
-int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
-  const int n = a.n, T = a.T, nq = a.nq, TT = T * T;
-  const size_t G = static_cast<size_t>(a.nchan) * a.nw, nn = static_cast<size_t>(n) * n;
-  const int N = nq * T, ntile = static_cast<int>(ceil_div(N, SH_TN));
-  const size_t items = G * nq;
-  // groups per batch: basis, operands and iterate of at most 24 GiB
-  const size_t vec1 = static_cast<size_t>(n) * N * sizeof(double2);
-  size_t gb = (size_t(24) << 30) / (vec1 * (SH_M + 4) + 2 * nn * sizeof(double2));
-  gb = std::max<size_t>(1, std::min(gb, G));
-  gb = std::min<size_t>(gb, 65535);
-  const size_t cols = gb * N;
+// A batch by one launch per product and per pass over the basis: vec and st hold the vectors and the
+// columns' data of ng groups.
+static size_t large_vectors(const LadderArgs& a, size_t groups, int N) {
+  return groups * N * (static_cast<size_t>(a.n) * (SH_M + 4) + (a.v_r ? a.T : 0));
+}
+static size_t large_state(size_t groups, int N) {
+  const size_t per_col = sizeof(double2) * (SH_M + SH_ROT + SH_M + 1) + sizeof(double) * (SH_M + 3) + 2 * sizeof(int);
+  return groups * (N * per_col + 2 * ceil_div(N, SH_TN) * sizeof(int));
+}
 
-  const size_t rows = static_cast<size_t>(a.nw) * TT * a.nv;
-  const size_t vsz = a.v_r ? static_cast<size_t>(a.nchan) * TT : 0, dvsz = vsz * nq;
-  const size_t szc = rows + rows * nq + vsz + dvsz + gb * nn * 2 + gb * n * T;
-  double2* m = static_cast<double2*>(workspace(WS_SHARED, szc * sizeof(double2)));
-  const size_t vecs = gb * static_cast<size_t>(n) * N;
-  const size_t sumsz = a.v_r ? gb * T * N : 0;
-  double2* vp = static_cast<double2*>(workspace(WS_SHARED_VEC, (vecs * (SH_M + 4) + sumsz) * sizeof(double2)));
-  const size_t per_col = sizeof(double2) * (SH_M + SH_ROT + SH_M + 1) + sizeof(double) * (SH_M + 3) + 3 * sizeof(int);
-  char* st = static_cast<char*>(
-      workspace(WS_SHARED_STATE, cols * per_col + (2 * gb * ntile + items + gb + 64) * sizeof(int)));
-  if (!m || !vp || !st) return -2;
-
+static int shared_large_solve(const SharedGroups& sg, double2* vec, void* st, hipStream_t stream) {
   SharedArgs s{};
-  s.a = a;
-  double2* mean = m;
-  double2* dd = mean + rows;
-  double2* vmean = dd + rows * nq;
-  double2* dv = vmean + vsz;
-  double2* A0 = dv + dvsz;
-  double2* P = A0 + gb * nn;
-  double2* z0 = P + gb * nn;
-  s.dd = dd;
-  s.dv = a.v_r ? dv : nullptr;
-  s.P = P;
-  s.z0 = z0;
-  s.N = N;
-  s.ntile = ntile;
-  s.rs = reinterpret_cast<double2*>(st);
+  static_cast<SharedGroups&>(s) = sg;
+  const size_t cols = static_cast<size_t>(s.groups) * s.N, used = cols * s.a.n;
+  s.ntile = static_cast<int>(ceil_div(s.N, SH_TN));
+  s.cols = cols;
+  s.V = vec;
+  s.u = s.V + used * (SH_M + 1);
+  s.g = s.u + used;
+  s.X = s.g + used;
+  s.sums = s.X + used;
+  s.rs = static_cast<double2*>(st);
   s.R = s.rs + SH_M * cols;
   s.gv = s.R + SH_ROT * cols;
   s.rc = reinterpret_cast<double*>(s.gv + (SH_M + 1) * cols);
@@ -652,11 +615,60 @@ int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
   s.target = s.beta0 + cols;
   s.xnorm = s.target + cols;
   s.kdim = reinterpret_cast<int*>(s.xnorm + cols);
-  s.state = s.kdim + cols;
-  s.live = s.state + cols;
+  s.live = s.kdim + cols;
   s.tile_run = s.live + cols;
-  s.tile_live = s.tile_run + gb * ntile;
-  int* list = s.tile_live + gb * ntile;
+  s.tile_live = s.tile_run + static_cast<size_t>(s.groups) * s.ntile;
+  int rc = 0;
+  switch (s.a.T) {
+    case 1: rc = shared_solve<1>(s, s.A0, stream); break;
+    case 4: rc = shared_solve<4>(s, s.A0, stream); break;
+    case 9: rc = shared_solve<9>(s, s.A0, stream); break;
+    default: rc = shared_solve<16>(s, s.A0, stream); break;
+  }
+  if (rc) return rc;
+  hipLaunchKernelGGL(shared_output_kernel, dim3(s.a.n, s.groups), dim3(256), 0, stream, s);
+  DGAMI_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
+  const int n = a.n, T = a.T, nq = a.nq, TT = T * T, N = nq * T;
+  const size_t G = static_cast<size_t>(a.nchan) * a.nw, nn = static_cast<size_t>(n) * n;
+  const size_t items = G * nq;
+  const bool tiles = n <= SHARED_TILE_N;
+  const size_t pk = tiles ? shared_packed(n) : 0;
+  // groups per batch: matrices and, for large sizes, vectors of at most 24 GiB
+  const size_t per_group = (2 * (nn + pk) + (tiles ? 0 : large_vectors(a, 1, N))) * sizeof(double2);
+  const size_t gb = std::max<size_t>(1, std::min<size_t>({(size_t(24) << 30) / per_group, G, 65535}));
+  SharedGroups s{};
+  s.a = a;
+  s.N = N;
+  s.groups = static_cast<int>(gb);
+
+  const size_t rows = static_cast<size_t>(a.nw) * TT * a.nv;
+  const size_t vsz = a.v_r ? static_cast<size_t>(a.nchan) * TT : 0, dvsz = vsz * nq;
+  const size_t szc = rows + rows * nq + vsz + dvsz + gb * (nn + pk) * 2 + gb * n * T;
+  double2* mean = static_cast<double2*>(workspace(WS_SHARED, szc * sizeof(double2)));
+  double2* vec = static_cast<double2*>(
+      workspace(WS_SHARED_VEC, (tiles ? shared_tile_workspace(s) : large_vectors(a, gb, N)) * sizeof(double2)));
+  const size_t ints = gb * N + NUM_XCD + items + gb + 64;
+  char* st = static_cast<char*>(workspace(WS_SHARED_STATE, (tiles ? 0 : large_state(gb, N)) + ints * sizeof(int)));
+  if (!mean || !vec || !st) return -2;
+  double2* dd = mean + rows;
+  double2* vmean = dd + rows * nq;
+  double2* dv = vmean + vsz;
+  double2* A0 = dv + dvsz;
+  double2* P = A0 + gb * nn;
+  double2* pack = P + gb * nn;
+  double2* z0 = pack + 2 * gb * pk;
+  s.dd = dd;
+  s.dv = a.v_r ? dv : nullptr;
+  s.A0 = A0;
+  s.P = P;
+  s.z0 = z0;
+  s.state = reinterpret_cast<int*>(st + (tiles ? 0 : large_state(gb, N)));
+  int* next = s.state + gb * N;
+  int* list = next + NUM_XCD;
   int* count = list + items;
   int* pinfo = count + 1;  // [gb] of the inversions; a singular mean matrix shows in the columns
 
@@ -671,13 +683,6 @@ int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
     const int ng = static_cast<int>(std::min(gb, G - g0));
     s.group0 = static_cast<int>(g0);
     s.groups = ng;
-    s.cols = static_cast<size_t>(ng) * N;
-    const size_t used = static_cast<size_t>(ng) * n * N;
-    s.V = vp;
-    s.u = s.V + used * (SH_M + 1);
-    s.g = s.u + used;
-    s.X = s.g + used;
-    s.sums = s.X + used;
     hipLaunchKernelGGL(shared_matrix_kernel, dim3(ceil_div(nn, 256), ng), dim3(256), 0, stream, a, mean,
                        a.v_r ? vmean : nullptr, A0, s.group0);
     DGAMI_HIP_CHECK(hipGetLastError());
@@ -687,15 +692,8 @@ int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL(shared_rhs_kernel, dim3(ceil_div(static_cast<size_t>(ng) * n, 4)), dim3(256), 0, stream, P, z0,
                        ng * n, n, T, a.nv);
     DGAMI_HIP_CHECK(hipGetLastError());
-    switch (T) {
-      case 1: rc = shared_solve<1>(s, A0, stream); break;
-      case 4: rc = shared_solve<4>(s, A0, stream); break;
-      case 9: rc = shared_solve<9>(s, A0, stream); break;
-      default: rc = shared_solve<16>(s, A0, stream); break;
-    }
+    rc = tiles ? shared_tile_solve(s, pack, vec, next, stream) : shared_large_solve(s, vec, st, stream);
     if (rc) return rc;
-    hipLaunchKernelGGL(shared_output_kernel, dim3(n, ng), dim3(256), 0, stream, s);
-    DGAMI_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(shared_collect_kernel, dim3(1), dim3(1024), 0, stream, s, list, count, g0 == 0 ? 1 : 0);
     DGAMI_HIP_CHECK(hipGetLastError());
   }

@@ -44,6 +44,44 @@ __device__ __forceinline__ double2 zmma_value(const ZmmaAcc<MI, NJ, THREE>& c, i
     return make_double2(c.re[i][j][r], c.im[i][j][r]);
 }
 
+// c += A B for one k-step of 4: av[i], bv[j] are this lane's operands A[l%16][l/16] and B[l/16][l%16] of
+// row block i and column block j.
+template <int MI, int NJ, bool THREE>
+__device__ __forceinline__ void zmma_step(ZmmaAcc<MI, NJ, THREE>& c, const double2 (&av)[MI], const double2 (&bv)[NJ]) {
+  if constexpr (THREE) {
+    double as[MI], bs[NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) as[i] = av[i].x + av[i].y;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) bs[j] = bv[j].x + bv[j].y;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        c.re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].x, bv[j].x, c.re[i][j], 0, 0, 0);
+        c.im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].y, bv[j].y, c.im[i][j], 0, 0, 0);
+        c.sum[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[i], bs[j], c.sum[i][j], 0, 0, 0);
+      }
+  } else {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        c.re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].x, bv[j].x, c.re[i][j], 0, 0, 0);
+        c.im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].x, bv[j].y, c.im[i][j], 0, 0, 0);
+      }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const double nai = -av[i].y;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        c.re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai, bv[j].y, c.re[i][j], 0, 0, 0);
+        c.im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].y, bv[j].x, c.im[i][j], 0, 0, 0);
+      }
+    }
+  }
+}
+
 // c += A B for one chunk of TK (a multiple of 4) staged in LDS: sa[row][k], sb[k][col]; the
 // wavefront's blocks start at row wm and column wn.
 template <int MI, int NJ, int TM, int TN, int TK, bool THREE>
@@ -57,38 +95,7 @@ __device__ __forceinline__ void zmma_chunk(ZmmaAcc<MI, NJ, THREE>& c, const doub
     for (int i = 0; i < MI; ++i) av[i] = sa[wm + 16 * i + l16][k + kg];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) bv[j] = sb[k + kg][wn + 16 * j + l16];
-    if constexpr (THREE) {
-      double as[MI], bs[NJ];
-#pragma unroll
-      for (int i = 0; i < MI; ++i) as[i] = av[i].x + av[i].y;
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) bs[j] = bv[j].x + bv[j].y;
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          c.re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].x, bv[j].x, c.re[i][j], 0, 0, 0);
-          c.im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].y, bv[j].y, c.im[i][j], 0, 0, 0);
-          c.sum[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[i], bs[j], c.sum[i][j], 0, 0, 0);
-        }
-    } else {
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          c.re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].x, bv[j].x, c.re[i][j], 0, 0, 0);
-          c.im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].x, bv[j].y, c.im[i][j], 0, 0, 0);
-        }
-#pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        const double nai = -av[i].y;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          c.re[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai, bv[j].y, c.re[i][j], 0, 0, 0);
-          c.im[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].y, bv[j].x, c.im[i][j], 0, 0, 0);
-        }
-      }
-    }
+    zmma_step(c, av, bv);
   }
 }
 
