@@ -64,7 +64,9 @@ struct SharedArgs : SharedGroups {
 // ---------------------------------------------------------------------------
 // D(q) = chi0^-1(q) - mean over q and the mean, one wavefront per (w, block, v).
 __global__ void __launch_bounds__(256) shared_mean_kernel(const double2* __restrict__ ci, double2* __restrict__ mean,
-                                                          double2* __restrict__ dd, int rows, int nq) {
+                                                          double2* __restrict__ dd, int rows, int nq,
+                                                          int* __restrict__ count) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // of the unconverged problems
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= rows) return;
   const double2* src = ci + static_cast<size_t>(row) * nq;
@@ -199,6 +201,7 @@ __global__ void __launch_bounds__(256) shared_start_kernel(SharedArgs s, int fir
     const double xn = first ? nrm : s.xnorm[x.col];
     if (!(nrm <= 1e300)) st = SH_FAIL;  // infinite or NaN
     if (st == SH_RUN && nrm <= SH_DONE_TOL * xn) st = SH_DONE;
+    if (st == SH_RUN && !first && nrm > SH_STAGNATION * xn) st = SH_FAIL;  // P is no inverse
     const int live = x.in && st == SH_RUN;
     if (x.in) {
       s.state[x.col] = st;
@@ -383,8 +386,8 @@ __global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs s, int cy
       const double res = hypot(g.x, g.y), b0 = s.beta0[col];
       if (!(xn <= 1e300) || !(res <= 1e300))
         st = SH_FAIL;
-      else if (cycle > 0 && res <= 2.0 * SH_DONE_TOL * xn)
-        st = SH_DONE;  // the residual it started from was formed from A itself
+      else if (cycle > 0 && res <= 2.0 * SH_DONE_TOL * xn && b0 <= SH_TRUST * xn)
+        st = SH_DONE;
       else if (last || !(res <= SH_STAGNATION * b0))
         st = SH_FAIL;
     }
@@ -468,34 +471,18 @@ __global__ void __launch_bounds__(256) shared_output_kernel(SharedArgs s) {
   }
 }
 
-// info 0 for the converged problems of the batch; the others are appended to the list (in item
-// order, so the LU sees the same list on every run). One workgroup.
-__global__ void __launch_bounds__(1024) shared_collect_kernel(SharedGroups s, int* __restrict__ list, int* __restrict__ count,
-                                                              int clear) {
-  __shared__ int s_cnt[16];
-  const int items = s.groups * s.a.nq, T = s.a.T;
-  int base = clear ? 0 : *count;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int i0 = 0; i0 < items; i0 += 1024) {
-    const int i = i0 + threadIdx.x;
-    bool bad = false;
-    if (i < items) {
-      for (int t = 0; t < T; ++t) bad |= s.state[static_cast<size_t>(i) * T + t] != SH_DONE;
-      if (!bad && s.a.info) s.a.info[static_cast<size_t>(s.group0) * s.a.nq + i] = 0;
-    }
-    const unsigned long long m = __ballot(bad);
-    __syncthreads();
-    if (lane == 0) s_cnt[wave] = __popcll(m);
-    __syncthreads();
-    int off = base, tot = 0;
-    for (int k = 0; k < 16; ++k) {
-      if (k < wave) off += s_cnt[k];
-      tot += s_cnt[k];
-    }
-    if (bad) list[off + __popcll(m & ((1ull << lane) - 1))] = s.group0 * s.a.nq + i;
-    base += tot;
-  }
-  if (threadIdx.x == 0) *count = base;
+// info 0 for the converged problems of the batch; the others are appended to the list (in no order: the
+// LU of a problem does not depend on its place).
+__global__ void __launch_bounds__(256) shared_collect_kernel(SharedGroups s, int* __restrict__ list, int* __restrict__ count) {
+  const int i = blockIdx.x * 256 + threadIdx.x, T = s.a.T;
+  if (i >= s.groups * s.a.nq) return;
+  bool bad = false;
+  for (int t = 0; t < T; ++t) bad |= s.state[static_cast<size_t>(i) * T + t] != SH_DONE;
+  const int item = s.group0 * s.a.nq + i;
+  if (bad)
+    list[atomicAdd(count, 1)] = item;
+  else if (s.a.info)
+    s.a.info[item] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -578,12 +565,16 @@ static int shared_solve(SharedArgs& s, const double2* A0, hipStream_t stream) {
   return 0;
 }
 
-bool ladder_shared_applies(const LadderArgs& a) {
+bool ladder_shared_applies(const LadderArgs& a, int precision) {
   if (a.dense || a.rhs_mode != LADDER_RHS_INDICATOR || a.items) return false;
   if (a.T != 1 && a.T != 4 && a.T != 9 && a.T != 16) return false;
-  if (a.n <= SHARED_MIN_N || a.n > 1536 || a.nq < SHARED_MIN_NQ) return false;
+  if (a.n > 1536 || a.nq < 2) return false;
   const char* v = getenv("DGAMI_LADDER_SHARED");
-  return !(v && std::string(v) == "0");
+  if (v && *v) return std::string(v) == "1";
+  if (a.nq < SHARED_MIN_NQ) return false;
+  const double ratio = a.n / (3.0 * a.T) + 1.0, work = static_cast<double>(a.nchan) * a.nw * a.nq * ratio;
+  if (a.n <= SHARED_TILE_N && a.T <= 4) return work >= SHARED_MIN_WORK;
+  return ratio >= SHARED_MIN_RATIO && work >= (precision == DGAMI_MIXED_BF16X3_IR ? SHARED_MIN_WORK_BF16 : SHARED_MIN_WORK);
 }
 
 // A batch by one launch per product and per pass over the basis: vec and st hold the vectors and the
@@ -673,7 +664,7 @@ int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
   int* pinfo = count + 1;  // [gb] of the inversions; a singular mean matrix shows in the columns
 
   hipLaunchKernelGGL(shared_mean_kernel, dim3(ceil_div(rows, 4)), dim3(256), 0, stream, a.chi0_inv, mean, dd,
-                     static_cast<int>(rows), nq);
+                     static_cast<int>(rows), nq, count);
   DGAMI_HIP_CHECK(hipGetLastError());
   if (a.v_r) {
     hipLaunchKernelGGL(shared_vmean_kernel, dim3(static_cast<unsigned>(vsz)), dim3(64), 0, stream, a, vmean, dv);
@@ -683,18 +674,28 @@ int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
     const int ng = static_cast<int>(std::min(gb, G - g0));
     s.group0 = static_cast<int>(g0);
     s.groups = ng;
-    hipLaunchKernelGGL(shared_matrix_kernel, dim3(ceil_div(nn, 256), ng), dim3(256), 0, stream, a, mean,
-                       a.v_r ? vmean : nullptr, A0, s.group0);
-    DGAMI_HIP_CHECK(hipGetLastError());
-    int rc = dgami_invert_dense(ng, n, reinterpret_cast<const dgami_c128*>(A0), reinterpret_cast<dgami_c128*>(P), pinfo,
-                                stream);
+    int rc = 0;
+    if (n <= SHARED_SMALL_N) {
+      rc = shared_invert_small(s, mean, a.v_r ? vmean : nullptr, A0, P, stream);
+    } else {
+      hipLaunchKernelGGL(shared_matrix_kernel, dim3(ceil_div(nn, 256), ng), dim3(256), 0, stream, a, mean,
+                         a.v_r ? vmean : nullptr, A0, s.group0);
+      DGAMI_HIP_CHECK(hipGetLastError());
+      rc = dgami_invert_dense(ng, n, reinterpret_cast<const dgami_c128*>(A0), reinterpret_cast<dgami_c128*>(P), pinfo,
+                              stream);
+    }
     if (rc) return rc;
-    hipLaunchKernelGGL(shared_rhs_kernel, dim3(ceil_div(static_cast<size_t>(ng) * n, 4)), dim3(256), 0, stream, P, z0,
-                       ng * n, n, T, a.nv);
-    DGAMI_HIP_CHECK(hipGetLastError());
-    rc = tiles ? shared_tile_solve(s, pack, vec, next, stream) : shared_large_solve(s, vec, st, stream);
+    if (tiles) {
+      rc = shared_tile_solve(s, pack, z0, vec, next, stream);
+    } else {
+      hipLaunchKernelGGL(shared_rhs_kernel, dim3(ceil_div(static_cast<size_t>(ng) * n, 4)), dim3(256), 0, stream, P, z0,
+                         ng * n, n, T, a.nv);
+      DGAMI_HIP_CHECK(hipGetLastError());
+      rc = shared_large_solve(s, vec, st, stream);
+    }
     if (rc) return rc;
-    hipLaunchKernelGGL(shared_collect_kernel, dim3(1), dim3(1024), 0, stream, s, list, count, g0 == 0 ? 1 : 0);
+    hipLaunchKernelGGL(shared_collect_kernel, dim3(ceil_div(static_cast<size_t>(ng) * nq, 256)), dim3(256), 0, stream, s, list,
+                       count);
     DGAMI_HIP_CHECK(hipGetLastError());
   }
   // the problems that did not converge, by the LU: its kernels are launched for every problem and

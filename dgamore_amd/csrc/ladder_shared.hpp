@@ -7,9 +7,19 @@
 
 namespace dgami {
 
-// Compound sizes above SHARED_MIN_N with at least SHARED_MIN_NQ q-points per group take it.
-constexpr int SHARED_MIN_N = 64;
+// The rule: at least SHARED_MIN_NQ q-points share a matrix (its inversion costs three LUs), and there are
+// enough problems for the LU to be past its own latency, by how much more an LU computes per problem than a
+// product: problems x ratio >= SHARED_MIN_WORK with ratio = n / (3 T) + 1. Beyond one or two orbitals of up to
+// n = 256 the ratio itself has to reach SHARED_MIN_RATIO (the iteration's passes and D(q) blocks grow with T),
+// and the split-BF16 LU, twice as fast as the complex128 one, needs more problems to lose. Measured, LU form /
+// shared form in us, U = 2 ... 8. Complex128 below the line: n = 40, 450 problems 117 / 290; n = 120, 450 problems
+// 597 / 725; T = 9: n = 108, 588 problems 703 / 1499; n = 252, 2002 problems 5818 / 6899; n = 360, 5460 problems
+// 34644 / 39856; n = 720, 336 problems 12650 / 16370. Above: n = 40, 1890 problems 276 / 198; n = 64, 1890
+// problems 644 / 328; n = 120, 9702 problems 5095 / 1427; T = 4: n = 256, 2992 problems 8219 / 3502; n = 400, 990
+// problems 8434 / 7238. Split-BF16 below: T = 4, n = 400, 1890 problems 9407 / 10074; T = 9, n = 720, 1638
+// problems 29105 / 35937, 3822 problems 63206 / 67692; above: n = 480, 5712 problems 36712 / 23475; n = 720, 5642 problems 93079 / 86299.
 constexpr int SHARED_MIN_NQ = 16;
+constexpr double SHARED_MIN_WORK = 25000.0, SHARED_MIN_WORK_BF16 = 120000.0, SHARED_MIN_RATIO = 18.0;
 constexpr int SHARED_TILE_N = 256;
 
 constexpr int SH_M = 10;           // Krylov vectors of a cycle
@@ -17,9 +27,12 @@ constexpr int SH_ROT = SH_M * (SH_M + 1) / 2;
 
 // A cycle stops a column at a residual of SH_CYCLE_TOL of its start (below that the error of P
 // decides); the column is done when its residual is below SH_DONE_TOL of |X|.
-constexpr int SH_CYCLES = 4;
+constexpr int SH_CYCLES = 5;
 constexpr double SH_CYCLE_TOL = 1e-10;
 constexpr double SH_DONE_TOL = 2e-16;
+// ... provided that the cycle began at a residual below SH_TRUST of |X|: the preceding cycle then was right
+// to SH_TRUST, so P is the inverse of A0 to SH_TRUST and this cycle's error is at most that part of its start.
+constexpr double SH_TRUST = 1e-7;
 // A cycle that leaves more than this of its residual is stagnating.
 constexpr double SH_STAGNATION = 0.3;
 
@@ -38,13 +51,19 @@ struct SharedGroups {
   int* state;             // [groups][N] SharedState
 };
 
-bool ladder_shared_applies(const LadderArgs& a);
+// DGAMI_LADDER_SHARED = 0 / 1: never / wherever the form can run (for comparisons and tests).
+bool ladder_shared_applies(const LadderArgs& a, int precision);
 int ladder_solve_shared(const LadderArgs& a, hipStream_t stream);
 
-// The solution of a batch of n <= SHARED_TILE_N, to the output and the columns' state. pack: space for two
+// A batch of n <= SHARED_TILE_N, to the output and the columns' state, with z0 = P B. pack: space for two
 // packed matrices per group (shared_packed); next: NUM_XCD integers.
 size_t shared_packed(int n);
 size_t shared_tile_workspace(const SharedGroups& s);
-int shared_tile_solve(const SharedGroups& s, double2* pack, double2* vec, int* next, hipStream_t stream);
+int shared_tile_solve(const SharedGroups& s, double2* pack, double2* z0, double2* vec, int* next, hipStream_t stream);
+
+// Mean matrices and their inverses for n <= SHARED_SMALL_N in one launch (vmean may be null).
+constexpr int SHARED_SMALL_N = 128;
+int shared_invert_small(const SharedGroups& s, const double2* mean, const double2* vmean, double2* A0, double2* P,
+                        hipStream_t stream);
 
 }  // namespace dgami

@@ -17,12 +17,15 @@
 
 namespace dgami {
 
-// Shape of a tile kernel: T = nb^2, NC columns, NW wavefronts that share the rows of a product (32 each).
-template <int T_, int NW_>
+// Shape of a tile kernel: T = nb^2, NW wavefronts that share the rows of a product (16 MI each), and sweeps of
+// JB basis vectors in the orthogonalisation.
+template <int T_, int NW_, int MI_>
 struct SharedShape {
   static constexpr int T = T_, NC = 16, NW = NW_, TH = 64 * NW_, RG = TH / NC;
-  static constexpr int PF = 2;  // k-steps that a product loads ahead
-  static constexpr int JB = 4;  // basis vectors of one sweep of the orthogonalisation
+  static constexpr int MI = MI_;
+  static constexpr int PF = MI == 1 ? 4 : 2;  // k-steps that a product loads ahead
+  static constexpr int JB = 4;
+  static constexpr int RB = MI == 1 ? 4 : 8;  // rows of a thread at a time
 };
 
 struct SharedTileArgs {
@@ -39,7 +42,7 @@ template <typename H>
 struct SharedLds {
   double2 red[H::NW][H::JB + 1][H::NC];
   double2 R[SH_ROT][H::NC];     // triangular factor, column j at j (j + 1) / 2
-  double2 h[SH_M][H::NC];       // projections of the current vector; at the end of a cycle the coefficients of X
+  double2 h[SH_M + 1][H::NC];   // projections of the current vector; at the end of a cycle the coefficients of X
   double2 rs[SH_M][H::NC];      // rotations
   double2 gv[SH_M + 1][H::NC];  // rotated residual
   double rc[SH_M][H::NC];
@@ -65,24 +68,159 @@ __host__ __device__ inline int shared_blocks(int n) { return 2 * ((n + 31) / 32)
 __host__ __device__ inline int shared_steps(int n) { return (n + 3) / 4; }
 size_t shared_packed(int n) { return static_cast<size_t>(shared_blocks(n)) * shared_steps(n) * 64; }
 
-// grid (ceil(packed / 256), groups)
-__global__ void __launch_bounds__(256) shared_pack_kernel(const double2* __restrict__ M, double2* __restrict__ out, int n) {
-  const size_t size = static_cast<size_t>(shared_blocks(n)) * shared_steps(n) * 64, e = blockIdx.x * static_cast<size_t>(256) + threadIdx.x;
-  if (e >= size) return;
-  const int nk = shared_steps(n), lane = static_cast<int>(e & 63);
-  const int ks = static_cast<int>((e >> 6) % nk), rb = static_cast<int>((e >> 6) / nk);
-  const int r = 16 * rb + (lane & 15), k = 4 * ks + (lane >> 4);
-  out[blockIdx.y * size + e] = r < n && k < n ? M[blockIdx.y * static_cast<size_t>(n) * n + static_cast<size_t>(r) * n + k]
-                                              : make_double2(0.0, 0.0);
+// Both matrices packed, z0 = P B (sums of P over the frequencies of every orbital pair), and the tile
+// counters cleared. grid (2 ceil(packed / 256) + ceil(n / 4), groups).
+__global__ void __launch_bounds__(256) shared_pack_kernel(SharedGroups s, double2* __restrict__ out, double2* __restrict__ z0,
+                                                          int* __restrict__ next) {
+  const int n = s.a.n, T = s.a.T, nv = s.a.nv, nk = shared_steps(n);
+  const size_t size = static_cast<size_t>(shared_blocks(n)) * nk * 64;
+  const unsigned nb = static_cast<unsigned>((size + 255) / 256);
+  const size_t mat = blockIdx.y * static_cast<size_t>(n) * n;
+  const int lane = threadIdx.x & 63;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < NUM_XCD) next[threadIdx.x] = 0;
+  if (blockIdx.x < 2 * nb) {
+    const bool inv = blockIdx.x >= nb;
+    const size_t e = (blockIdx.x - (inv ? nb : 0)) * static_cast<size_t>(256) + threadIdx.x;
+    if (e >= size) return;
+    const int ks = static_cast<int>((e >> 6) % nk), rb = static_cast<int>((e >> 6) / nk);
+    const int r = 16 * rb + (lane & 15), k = 4 * ks + (lane >> 4);
+    const double2* M = (inv ? s.P : s.A0) + mat;
+    out[((inv ? s.groups : 0) + blockIdx.y) * size + e] =
+        r < n && k < n ? M[static_cast<size_t>(r) * n + k] : make_double2(0.0, 0.0);
+    return;
+  }
+  const int row = (blockIdx.x - 2 * nb) * 4 + (threadIdx.x >> 6);
+  if (row >= n) return;
+  for (int t = 0; t < T; ++t) {
+    const double2* src = s.P + mat + static_cast<size_t>(row) * n + t * nv;
+    double2 acc = make_double2(0.0, 0.0);
+    for (int v = lane; v < nv; v += 64) acc = cadd(acc, src[v]);
+    for (int o = 32; o > 0; o >>= 1) acc = cadd(acc, make_double2(__shfl_xor(acc.x, o), __shfl_xor(acc.y, o)));
+    if (lane == 0) z0[(blockIdx.y * static_cast<size_t>(n) + row) * T + t] = acc;
+  }
+}
+
+// Mean matrices of the groups and their inverses for n <= 32 RA, n <= 16 CB: one workgroup per group holds the
+// matrix in registers (thread (tr, tc) the elements (tr + 32 a, tc + 16 b)) and inverts it in place by
+// Gauss-Jordan steps with partial pivoting, two barriers each: the owners of column k publish it and their
+// best candidate, every wavefront picks the pivot row p from the 32 candidates, its owners publish it.
+// Rows are not moved: row p of step k ends as row k of the inverse, column j as its column p_j. Bound by the
+// chain of n steps (0.8 us each at n = 120); the blocked LU with n right-hand sides took 0.5 ms for 122
+// matrices of n = 120 and 0.45 ms for 28 of n = 108 in about 40 launches.
+template <int RA, int CB>
+__global__ void __launch_bounds__(512) shared_invert_kernel(LadderArgs a, const double2* __restrict__ mean,
+                                                            const double2* __restrict__ vmean, double2* __restrict__ A0,
+                                                            double2* __restrict__ P, int g0) {
+  __shared__ double2 s_col[2][32 * RA];
+  __shared__ double2 s_row[2][16 * CB];
+  __shared__ unsigned s_key[2][32];
+  __shared__ int s_idx[2][32];
+  __shared__ int s_prow[16 * CB], s_krow[32 * RA];
+  const int n = a.n, T = a.T, nv = a.nv, tid = threadIdx.x, tr = tid >> 4, tc = tid & 15, lane = tid & 63;
+  const int grp = g0 + blockIdx.x, chan = grp / a.nw, w = grp - chan * a.nw;
+  const size_t mat = blockIdx.x * static_cast<size_t>(n) * n;
+  const double2* G = a.gamma + static_cast<size_t>(grp) * n * n;
+  double2 x[RA][CB];
+  unsigned used = 0;
+  bool bad = false;
+#pragma unroll
+  for (int r = 0; r < RA; ++r) {
+    const int i = tr + 32 * r, ri = i / nv, vi = i - ri * nv;
+    if (i >= n) used |= 1u << r;
+#pragma unroll
+    for (int b = 0; b < CB; ++b) {
+      const int j = tc + 16 * b, cj = j / nv, vj = j - cj * nv;
+      x[r][b] = make_double2(0.0, 0.0);
+      if (i < n && j < n) {
+        double2 uv = a.u_r[chan * T * T + ri * T + cj];
+        if (vmean) uv = cadd(uv, vmean[chan * T * T + ri * T + cj]);
+        double2 v = cscale(csub(G[static_cast<size_t>(i) * n + j], uv), a.inv_beta2);
+        if (vi == vj) v = cadd(v, mean[(static_cast<size_t>(w) * T * T + ri * T + cj) * nv + vi]);
+        x[r][b] = v;
+        A0[mat + static_cast<size_t>(i) * n + j] = v;
+      }
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < CB; ++b) {
+#pragma unroll 1
+    for (int kk = 0; kk < 16; ++kk) {
+      const int k = 16 * b + kk, buf = k & 1;
+      if (k >= n) break;
+      if (tc == kk) {
+        unsigned best = 0;
+        int idx = tr;
+#pragma unroll
+        for (int r = 0; r < RA; ++r) {
+          s_col[buf][tr + 32 * r] = x[r][b];
+          const double m = cabs1(x[r][b]);
+          const unsigned key = pivot_key(m, !((used >> r) & 1u) && m <= 1.7e308);
+          if (key > best) {
+            best = key;
+            idx = tr + 32 * r;
+          }
+        }
+        s_key[buf][tr] = best;
+        s_idx[buf][tr] = idx;
+      }
+      __syncthreads();
+      const unsigned key = s_key[buf][lane & 31], wkey = wave_max_u32(key);
+      const int first = __ffsll(static_cast<long long>(__ballot(key == wkey))) - 1;
+      const int p = __builtin_amdgcn_readlane(s_idx[buf][lane & 31], first);
+      bad |= wkey == 0u;  // no finite candidate
+      if (tr == (p & 31)) {
+#pragma unroll
+        for (int r = 0; r < RA; ++r)
+          if (r == p >> 5) {
+            used |= 1u << r;
+#pragma unroll
+            for (int c = 0; c < CB; ++c) s_row[buf][tc + 16 * c] = x[r][c];
+          }
+      }
+      if (tid == 0) {
+        s_prow[k] = p;
+        s_krow[p] = k;
+      }
+      __syncthreads();
+      const double2 pinv = cinv(s_row[buf][k]);
+      double2 rv[CB];
+#pragma unroll
+      for (int c = 0; c < CB; ++c) rv[c] = tc + 16 * c == k ? pinv : cmul(s_row[buf][tc + 16 * c], pinv);
+#pragma unroll
+      for (int r = 0; r < RA; ++r) {
+        const double2 f = s_col[buf][tr + 32 * r];
+        const bool prow = tr + 32 * r == p;
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+          const double2 old = tc + 16 * c == k ? make_double2(0.0, 0.0) : x[r][c];
+          x[r][c] = prow ? rv[c] : cfms(old, f, rv[c]);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const double nan = __longlong_as_double(0x7ff8000000000000ll);
+#pragma unroll
+  for (int r = 0; r < RA; ++r)
+#pragma unroll
+    for (int b = 0; b < CB; ++b) {
+      const int i = tr + 32 * r, j = tc + 16 * b;
+      if (i >= n || j >= n) continue;
+      // a singular or non-finite mean matrix: NaN, so that no column of the group converges
+      if (bad)
+        P[mat + static_cast<size_t>(i) * n + j] = make_double2(nan, nan);
+      else
+        P[mat + static_cast<size_t>(s_krow[i]) * n + s_prow[j]] = x[r][b];
+    }
 }
 
 // B <- A B for the tile in LDS: A packed, B [rows][NC] with zero rows up to a multiple of 4. A wavefront
-// owns 32 rows; A comes from L2 in the matrix cores' layout, PF k-steps ahead, and B from LDS, so no barrier
+// owns 16 MI rows; A comes from L2 in the matrix cores' layout, PF k-steps ahead, and B from LDS, so no barrier
 // holds a wavefront up until the result takes B's place.
 template <typename H, bool THREE>
 __device__ __forceinline__ void shared_product(const double2* __restrict__ A, double2* B, int n) {
-  constexpr int MI = 2, PF = H::PF, NC = H::NC;
-  const int lane = threadIdx.x & 63, r0 = 32 * (threadIdx.x >> 6), l16 = lane & 15, kg = lane >> 4;
+  constexpr int MI = H::MI, PF = H::PF, NC = H::NC;
+  const int lane = threadIdx.x & 63, r0 = 16 * MI * (threadIdx.x >> 6), l16 = lane & 15, kg = lane >> 4;
   const int nk = shared_steps(n);
   ZmmaAcc<MI, 1, THREE> acc;
   zmma_zero(acc);
@@ -190,11 +328,46 @@ __device__ __forceinline__ void shared_apply(const SharedGroups& s, SharedLds<H>
   }
 }
 
-// Orthogonalisation of w against V_0 .. V_k, V_(k+1), and the column's Hessenberg matrix (1 + P D(q)
-// projected). w = P D(q) V_k itself is orthogonalised, not V_k + w, so |w - projection|^2 =
-// |w|^2 - sum |h|^2 cancels little, and V and the Hessenberg matrix stay consistent. The threads of row
-// group 0 keep the column's state: they return whether it goes on, and its residual in res. Bound by the two
-// reads of the basis.
+// The column's Hessenberg matrix (1 + P D(q) projected): the rotations of column k, whose projections are in
+// sh.h and whose remainder is hn; returns whether the column goes on, and its residual in res. Called by
+// row group 0 for its columns (live: the column iterates).
+template <typename H>
+__device__ __forceinline__ bool shared_rotate(SharedLds<H>& sh, int col, int k, double hn, bool live, double target,
+                                              double& res) {
+  if (live) {  // row group 0 only
+    const int rk = k * (k + 1) / 2;
+    double2 hj = sh.h[0][col];
+#pragma unroll 1
+    for (int j = 0; j < k; ++j) {
+      double2 h1 = sh.h[j + 1][col];
+      if (j + 1 == k) h1.x += 1.0;
+      const double c = sh.rc[j][col];
+      const double2 sn = sh.rs[j][col];
+      sh.R[rk + j][col] = cfma(cscale(hj, c), sn, h1);
+      hj = cfms(cscale(h1, c), cconj(sn), hj);
+    }
+    if (k == 0) hj.x += 1.0;
+    const double ah = hypot(hj.x, hj.y), r = hypot(ah, hn);
+    const double c = r > 0.0 ? ah / r : 1.0;
+    const double2 ph = ah > 0.0 ? cscale(hj, 1.0 / ah) : make_double2(1.0, 0.0);
+    const double2 sn = cscale(ph, r > 0.0 ? hn / r : 0.0);
+    sh.rc[k][col] = c;
+    sh.rs[k][col] = sn;
+    sh.R[rk + k][col] = cscale(ph, r);
+    const double2 gk = sh.gv[k][col];
+    const double2 gn = cmul(make_double2(-sn.x, sn.y), gk);
+    sh.gv[k][col] = cscale(gk, c);
+    sh.gv[k + 1][col] = gn;
+    res = hypot(gn.x, gn.y);
+    // converged, broken down, or not a number: the column waits for the end of the cycle
+    live = res > target && hn > 0.0 && k + 1 < SH_M;
+  }
+  return live;
+}
+
+// Orthogonalisation of w against V_0 .. V_k, and V_(k+1). w = P D(q) V_k itself is orthogonalised, not
+// V_k + w, so |w - projection|^2 = |w|^2 - sum |h|^2 cancels little, and V and the Hessenberg matrix stay
+// consistent. Bound by the two reads of the basis.
 template <typename H>
 __device__ __forceinline__ bool shared_step(SharedLds<H>& sh, const SharedTile& x, const double2* V, double2* w,
                                             double2* Vn, int n, int stride, int k, bool live, double target,
@@ -233,7 +406,7 @@ __device__ __forceinline__ bool shared_step(SharedLds<H>& sh, const SharedTile& 
   const double hn = sqrt(fmax(left, 0.0));
   const double inv = hn > 1e-150 ? 1.0 / hn : 0.0;
   __syncthreads();  // sh.h
-  constexpr int RB = 8;  // rows of a thread at a time
+  constexpr int RB = H::RB;
 #pragma unroll 1
   for (int i0 = x.rg; i0 < n; i0 += RB * RG) {
     int o[RB];
@@ -258,43 +431,13 @@ __device__ __forceinline__ bool shared_step(SharedLds<H>& sh, const SharedTile& 
         w[o[m]] = y[m];  // D(q) is applied to it there
       }
   }
-  if (live) {  // row group 0 only
-    const int rk = k * (k + 1) / 2;
-    double2 hj = sh.h[0][x.c];
-#pragma unroll 1
-    for (int j = 0; j < k; ++j) {
-      double2 h1 = sh.h[j + 1][x.c];
-      if (j + 1 == k) h1.x += 1.0;
-      const double c = sh.rc[j][x.c];
-      const double2 sn = sh.rs[j][x.c];
-      sh.R[rk + j][x.c] = cfma(cscale(hj, c), sn, h1);
-      hj = cfms(cscale(h1, c), cconj(sn), hj);
-    }
-    if (k == 0) hj.x += 1.0;
-    const double ah = hypot(hj.x, hj.y), r = hypot(ah, hn);
-    const double c = r > 0.0 ? ah / r : 1.0;
-    const double2 ph = ah > 0.0 ? cscale(hj, 1.0 / ah) : make_double2(1.0, 0.0);
-    const double2 sn = cscale(ph, r > 0.0 ? hn / r : 0.0);
-    sh.rc[k][x.c] = c;
-    sh.rs[k][x.c] = sn;
-    sh.R[rk + k][x.c] = cscale(ph, r);
-    const double2 gk = sh.gv[k][x.c];
-    const double2 gn = cmul(make_double2(-sn.x, sn.y), gk);
-    sh.gv[k][x.c] = cscale(gk, c);
-    sh.gv[k + 1][x.c] = gn;
-    res = hypot(gn.x, gn.y);
-    // converged, broken down, or not a number: the column waits for the end of the cycle
-    live = res > target && hn > 0.0 && k + 1 < SH_M;
-  }
-  return live;
+  return shared_rotate<H>(sh, x.c, k, hn, live, target, res);
 }
 
-// X (+)= sum_j y_j V_j over the kmax vectors of the cycle, with y from the column's triangular factor
-// (kd of row group 0: the column's own vectors); returns |X| of the column.
+// The coefficients y of the cycle's vectors, from the column's triangular factor, into sh.h (kd of row
+// group 0: the column's own vectors, of kmax in the tile).
 template <typename H>
-__device__ __forceinline__ double shared_update(SharedLds<H>& sh, const SharedTile& x, const double2* V, double2* X,
-                                                int n, int stride, int kd, int kmax, bool first) {
-  constexpr int RG = H::RG, NC = H::NC;
+__device__ __forceinline__ void shared_coefficients(SharedLds<H>& sh, const SharedTile& x, int kd, int kmax) {
   if (x.rg == 0) {
 #pragma unroll 1
     for (int j = kmax - 1; j >= 0; --j) {
@@ -309,8 +452,16 @@ __device__ __forceinline__ double shared_update(SharedLds<H>& sh, const SharedTi
     }
   }
   __syncthreads();
+}
+
+// X (+)= sum_j y_j V_j over the kmax vectors of the cycle; returns |X| of the column.
+template <typename H>
+__device__ __forceinline__ double shared_update(SharedLds<H>& sh, const SharedTile& x, const double2* V, double2* X,
+                                                int n, int stride, int kd, int kmax, bool first) {
+  constexpr int RG = H::RG, NC = H::NC;
+  shared_coefficients<H>(sh, x, kd, kmax);
   double2 nrm[1] = {make_double2(0.0, 0.0)};
-  constexpr int RB = 8;
+  constexpr int RB = H::RB;
 #pragma unroll 1
   for (int i0 = x.rg; i0 < n; i0 += RB * RG) {
     int o[RB];
@@ -397,6 +548,7 @@ __device__ __forceinline__ void shared_tile(const SharedTileArgs& ta, SharedLds<
     if (cycle == 0) xn = beta0;
     if (!(beta0 <= 1e300)) state = SH_FAIL;  // infinite or NaN
     if (state == SH_RUN && beta0 <= SH_DONE_TOL * xn) state = SH_DONE;
+    if (state == SH_RUN && cycle > 0 && beta0 > SH_STAGNATION * xn) state = SH_FAIL;  // P is no inverse
     const double target = fmax(SH_CYCLE_TOL * beta0, SH_DONE_TOL * xn);
     if (x.rg == 0) sh.gv[0][x.c] = make_double2(beta0, 0.0);
     bool live = state == SH_RUN;
@@ -416,8 +568,8 @@ __device__ __forceinline__ void shared_tile(const SharedTileArgs& ta, SharedLds<
       xn = xnew;
       if (!(xn <= 1e300) || !(res <= 1e300))
         state = SH_FAIL;
-      else if (cycle > 0 && res <= 2.0 * SH_DONE_TOL * xn)
-        state = SH_DONE;  // the residual it started from was formed from A itself
+      else if (cycle > 0 && res <= 2.0 * SH_DONE_TOL * xn && beta0 <= SH_TRUST * xn)
+        state = SH_DONE;
       else if (!(res <= SH_STAGNATION * beta0))
         state = SH_FAIL;
     }
@@ -455,13 +607,14 @@ __global__ void __launch_bounds__(H::TH, WG_PER_CU * H::NW / 4) shared_tile_kern
   }
 }
 
-__global__ void __launch_bounds__(64) shared_clear_kernel(int* __restrict__ next) {
-  if (threadIdx.x < NUM_XCD) next[threadIdx.x] = 0;
+// ---------------------------------------------------------------------------
+// Up to n = 128: four wavefronts of 32 rows and two workgroups per CU, which overlap one another's products and
+// sweeps, where there are tiles for them; with fewer tiles eight wavefronts of 16 rows, each with half the
+// rows to pass over. Up to 256 eight wavefronts of 32 rows.
+static bool tile_pairs(const SharedGroups& s) {
+  return s.a.n <= 128 && static_cast<size_t>(s.groups) * ceil_div(s.N, 16) > 512;
 }
 
-// ---------------------------------------------------------------------------
-// Up to n = 128 four wavefronts hold the rows of a product and two workgroups fit a CU; up to 256
-// eight wavefronts, one workgroup.
 static int tile_workgroups(const SharedGroups& s) {
   const size_t tiles = static_cast<size_t>(s.groups) * ceil_div(s.N, 16);
   return static_cast<int>(std::min<size_t>(s.a.n <= 128 ? 512 : 256, tiles));
@@ -483,20 +636,29 @@ static int tile_launch(const SharedTileArgs& ta, hipStream_t stream) {
 
 template <int T>
 static int tile_launch_t(const SharedTileArgs& ta, hipStream_t stream) {
-  return ta.s.a.n <= 128 ? tile_launch<SharedShape<T, 4>, 2>(ta, stream) : tile_launch<SharedShape<T, 8>, 1>(ta, stream);
+  if (tile_pairs(ta.s)) return tile_launch<SharedShape<T, 4, 2>, 2>(ta, stream);
+  if (ta.s.a.n <= 128) return tile_launch<SharedShape<T, 8, 1>, 1>(ta, stream);
+  return tile_launch<SharedShape<T, 8, 2>, 1>(ta, stream);
 }
 
-int shared_tile_solve(const SharedGroups& s, double2* pack, double2* vec, int* next, hipStream_t stream) {
+int shared_invert_small(const SharedGroups& s, const double2* mean, const double2* vmean, double2* A0, double2* P,
+                        hipStream_t stream) {
+  const dim3 gd(s.groups), bd(512);
+  if (s.a.n <= 64)
+    hipLaunchKernelGGL((shared_invert_kernel<2, 4>), gd, bd, 0, stream, s.a, mean, vmean, A0, P, s.group0);
+  else
+    hipLaunchKernelGGL((shared_invert_kernel<4, 8>), gd, bd, 0, stream, s.a, mean, vmean, A0, P, s.group0);
+  DGAMI_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+int shared_tile_solve(const SharedGroups& s, double2* pack, double2* z0, double2* vec, int* next, hipStream_t stream) {
   const int n = s.a.n;
   const size_t pk = shared_packed(n);
-  double2* Pp = pack + pk * s.groups;
-  hipLaunchKernelGGL(shared_pack_kernel, dim3(ceil_div(pk, 256), s.groups), dim3(256), 0, stream, s.A0, pack, n);
+  hipLaunchKernelGGL(shared_pack_kernel, dim3(2 * ceil_div(pk, 256) + ceil_div(n, 4), s.groups), dim3(256), 0, stream, s,
+                     pack, z0, next);
   DGAMI_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(shared_pack_kernel, dim3(ceil_div(pk, 256), s.groups), dim3(256), 0, stream, s.P, Pp, n);
-  DGAMI_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(shared_clear_kernel, dim3(1), dim3(64), 0, stream, next);
-  DGAMI_HIP_CHECK(hipGetLastError());
-  const SharedTileArgs ta{s, pack, Pp, static_cast<int>(ceil_div(s.N, 16)), vec, next};
+  const SharedTileArgs ta{s, pack, pack + pk * s.groups, static_cast<int>(ceil_div(s.N, 16)), vec, next};
   switch (s.a.T) {
     case 1: return tile_launch_t<1>(ta, stream);
     case 4: return tile_launch_t<4>(ta, stream);

@@ -17,6 +17,12 @@ def say(msg):
     sys.stdout.flush()
 
 
+@pytest.fixture(autouse=True)
+def shared_form(monkeypatch):
+    """The form is taken from far more problems on (ladder_shared.hpp); here wherever it can run."""
+    monkeypatch.setenv("DGAMI_LADDER_SHARED", "1")
+
+
 @pytest.fixture(scope="module")
 def K():
     if not torch.cuda.is_available():
@@ -46,15 +52,24 @@ def _rel(a, b):
 
 @pytest.mark.parametrize("precision", [0, 1, 2])
 @pytest.mark.parametrize("nb,niv,niw,nq,with_v", [
-    (1, 33, 1, 16, False),   # n = 66, the smallest of the rule; 16 columns
+    (1, 1, 1, 2, False),     # n = 2, 2 columns
+    (1, 8, 40, 33, True),    # n = 16, one wavefront's rows; 123 tiles
+    (1, 17, 1, 16, False),   # n = 34, 16 columns
+    (2, 4, 1, 17, True),     # n = 32
+    (1, 32, 90, 95, False),  # n = 64, 546 tiles: two workgroups per CU
     (1, 35, 2, 65, True),    # n = 70, one column in the second tile, V_r
-    (1, 60, 0, 64, False),   # n = 120, exactly one tile
+    (1, 60, 0, 64, False),   # n = 120, exactly four tiles
+    (1, 64, 0, 20, True),    # n = 128, the largest of four-wavefront tiles
+    (1, 65, 0, 20, False),   # n = 130
     (2, 9, 1, 17, False),    # n = 72, 68 columns: a q-point in both tiles' range
     (2, 14, 1, 16, True),    # n = 112
     (3, 4, 2, 16, False),    # n = 72, 9 right-hand sides that cross the tiles
     (3, 9, 0, 23, True),     # n = 162
     (4, 3, 0, 17, True),     # n = 96, 16 right-hand sides
+    (4, 8, 0, 17, False),    # n = 256, the largest of the tiles
+    (1, 129, 0, 65, True),   # n = 258, the large form
     (2, 33, 0, 19, False),   # n = 264
+    (3, 15, 1, 16, True),    # n = 270
 ])
 def test_shared_ladder_matches_oracle(K, nb, niv, niw, nq, with_v, precision):
     say(f"shared ladder nb={nb} niv={niv} niw={niw} nq={nq} n={nb * nb * 2 * niv} V={with_v} precision={precision}")
@@ -67,7 +82,7 @@ def test_shared_ladder_matches_oracle(K, nb, niv, niw, nq, with_v, precision):
     assert _rel(K.qf_to_ref4(out[0], nb).cpu().numpy(), ref) < (1e-10 if precision == 0 else 1e-8)
 
 
-@pytest.mark.parametrize("nb,niv,nq", [(1, 40, 20), (2, 20, 18)])  # n = 80: column kernel; n = 160: blocked LU
+@pytest.mark.parametrize("nb,niv,nq", [(1, 40, 20), (2, 20, 18), (2, 33, 16)])  # n = 80: column kernel; 160, 264: blocked LU
 def test_unconverged_problems_take_the_lu(K, nb, niv, nq):
     """chi0^-1 that differs between the q-points by more than its mean: the iteration does not converge
     and every problem is solved by the LU; one singular matrix is reported as the LU reports it."""
