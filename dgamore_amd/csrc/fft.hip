@@ -1,25 +1,24 @@
 // Batched momentum-grid FFTs and the two-point layout transform.
 //
 // One workgroup transforms one [nx][ny][nz] slab entirely in LDS (mixed-radix
-// Stockham, radices 2/3/4/5). Grids of the hot path are at most 64x64 points
-// (64 KiB of complex128), so the slab never leaves LDS between passes.
+// Stockham). Grids of the hot path are at most 64x64 points (64 KiB of
+// complex128), so the slab never leaves LDS between passes.
 #include "dgami.h"
 #include "dgami_internal.hpp"
 #include "dgami_launch.hpp"
 
 namespace dgami {
 
-__global__ void __launch_bounds__(256) fft_grid_kernel(const double2* __restrict__ in, double2* out, FftPlan3D plan,
-                                                       double sign, double scale) {
+template <bool BACK>
+__global__ void __launch_bounds__(FFT_MAX_THREADS) fft_grid_kernel(const double2* __restrict__ in, double2* out,
+                                                                   FftPlan3D plan, double scale) {
   extern __shared__ double2 smem[];
   double2* buf = smem;
-  double2* tw = smem + plan.ntot;
+  double2* tw = smem + plan.nlds;
   const size_t off = static_cast<size_t>(blockIdx.x) * plan.ntot;
-  fft_twiddles_3d(tw, plan, sign);
-  for (int i = threadIdx.x; i < plan.ntot; i += blockDim.x) buf[i] = in[off + i];
-  __syncthreads();
-  fft_3d_lds(buf, plan, tw, sign);
-  for (int i = threadIdx.x; i < plan.ntot; i += blockDim.x) out[off + i] = cscale(buf[i], scale);
+  fft_twiddles<BACK>(tw, plan);
+  fft_3d<BACK>(buf, plan, tw, FftLoadGrid{in + off, plan.naxis ? plan.ntot / plan.axis[0] : 1});
+  for (int i = threadIdx.x; i < plan.ntot; i += blockDim.x) out[off + i] = cscale(buf[fft_pos(plan, i)], scale);
 }
 
 __global__ void ref2_to_gk_kernel(const double2* __restrict__ in, double2* __restrict__ out, int nk, int nb,
@@ -42,15 +41,14 @@ int launch_fft_grid(const double2* in, double2* out, int64_t batch, int nx, int 
   DGAMI_ARG_CHECK(nx > 0 && ny > 0 && nz > 0 && batch >= 0, "fft: grid sizes must be positive");
   DGAMI_ARG_CHECK(fft_plan_3d(nx, ny, nz, &plan), "fft: grid lengths must factor into 2, 3 and 5");
   DGAMI_ARG_CHECK(sign == 1 || sign == -1, "fft: sign must be +1 or -1");
-  const size_t lds = (plan.ntot + nx + ny + nz) * sizeof(double2);
-  DGAMI_ARG_CHECK(lds <= 160 * 1024, "fft: grid too large for one LDS slab (max ~10000 points)");
+  DGAMI_ARG_CHECK(fft_grid_fits(plan), "fft: grid too large for one workgroup (max 4096 points)");
+  const size_t lds = fft_lds_bytes(plan);
   const int threads = fft_block_threads(plan);
-  DGAMI_ARG_CHECK(threads <= 256, "fft: grid too large for one workgroup (max 4096 points)");
   if (batch == 0) return 0;
   DGAMI_ARG_CHECK(batch < (int64_t(1) << 31), "fft: batch too large");
-  allow_lds(fft_grid_kernel, lds);
-  hipLaunchKernelGGL(fft_grid_kernel, dim3(static_cast<unsigned>(batch)), dim3(threads), lds, stream, in, out, plan,
-                     static_cast<double>(sign), scale);
+  auto kernel = sign == 1 ? fft_grid_kernel<true> : fft_grid_kernel<false>;
+  allow_lds(kernel, lds);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(batch)), dim3(threads), lds, stream, in, out, plan, scale);
   DGAMI_HIP_CHECK(hipGetLastError());
   return 0;
 }

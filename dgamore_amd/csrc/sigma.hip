@@ -21,37 +21,65 @@
 
 namespace dgami {
 
-constexpr int SIG_ACC = 16;  // accumulator elements per thread (N <= 16 * threads)
+// Load of the kernel's transform: K(q) = K_irr(irrk_inv[q]) (conjugated for w < 0), from LDS or
+// memory; an entry of the map outside the kernel's range reads NaN.
+template <typename I>
+struct SigmaLoad {
+  const double2* k;
+  const I* inv;
+  unsigned nq;
+  int rest;
+  bool conj;
+  __device__ __forceinline__ int begin(int f) const { return f; }
+  __device__ __forceinline__ double2 operator()(int f, int x, int) const {
+    const unsigned q = static_cast<unsigned>(inv[x * rest + f]);
+    const double2 v = q < nq ? k[q] : make_double2(__builtin_nan(""), __builtin_nan(""));
+    return conj ? cconj(v) : v;
+  }
+};
 
-__global__ void __launch_bounds__(256) sigma_partial_kernel(const double2* __restrict__ kirr,
-                                                            const int32_t* __restrict__ irrk_inv,
-                                                            const double2* __restrict__ g_r, double2* __restrict__ part,
-                                                            FftPlan3D plan, int nb, int niw, int niv_core, int nvg,
-                                                            int nq, int nchunk, int wper) {
+// What bounds it: the transforms in LDS (two radix stages per axis, 4-5 passes over the slab) and
+// their FP64 arithmetic at the 3 wavefronts per SIMD that 157 registers allow (128 registers spill
+// and take 0.86 ms where this takes 0.72 at 24x24, 3 orbitals, niw = 30, niv = 40; with three stages
+// per axis, run-time divisions and the gather from memory it was 3.08 ms). STAGED keeps the map (16 bits) and the irreducible kernel of the current (w, a, d) in
+// LDS, read once in order; the gather of the full zone then costs no memory access. It pays where
+// the irreducible list is short against the grid; without a reduction (STAGED false) the map is close
+// to the identity and the gather from memory is in order by itself.
+// The blocks that read the same G(R, v - w), i.e. all (i, j) of one v and one w-chunk, are 8 apart:
+// they run on one XCD at about the same time and share its L2.
+template <bool STAGED>
+__global__ void __launch_bounds__(FFT_MAX_THREADS) sigma_partial_kernel(
+    const double2* __restrict__ kirr, const int32_t* __restrict__ irrk_inv, const double2* __restrict__ g_r,
+    double2* __restrict__ part, FftPlan3D plan, int nb, int niw, int niv_core, int nvg, int nq, int nchunk, int wper) {
   extern __shared__ double2 smem[];
   const int N = plan.ntot;
-  double2* buf = smem;
-  double2* tw = smem + N;
-  int* s_inv = reinterpret_cast<int*>(tw + plan.n[0] + plan.n[1] + plan.n[2]);
   const int T = nb * nb;
-  int idx = blockIdx.x;
-  const int chunk = idx % nchunk;
-  idx /= nchunk;
-  const int v = idx % niv_core;
-  idx /= niv_core;
-  const int j = idx % nb;
-  const int i = idx / nb;
+  double2* buf = smem;
+  double2* tw = smem + plan.nlds;
+  double2* s_k = tw + plan.ntw;
+  uint16_t* s_inv = reinterpret_cast<uint16_t*>(s_k + nq);
+  const int vc = blockIdx.x / (8 * T) * 8 + blockIdx.x % 8;  // (v, w-chunk), chunk fastest
+  const int ij = blockIdx.x / 8 % T;
+  if (vc >= niv_core * nchunk) return;
+  const int chunk = vc % nchunk;
+  const int v = vc / nchunk;
+  const int j = ij % nb;
+  const int i = ij / nb;
   const int nvk = 2 * niv_core;
 
-  fft_twiddles_3d(tw, plan, 1.0);
-  for (int r = threadIdx.x; r < N; r += blockDim.x) s_inv[r] = irrk_inv[r];
-  double2 acc[SIG_ACC];
+  fft_twiddles<true>(tw, plan);
+  if constexpr (STAGED)
+    for (int r = threadIdx.x; r < N; r += blockDim.x) {
+      const int q = irrk_inv[r];
+      s_inv[r] = static_cast<uint16_t>(q >= 0 && q < nq ? q : 0xffff);
+    }
+  double2 acc[FFT_MAX_ELEMS];
 #pragma unroll
-  for (int e = 0; e < SIG_ACC; ++e) acc[e] = make_double2(0.0, 0.0);
-  __syncthreads();
+  for (int e = 0; e < FFT_MAX_ELEMS; ++e) acc[e] = make_double2(0.0, 0.0);
 
   const int w_begin = -niw + chunk * wper;
   const int w_end = (w_begin + wper - 1 < niw) ? w_begin + wper - 1 : niw;
+  const int rest = plan.naxis ? N / plan.axis[0] : 1;
   for (int w = w_begin; w <= w_end; ++w) {
     const int aw = w < 0 ? -w : w;
     const int vk = w < 0 ? niv_core - 1 - v : niv_core + v;  // frequency index in the kernel's 2*niv_core box
@@ -59,53 +87,72 @@ __global__ void __launch_bounds__(256) sigma_partial_kernel(const double2* __res
       for (int d = 0; d < nb; ++d) {
         const int blk = ((a * nb + i) * nb + d) * nb + j;  // M order of (o1,o2,o3,o4) = (a,i,j,d)
         const double2* ks = kirr + ((static_cast<size_t>(aw) * T * T + blk) * nvk + vk) * nq;
-        for (int r = threadIdx.x; r < N; r += blockDim.x) {
-          const int qi = s_inv[r];
-          double2 x = (qi >= 0 && qi < nq) ? ks[qi] : make_double2(__builtin_nan(""), __builtin_nan(""));
-          buf[r] = w < 0 ? cconj(x) : x;
+        if constexpr (STAGED) {
+          for (int q = threadIdx.x; q < nq; q += blockDim.x) s_k[q] = ks[q];
+          __syncthreads();
+          fft_3d<true>(buf, plan, tw,
+                       SigmaLoad<uint16_t>{s_k, s_inv, static_cast<unsigned>(nq), rest, w < 0});
+        } else {
+          fft_3d<true>(buf, plan, tw,
+                       SigmaLoad<int32_t>{ks, irrk_inv, static_cast<unsigned>(nq), rest, w < 0});
         }
-        __syncthreads();
-        fft_3d_lds(buf, plan, tw, 1.0);
         const double2* gs = g_r + (static_cast<size_t>(a * nb + d) * nvg + (v - w + niv_core + niw)) * N;
 #pragma unroll
-        for (int e = 0; e < SIG_ACC; ++e) {
+        for (int e = 0; e < FFT_MAX_ELEMS; ++e) {
           const int r = threadIdx.x + e * blockDim.x;
-          if (r < N) acc[e] = cfma(acc[e], gs[r], buf[r]);
+          if (r < N) acc[e] = cfma(acc[e], gs[r], buf[fft_pos(plan, r)]);
         }
-        __syncthreads();
       }
     }
   }
-  double2* dst = part + ((static_cast<size_t>(chunk) * T + i * nb + j) * niv_core + v) * N;
+  double2* dst = part + ((static_cast<size_t>(chunk) * T + ij) * niv_core + v) * N;
 #pragma unroll
-  for (int e = 0; e < SIG_ACC; ++e) {
+  for (int e = 0; e < FFT_MAX_ELEMS; ++e) {
     const int r = threadIdx.x + e * blockDim.x;
     if (r < N) dst[r] = acc[e];
   }
 }
 
-__global__ void __launch_bounds__(256) sigma_final_kernel(const double2* __restrict__ part, double2* __restrict__ sigma,
-                                                          FftPlan3D plan, int nb, int niv_core, int nchunk,
-                                                          double prefactor) {
+// Chunk sums, prefactor, transform to k. The sum over chunks is a chain of loads (16x16, one orbital,
+// 61 chunks: 50 us as one chain per element, 10 us in this form): on a small grid
+// the block holds several groups of threads that each add a share of the chunks in order, and the
+// shares are added in order of the groups.
+__global__ void __launch_bounds__(FFT_MAX_THREADS) sigma_final_kernel(const double2* __restrict__ part,
+                                                                      double2* __restrict__ sigma, FftPlan3D plan,
+                                                                      int nb, int niv_core, int nchunk, int groups,
+                                                                      double prefactor) {
   extern __shared__ double2 smem[];
   const int N = plan.ntot;
-  double2* buf = smem;
-  double2* tw = smem + N;
+  double2* tw = smem;
+  double2* buf = smem + plan.ntw;
+  double2* sum = buf;  // [groups][N]; the transform has read it before it writes
   const int T = nb * nb;
   const int v = blockIdx.x % niv_core;
   const int ij = blockIdx.x / niv_core;
-  fft_twiddles_3d(tw, plan, 1.0);
-  for (int r = threadIdx.x; r < N; r += blockDim.x) {
+  fft_twiddles<true>(tw, plan);
+  const int per = (nchunk + groups - 1) / groups;
+  const size_t cstride = static_cast<size_t>(T) * niv_core * N;
+  for (int idx = threadIdx.x; idx < groups * N; idx += blockDim.x) {
+    const int g = idx / N, r = idx - g * N;
+    const int c1 = (g + 1) * per < nchunk ? (g + 1) * per : nchunk;
+    const double2* src = part + (static_cast<size_t>(ij) * niv_core + v) * N + r;
     double2 s = make_double2(0.0, 0.0);
-    for (int c = 0; c < nchunk; ++c) s = cadd(s, part[((static_cast<size_t>(c) * T + ij) * niv_core + v) * N + r]);
-    buf[r] = cscale(s, prefactor);
+#pragma unroll 8
+    for (int c = g * per; c < c1; ++c) s = cadd(s, src[c * cstride]);
+    sum[idx] = s;
   }
   __syncthreads();
-  fft_3d_lds(buf, plan, tw, 1.0);
+  for (int r = threadIdx.x; r < N; r += blockDim.x) {
+    double2 s = sum[r];
+    for (int g = 1; g < groups; ++g) s = cadd(s, sum[g * N + r]);
+    sum[r] = cscale(s, prefactor);
+  }
+  __syncthreads();
+  fft_3d<true>(buf, plan, tw, FftLoadGrid{sum, plan.naxis ? N / plan.axis[0] : 1});
   const double inv_n = 1.0 / N;
   const int nvs = 2 * niv_core;
   for (int k = threadIdx.x; k < N; k += blockDim.x) {
-    const double2 s = cscale(buf[k], inv_n);
+    const double2 s = cscale(buf[fft_pos(plan, k)], inv_n);
     double2* out = sigma + (static_cast<size_t>(k) * T + ij) * nvs;
     out[niv_core + v] = s;
     out[niv_core - 1 - v] = cconj(s);
@@ -197,9 +244,8 @@ extern "C" int dgami_sigma_from_kernel(int nx, int ny, int nz, int nb, int niw, 
   DGAMI_ARG_CHECK(nx > 0 && ny > 0 && nz > 0 && fft_plan_3d(nx, ny, nz, &plan),
                   "sigma: grid lengths must factor into 2, 3 and 5");
   const int N = plan.ntot;
-  int threads = fft_block_threads(plan);
-  while (threads * SIG_ACC < N) threads += 64;
-  DGAMI_ARG_CHECK(threads <= 256, "sigma: momentum grid too large (max 4096 points)");
+  DGAMI_ARG_CHECK(fft_grid_fits(plan), "sigma: momentum grid too large (max 4096 points)");
+  const int threads = fft_block_threads(plan);
   const int nvg = 2 * (niv_core + niw);
   const size_t gbytes = static_cast<size_t>(nb) * nb * nvg * N * sizeof(double2);
   double2* gk = static_cast<double2*>(workspace(WS_GK, gbytes));
@@ -212,8 +258,8 @@ extern "C" int dgami_sigma_from_kernel(int nx, int ny, int nz, int nb, int niw, 
   if (rc) return rc;
   const int nw_full = 2 * niw + 1;
   const int base = nb * nb * niv_core;
-  // enough workgroups (about 16k) that the gathers of the kernel are hidden: measured at 24x24, 3
-  // orbitals, niw = 30, niv = 40: 5.4 ms with 2k workgroups, 3.7 ms with 16k, 3.9 ms with 64k
+  // enough workgroups (about 16k) that the loads of G and of the kernel are hidden: measured at
+  // 24x24, 3 orbitals, niw = 30, niv = 40: 0.99 ms with 2k workgroups, 0.77 ms with 8k, 0.75 ms with 16k
   int nchunk = (16384 + base - 1) / base;
   if (nchunk > nw_full) nchunk = nw_full;
   if (nchunk < 1) nchunk = 1;
@@ -221,17 +267,21 @@ extern "C" int dgami_sigma_from_kernel(int nx, int ny, int nz, int nb, int niw, 
   nchunk = (nw_full + wper - 1) / wper;
   double2* part = static_cast<double2*>(workspace(WS_SIGMA_PART, static_cast<size_t>(nchunk) * base * N * sizeof(double2)));
   if (!part) return -2;
-  const size_t lds1 = (N + nx + ny + nz) * sizeof(double2) + N * sizeof(int);
-  DGAMI_ARG_CHECK(lds1 <= 160 * 1024, "sigma: momentum grid too large for LDS");
-  allow_lds(sigma_partial_kernel, lds1);
-  hipLaunchKernelGGL(sigma_partial_kernel, dim3(base * nchunk), dim3(threads), lds1, stream,
+  const size_t stage = nq_irr * sizeof(double2) + N * sizeof(uint16_t);
+  const bool staged = nq_irr <= N / 2 && fft_lds_bytes(plan) + stage <= 160 * 1024;
+  const size_t lds1 = fft_lds_bytes(plan) + (staged ? stage : 0);
+  auto partial = staged ? sigma_partial_kernel<true> : sigma_partial_kernel<false>;
+  allow_lds(partial, lds1);
+  const size_t blocks = static_cast<size_t>(ceil_div(static_cast<size_t>(niv_core) * nchunk, 8)) * 8 * nb * nb;
+  hipLaunchKernelGGL(partial, dim3(static_cast<unsigned>(blocks)), dim3(threads), lds1, stream,
                      reinterpret_cast<const double2*>(kernel_irr), irrk_inv, gr, part, plan, nb, niw, niv_core, nvg,
                      nq_irr, nchunk, wper);
   DGAMI_HIP_CHECK(hipGetLastError());
-  const size_t lds2 = (N + nx + ny + nz) * sizeof(double2);
+  const int groups = std::max(1, FFT_MAX_THREADS / N);
+  const size_t lds2 = (plan.ntw + std::max<size_t>(plan.nlds, static_cast<size_t>(groups) * N)) * sizeof(double2);
   allow_lds(sigma_final_kernel, lds2);
-  hipLaunchKernelGGL(sigma_final_kernel, dim3(base), dim3(threads), lds2, stream, part,
-                     reinterpret_cast<double2*>(sigma), plan, nb, niv_core, nchunk, -0.5 / beta / N);
+  hipLaunchKernelGGL(sigma_final_kernel, dim3(base), dim3(FFT_MAX_THREADS), lds2, stream, part,
+                     reinterpret_cast<double2*>(sigma), plan, nb, niv_core, nchunk, groups, -0.5 / beta / N);
   DGAMI_HIP_CHECK(hipGetLastError());
   return 0;
 }
