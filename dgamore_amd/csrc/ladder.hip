@@ -45,7 +45,7 @@ int ladder_solve_fp64(const LadderArgs& a, hipStream_t stream) {
     const int v = ladder_col_variant(a.n, a.T);
     if (v >= 0) return ladder_col_launch(v, a, stream);
   }
-  if (f.empty() && ladder_shared_applies(a, DGAMI_PLAIN_FP64)) return ladder_solve_shared(a, stream);
+  if (f.empty() && ladder_shared_applies(a, DGAMI_PLAIN_FP64)) return ladder_solve_shared(a, DGAMI_PLAIN_FP64, stream);
   if (f.empty()) {
     const int tuned = ladder_tuned_kernel(a.n, a.T, DGAMI_PLAIN_FP64);
     if (tuned >= 0) {
@@ -98,7 +98,7 @@ static int ladder_multi(int nmodels, const dgami_ladder_model* models, int preci
     DGAMI_ARG_CHECK(items < (size_t(1) << 30), "ladder_multi: too many problems in a model");
     const char* force = getenv("DGAMI_LADDER_KERNEL");
     if (!(force && *force) && ladder_shared_applies(a, precision)) {
-      if ((rc = ladder_solve_shared(a, s)) != 0) return rc;
+      if ((rc = ladder_solve_shared(a, precision, s)) != 0) return rc;
     } else if (fp64_reg_choice(a.n, a.T) >= 0)
       small.push_back(a);
     else if ((rc = precision == DGAMI_PLAIN_FP64 ? ladder_solve_fp64(a, s) : ladder_solve_mixed(a, precision, s)) != 0)

@@ -386,7 +386,7 @@ int ladder_solve_mixed(const LadderArgs& a, int precision, hipStream_t stream) {
   DGAMI_ARG_CHECK(precision == DGAMI_MIXED_FP32_IR || precision == DGAMI_MIXED_BF16X3_IR,
                   "ladder: unknown mixed-precision mode");
   // the shared form solves in FP64 whatever the factors' form (its errors are the smaller ones)
-  if (ladder_shared_applies(a, precision)) return ladder_solve_shared(a, stream);
+  if (ladder_shared_applies(a, precision)) return ladder_solve_shared(a, precision, stream);
   // the split-BF16 factors carry ~2^-16 relative error per product instead of 2^-24, so
   // each refinement step gains fewer digits and more steps may be needed
   const int max_solves = precision == DGAMI_MIXED_BF16X3_IR ? MIXED_MAX_SOLVES_BF16 : MIXED_MAX_SOLVES_FP32;

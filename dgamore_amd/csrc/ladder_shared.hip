@@ -28,6 +28,7 @@
 #include "dgami_launch.hpp"
 #include "ladder_common.hpp"
 #include "ladder_shared.hpp"
+#include "cgemm.hpp"
 #include "zgemm.hpp"
 
 namespace dgami {
@@ -39,12 +40,18 @@ int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream);
 constexpr int SH_TN = ZG_TN;       // columns of a workgroup, and of a tile of the products
 constexpr int SH_WAVES = 4;        // wavefronts of a workgroup, which share the rows of its columns
 
+// S: type of the Krylov basis and of what it is multiplied with.
+template <typename S>
 struct SharedArgs : SharedGroups {
+  typedef S Scalar;
   int ntile;              // tiles of SH_TN columns
   size_t cols;            // columns of the batch
-  double2* V;             // [SH_M + 1][groups][n][N] Krylov basis
-  double2* u;             // operand of the products [groups][n][N]
-  double2* g;             // their result
+  const S* ps;            // P and D(q) in S (the originals where S is double2)
+  const S* ds;
+  S* V;                   // [SH_M + 1][groups][n][N] Krylov basis
+  S* u;                   // operand of the products [groups][n][N]
+  S* g;                   // their result
+  double2* ax;            // A0 X [groups][n][N] (where S is double2: g)
   double2* X;             // solution
   double2* sums;          // [groups][T][N] sums over v of the vector D(q) is applied to (with dv)
   // per column, column fastest
@@ -60,6 +67,35 @@ struct SharedArgs : SharedGroups {
   int* tile_run;          // [groups][ntile] 1 while the tile has a running column
   int* tile_live;         // [groups][ntile] 1 while the tile has a column iterating in this cycle
 };
+
+// Ends of a cycle and of the iteration, by the type of the basis (ladder_shared.hpp).
+template <typename S>
+struct SharedTol {
+  static constexpr double cycle = SH_CYCLE_TOL, done = SH_DONE_TOL, trust = SH_TRUST;
+};
+template <>
+struct SharedTol<float2> {
+  static constexpr double cycle = SH_CYCLE_TOL_C64, done = SH_DONE_TOL_C64, trust = SH_TRUST_C64;
+};
+
+__device__ __forceinline__ double2 sh_wide(double2 x) { return x; }
+__device__ __forceinline__ double2 sh_wide(float2 x) { return make_double2(x.x, x.y); }
+template <typename S>
+__device__ __forceinline__ S sh_narrow(double2 x) {
+  if constexpr (std::is_same<S, float2>::value)
+    return make_float2(static_cast<float>(x.x), static_cast<float>(x.y));
+  else
+    return x;
+}
+__device__ __forceinline__ float2 sh_zero(float2*) { return make_float2(0.f, 0.f); }
+__device__ __forceinline__ double2 sh_zero(double2*) { return make_double2(0.0, 0.0); }
+
+// Complex64 copy.
+__global__ void __launch_bounds__(256) shared_narrow_kernel(const double2* __restrict__ in, float2* __restrict__ out,
+                                                            size_t count) {
+  const size_t i = blockIdx.x * static_cast<size_t>(256) + threadIdx.x;
+  if (i < count) out[i] = sh_narrow<float2>(in[i]);
+}
 
 // ---------------------------------------------------------------------------
 // D(q) = chi0^-1(q) - mean over q and the mean, one wavefront per (w, block, v).
@@ -134,7 +170,8 @@ struct SharedTile {
   size_t base, col;              // offset of the column in a [groups][n][N] vector, column of the batch
 };
 
-__device__ __forceinline__ SharedTile shared_tile(const SharedArgs& s) {
+template <typename S>
+__device__ __forceinline__ SharedTile shared_tile(const SharedArgs<S>& s) {
   SharedTile x;
   x.grp = blockIdx.x / s.ntile;
   const int tile = blockIdx.x - x.grp * s.ntile;
@@ -162,26 +199,28 @@ __device__ __forceinline__ double2 wave_sum(double2 (&sh)[SH_WAVES][SH_TN], doub
 }
 
 // D(q) of a column's frequency-diagonal part for nb = 1 (row i = v).
-__device__ __forceinline__ const double2* shared_diag(const SharedArgs& s, const SharedTile& x) {
+template <typename S>
+__device__ __forceinline__ const double2* shared_diag(const SharedArgs<S>& s, const SharedTile& x) {
   const int w = (s.group0 + x.grp) % s.a.nw;
   return s.dd + static_cast<size_t>(w) * s.a.n * s.a.nq + x.q;
 }
 
 // Start of a cycle: b = z0 (first) or P r (in s.g); V_0 = b / |b| and the column's state. DIAG
 // (one orbital, no V_r): u = D(q) V_0 here too.
-template <bool DIAG>
-__global__ void __launch_bounds__(256) shared_start_kernel(SharedArgs s, int first) {
+template <typename S, bool DIAG>
+__global__ void __launch_bounds__(256) shared_start_kernel(SharedArgs<S> s, int first) {
   const int tile_id = blockIdx.x;
   if (!first && s.tile_run[tile_id] == 0) return;
   __shared__ double2 sh[SH_WAVES][SH_TN];
   const SharedTile x = shared_tile(s);
   const int n = s.a.n;
-  const double2* b = first ? s.z0 + static_cast<size_t>(x.grp) * n * s.a.T + x.t : s.g + x.base;
-  const size_t stride = first ? s.a.T : s.N;
+  const double2* b = s.z0 + static_cast<size_t>(x.grp) * n * s.a.T + x.t;
+  const S* g = s.g + x.base;
+  auto at = [&](int i) { return first ? b[static_cast<size_t>(i) * s.a.T] : sh_wide(g[static_cast<size_t>(i) * s.N]); };
   double nrm = 0.0;
 #pragma unroll 4
   for (int i = x.wave; i < n; i += SH_WAVES) {
-    const double2 y = b[i * stride];
+    const double2 y = at(i);
     nrm = fma(y.x, y.x, fma(y.y, y.y, nrm));
   }
   nrm = sqrt(wave_sum(sh, make_double2(nrm, 0.0), x).x);
@@ -189,25 +228,25 @@ __global__ void __launch_bounds__(256) shared_start_kernel(SharedArgs s, int fir
   const double2* dd = shared_diag(s, x);
 #pragma unroll 4
   for (int i = x.wave; i < n; i += SH_WAVES) {
-    const double2 v = cscale(b[i * stride], inv);
+    const double2 v = cscale(at(i), inv);
     const size_t o = x.base + static_cast<size_t>(i) * s.N;
-    if (x.in) s.V[o] = v;
+    if (x.in) s.V[o] = sh_narrow<S>(v);
     if constexpr (DIAG) {
-      if (x.in) s.u[o] = cmul(dd[static_cast<size_t>(i) * s.a.nq], v);
+      if (x.in) s.u[o] = sh_narrow<S>(cmul(dd[static_cast<size_t>(i) * s.a.nq], v));
     }
   }
   if (x.wave == 0) {
     int st = first ? SH_RUN : s.state[x.col];
     const double xn = first ? nrm : s.xnorm[x.col];
     if (!(nrm <= 1e300)) st = SH_FAIL;  // infinite or NaN
-    if (st == SH_RUN && nrm <= SH_DONE_TOL * xn) st = SH_DONE;
+    if (st == SH_RUN && nrm <= SharedTol<S>::done * xn) st = SH_DONE;
     if (st == SH_RUN && !first && nrm > SH_STAGNATION * xn) st = SH_FAIL;  // P is no inverse
     const int live = x.in && st == SH_RUN;
     if (x.in) {
       s.state[x.col] = st;
       s.live[x.col] = live;
       s.beta0[x.col] = nrm;
-      s.target[x.col] = fmax(SH_CYCLE_TOL * nrm, SH_DONE_TOL * xn);
+      s.target[x.col] = fmax(SharedTol<S>::cycle * nrm, SharedTol<S>::done * xn);
       s.kdim[x.col] = 0;
       s.gv[x.col] = make_double2(nrm, 0.0);
     }
@@ -221,18 +260,18 @@ __global__ void __launch_bounds__(256) shared_start_kernel(SharedArgs s, int fir
 // DIAG u = D(q) V_(k+1) too), and the column's Hessenberg matrix (1 + P D(q) projected) and
 // residual are updated. |w - projection| comes from |w|^2 - sum |h|^2: w = P D(q) V_k itself is
 // orthogonalised, not V_k + w, so little cancels, and V and the Hessenberg matrix stay consistent.
-template <bool DIAG, int KC>
-__global__ void __launch_bounds__(256) shared_step_kernel(SharedArgs s, int k) {
+template <typename S, bool DIAG, int KC>
+__global__ void __launch_bounds__(256) shared_step_kernel(SharedArgs<S> s, int k) {
   const int tile_id = blockIdx.x;
   if (s.tile_live[tile_id] == 0) return;
   __shared__ double2 sh[SH_WAVES][SH_TN];
   const SharedTile x = shared_tile(s);
   const int n = s.a.n, N = s.N;
   const size_t vec = static_cast<size_t>(s.groups) * n * N;
-  const double2* Vp[KC];
+  const S* Vp[KC];
 #pragma unroll
   for (int j = 0; j < KC; ++j) Vp[j] = s.V + static_cast<size_t>(j <= k ? j : k) * vec + x.base;
-  const double2* w = s.g + x.base;
+  const S* w = s.g + x.base;
   double2 h[KC];
 #pragma unroll
   for (int j = 0; j < KC; ++j) h[j] = make_double2(0.0, 0.0);
@@ -240,13 +279,13 @@ __global__ void __launch_bounds__(256) shared_step_kernel(SharedArgs s, int k) {
 #pragma unroll 2
   for (int i = x.wave; i < n; i += SH_WAVES) {
     const size_t o = static_cast<size_t>(i) * N;
-    const double2 y = w[o];
-    double2 p[KC];
+    const double2 y = sh_wide(w[o]);
+    S p[KC];
 #pragma unroll
     for (int j = 0; j < KC; ++j) p[j] = Vp[j][o];
     nrm = fma(y.x, y.x, fma(y.y, y.y, nrm));
 #pragma unroll
-    for (int j = 0; j < KC; ++j) h[j] = cfma(h[j], cconj(p[j]), y);
+    for (int j = 0; j < KC; ++j) h[j] = cfma(h[j], cconj(sh_wide(p[j])), y);
   }
   nrm = wave_sum(sh, make_double2(nrm, 0.0), x).x;
   double left = nrm;
@@ -259,21 +298,21 @@ __global__ void __launch_bounds__(256) shared_step_kernel(SharedArgs s, int k) {
   const double hn = sqrt(fmax(left, 0.0));
   const double inv = hn > 1e-150 ? 1.0 / hn : 0.0;
   const double2* dd = shared_diag(s, x);
-  double2* Vn = s.V + static_cast<size_t>(k + 1) * vec + x.base;
-  double2* un = s.u + x.base;
+  S* Vn = s.V + static_cast<size_t>(k + 1) * vec + x.base;
+  S* un = s.u + x.base;
 #pragma unroll 2
   for (int i = x.wave; i < n; i += SH_WAVES) {
     const size_t o = static_cast<size_t>(i) * N;
-    double2 y = w[o];
-    double2 p[KC];
+    double2 y = sh_wide(w[o]);
+    S p[KC];
 #pragma unroll
     for (int j = 0; j < KC; ++j) p[j] = Vp[j][o];
 #pragma unroll
-    for (int j = 0; j < KC; ++j) y = cfms(y, h[j], p[j]);
+    for (int j = 0; j < KC; ++j) y = cfms(y, h[j], sh_wide(p[j]));
     y = cscale(y, inv);
-    if (x.in) Vn[o] = y;
+    if (x.in) Vn[o] = sh_narrow<S>(y);
     if constexpr (DIAG) {
-      if (x.in) un[o] = cmul(dd[static_cast<size_t>(i) * s.a.nq], y);
+      if (x.in) un[o] = sh_narrow<S>(cmul(dd[static_cast<size_t>(i) * s.a.nq], y));
     }
   }
   if (x.wave == 0) {
@@ -324,7 +363,8 @@ __global__ void __launch_bounds__(256) shared_step_kernel(SharedArgs s, int k) {
 }
 
 // End of a cycle: X (+)= sum_j y_j V_j with the y of the column's triangular factor, and its state.
-__global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs s, int cycle, int last) {
+template <typename S>
+__global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs<S> s, int cycle, int last) {
   const int tile_id = blockIdx.x;
   if (cycle > 0 && s.tile_run[tile_id] == 0) return;
   __shared__ double2 sh[SH_WAVES][SH_TN];
@@ -359,13 +399,13 @@ __global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs s, int cy
 #pragma unroll 2
     for (int i = x.wave; i < n; i += SH_WAVES) {
       const size_t o = x.base + static_cast<size_t>(i) * N;
-      double2 p[KC];
+      S p[KC];
 #pragma unroll
       for (int j = 0; j < KC; ++j) p[j] = s.V[static_cast<size_t>(j < kmax ? j : 0) * vec + o];
       double2 acc = cycle > 0 ? s.X[o] : make_double2(0.0, 0.0);
 #pragma unroll
       for (int j = 0; j < KC; ++j)
-        if (j < kd) acc = cfma(acc, y[j], p[j]);
+        if (j < kd) acc = cfma(acc, y[j], sh_wide(p[j]));
       nrm = fma(acc.x, acc.x, fma(acc.y, acc.y, nrm));
       if (x.in) s.X[o] = acc;
     }
@@ -386,7 +426,7 @@ __global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs s, int cy
       const double res = hypot(g.x, g.y), b0 = s.beta0[col];
       if (!(xn <= 1e300) || !(res <= 1e300))
         st = SH_FAIL;
-      else if (cycle > 0 && res <= 2.0 * SH_DONE_TOL * xn && b0 <= SH_TRUST * xn)
+      else if (cycle > 0 && res <= 2.0 * SharedTol<S>::done * xn && b0 <= SharedTol<S>::trust * xn)
         st = SH_DONE;
       else if (last || !(res <= SH_STAGNATION * b0))
         st = SH_FAIL;
@@ -402,8 +442,8 @@ __global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs s, int cy
 
 // ---------------------------------------------------------------------------
 // Sums over v of every orbital pair's rows of v ([groups][T][N], for the V_r term). One workgroup per tile.
-template <int T>
-__global__ void __launch_bounds__(256) shared_sums_kernel(SharedArgs s, const double2* __restrict__ v,
+template <int T, typename S, typename V>
+__global__ void __launch_bounds__(256) shared_sums_kernel(SharedArgs<S> s, const V* __restrict__ v,
                                                           const int* __restrict__ tiles) {
   if (tiles[blockIdx.x] == 0) return;
   __shared__ double2 sh[SH_WAVES][SH_TN];
@@ -411,29 +451,36 @@ __global__ void __launch_bounds__(256) shared_sums_kernel(SharedArgs s, const do
   const int nv = s.a.nv, N = s.N;
   for (int c = 0; c < T; ++c) {
     double2 sv = make_double2(0.0, 0.0);
-    for (int vi = x.wave; vi < nv; vi += SH_WAVES) sv = cadd(sv, v[x.base + static_cast<size_t>(c * nv + vi) * N]);
+    for (int vi = x.wave; vi < nv; vi += SH_WAVES) sv = cadd(sv, sh_wide(v[x.base + static_cast<size_t>(c * nv + vi) * N]));
     sv = wave_sum(sh, sv, x);
     if (x.in && x.wave == 0) s.sums[(static_cast<size_t>(x.grp) * T + c) * N + x.e] = sv;
   }
 }
 
-// u = D(q) v, or (RESIDUAL) u = B - A0 v - D(q) v with A0 v in s.g. grid (tiles, ceil(nv / 4)), one
+// u = D(q) v, or (RESIDUAL, in FP64 throughout) u = B - A0 v - D(q) v with A0 v in s.ax. grid (tiles, ceil(nv / 4)), one
 // frequency per wavefront. The blocks of the tile's q-points are staged in LDS, coalesced over q; read
 // by every column from global memory they made this step 5 times slower than its traffic.
-template <int T, bool RESIDUAL>
-__global__ void __launch_bounds__(256) shared_apply_kernel(SharedArgs s, const double2* __restrict__ v,
-                                                           const int* __restrict__ tiles) {
+template <int T, bool RESIDUAL, typename S>
+__global__ void __launch_bounds__(256) shared_apply_kernel(
+    SharedArgs<S> s, const typename std::conditional<RESIDUAL, double2, S>::type* __restrict__ v,
+    const int* __restrict__ tiles) {
+  typedef typename std::conditional<RESIDUAL, double2, S>::type V;
   if (tiles[blockIdx.x] == 0) return;
   constexpr int QT = (63 + T - 1) / T + 1;  // most q-points of a tile
-  __shared__ double2 s_d[SH_WAVES][T * T][QT];
+  __shared__ V s_d[SH_WAVES][T * T][QT];
   const SharedTile x = shared_tile(s);
   const int nv = s.a.nv, nq = s.a.nq, N = s.N;
   const int vi = blockIdx.y * SH_WAVES + x.wave;
   const int g = s.group0 + x.grp, w = g % s.a.nw, chan = g / s.a.nw;
   const int q0 = (blockIdx.x - x.grp * s.ntile) * SH_TN / T;
-  double2 y[T];
+  V y[T];
   if (vi < nv) {
-    const double2* dd = s.dd + (static_cast<size_t>(w) * T * T * nv + vi) * nq;
+    const V* dd;
+    if constexpr (RESIDUAL)
+      dd = s.dd;
+    else
+      dd = s.ds;
+    dd += (static_cast<size_t>(w) * T * T * nv + vi) * nq;
     for (int e = x.lane; e < T * T * QT; e += 64) {
       const int blk = e / QT, qq = e - blk * QT;
       if (q0 + qq < nq) s_d[x.wave][blk][qq] = dd[static_cast<size_t>(blk) * nv * nq + q0 + qq];
@@ -446,21 +493,23 @@ __global__ void __launch_bounds__(256) shared_apply_kernel(SharedArgs s, const d
   const int qq = x.q - q0;
 #pragma unroll
   for (int r = 0; r < T; ++r) {
-    double2 acc = make_double2(0.0, 0.0);
+    V sum = sh_zero(static_cast<V*>(nullptr));
 #pragma unroll
-    for (int c = 0; c < T; ++c) acc = cfma(acc, s_d[x.wave][r * T + c][qq], y[c]);
+    for (int c = 0; c < T; ++c) sum = cfma(sum, s_d[x.wave][r * T + c][qq], y[c]);
+    double2 acc = sh_wide(sum);
     if (s.dv) {
       const double2* dv = s.dv + (static_cast<size_t>(chan) * nq + x.q) * T * T + r * T;
       for (int c = 0; c < T; ++c) acc = cfms(acc, dv[c], s.sums[(static_cast<size_t>(x.grp) * T + c) * N + x.e]);
     }
     const size_t o = x.base + static_cast<size_t>(r * nv + vi) * N;
-    if constexpr (RESIDUAL) acc = csub(make_double2(r == x.t ? 1.0 : 0.0, 0.0), cadd(s.g[o], acc));
-    s.u[o] = acc;
+    if constexpr (RESIDUAL) acc = csub(make_double2(r == x.t ? 1.0 : 0.0, 0.0), cadd(s.ax[o], acc));
+    s.u[o] = sh_narrow<S>(acc);
   }
 }
 
 // out = X / beta, q fastest. grid (n, groups).
-__global__ void __launch_bounds__(256) shared_output_kernel(SharedArgs s) {
+template <typename S>
+__global__ void __launch_bounds__(256) shared_output_kernel(SharedArgs<S> s) {
   const LadderArgs& a = s.a;
   const int i = blockIdx.x, grp = blockIdx.y;
   const double2* X = s.X + (static_cast<size_t>(grp) * a.n + i) * s.N;
@@ -486,56 +535,65 @@ __global__ void __launch_bounds__(256) shared_collect_kernel(SharedGroups s, int
 }
 
 // ---------------------------------------------------------------------------
-template <bool DIAG>
-static int shared_step(const SharedArgs& s, int k, hipStream_t stream) {
+template <bool DIAG, typename S>
+static int shared_step(const SharedArgs<S>& s, int k, hipStream_t stream) {
   const dim3 gd(static_cast<unsigned>(s.groups) * s.ntile), bd(256);
   switch (k / 2) {
-    case 0: hipLaunchKernelGGL((shared_step_kernel<DIAG, 2>), gd, bd, 0, stream, s, k); break;
-    case 1: hipLaunchKernelGGL((shared_step_kernel<DIAG, 4>), gd, bd, 0, stream, s, k); break;
-    case 2: hipLaunchKernelGGL((shared_step_kernel<DIAG, 6>), gd, bd, 0, stream, s, k); break;
-    case 3: hipLaunchKernelGGL((shared_step_kernel<DIAG, 8>), gd, bd, 0, stream, s, k); break;
-    default: hipLaunchKernelGGL((shared_step_kernel<DIAG, SH_M>), gd, bd, 0, stream, s, k); break;
+    case 0: hipLaunchKernelGGL((shared_step_kernel<S, DIAG, 2>), gd, bd, 0, stream, s, k); break;
+    case 1: hipLaunchKernelGGL((shared_step_kernel<S, DIAG, 4>), gd, bd, 0, stream, s, k); break;
+    case 2: hipLaunchKernelGGL((shared_step_kernel<S, DIAG, 6>), gd, bd, 0, stream, s, k); break;
+    case 3: hipLaunchKernelGGL((shared_step_kernel<S, DIAG, 8>), gd, bd, 0, stream, s, k); break;
+    default: hipLaunchKernelGGL((shared_step_kernel<S, DIAG, SH_M>), gd, bd, 0, stream, s, k); break;
   }
   DGAMI_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
-// u = D(q) v, or u = B - A v with A0 v in s.g.
-template <int T>
-static int shared_apply(const SharedArgs& s, const double2* v, bool residual, const int* tiles, hipStream_t stream) {
+// u = D(q) v (RESIDUAL: u = B - A v with A0 v in s.ax).
+template <int T, bool RESIDUAL, typename S, typename V>
+static int shared_apply(const SharedArgs<S>& s, const V* v, const int* tiles, hipStream_t stream) {
   const unsigned nt = static_cast<unsigned>(s.groups) * s.ntile;
   if (s.dv) {
-    hipLaunchKernelGGL((shared_sums_kernel<T>), dim3(nt), dim3(256), 0, stream, s, v, tiles);
+    hipLaunchKernelGGL((shared_sums_kernel<T, S, V>), dim3(nt), dim3(256), 0, stream, s, v, tiles);
     DGAMI_HIP_CHECK(hipGetLastError());
   }
   const dim3 gd(nt, ceil_div(s.a.nv, SH_WAVES)), bd(256);
-  if (residual)
-    hipLaunchKernelGGL((shared_apply_kernel<T, true>), gd, bd, 0, stream, s, v, tiles);
-  else
-    hipLaunchKernelGGL((shared_apply_kernel<T, false>), gd, bd, 0, stream, s, v, tiles);
+  hipLaunchKernelGGL((shared_apply_kernel<T, RESIDUAL, S>), gd, bd, 0, stream, s, v, tiles);
   DGAMI_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
 // C = A B of every group's n x n matrix, tiles without work left out.
-static int shared_product(const SharedArgs& s, const double2* A, const double2* B, const int* tiles, bool three,
-                          hipStream_t stream) {
-  ZgemmArgs g;
+template <typename G, typename S>
+static G shared_operands(const SharedGroups& s, const S* A, const S* B, S* C, const int* tiles) {
+  G g;
   g.A = A;
   g.B = B;
-  g.C = s.g;
+  g.C = C;
   g.M = g.K = g.lda = s.a.n;
   g.N = g.ldb = g.ldc = s.N;
   g.sa = static_cast<long long>(s.a.n) * s.a.n;
   g.sb = g.sc = static_cast<long long>(s.a.n) * s.N;
+  g.tile_active = tiles;
+  return g;
+}
+
+static int shared_product(const SharedGroups& s, const double2* A, const double2* B, double2* C, const int* tiles,
+                          bool three, hipStream_t stream) {
+  ZgemmArgs g = shared_operands<ZgemmArgs>(s, A, B, C, tiles);
   g.alpha = make_double2(1.0, 0.0);
   g.beta = make_double2(0.0, 0.0);
-  g.tile_active = tiles;
   return three ? launch_zgemm<true>(g, s.groups, stream) : launch_zgemm<false>(g, s.groups, stream);
 }
 
-template <int T>
-static int shared_solve(SharedArgs& s, const double2* A0, hipStream_t stream) {
+static int shared_product(const SharedGroups& s, const float2* A, const float2* B, float2* C, const int* tiles, bool,
+                          hipStream_t stream) {
+  static_assert(CG_TN == SH_TN, "the tiles whose activity is tracked");
+  return launch_cgemm(shared_operands<CgemmArgs>(s, A, B, C, tiles), s.groups, stream);
+}
+
+template <int T, typename S>
+static int shared_solve(SharedArgs<S>& s, hipStream_t stream) {
   const dim3 gd(static_cast<unsigned>(s.groups) * s.ntile), bd(256);
   const bool diag = T == 1 && !s.dv;
   const size_t vec = static_cast<size_t>(s.groups) * s.a.n * s.N;
@@ -544,21 +602,21 @@ static int shared_solve(SharedArgs& s, const double2* A0, hipStream_t stream) {
   if ((rc = (x)) != 0) return rc
   for (int cycle = 0; cycle < SH_CYCLES; ++cycle) {
     if (cycle > 0) {
-      DGAMI_STEP(shared_product(s, A0, s.X, s.tile_run, false, stream));
-      DGAMI_STEP(shared_apply<T>(s, s.X, true, s.tile_run, stream));
-      DGAMI_STEP(shared_product(s, s.P, s.u, s.tile_run, true, stream));
+      DGAMI_STEP(shared_product(s, s.A0, s.X, s.ax, s.tile_run, false, stream));
+      DGAMI_STEP((shared_apply<T, true>(s, s.X, s.tile_run, stream)));
+      DGAMI_STEP(shared_product(s, s.ps, s.u, s.g, s.tile_run, true, stream));
     }
     if (diag)
-      hipLaunchKernelGGL((shared_start_kernel<true>), gd, bd, 0, stream, s, cycle == 0 ? 1 : 0);
+      hipLaunchKernelGGL((shared_start_kernel<S, true>), gd, bd, 0, stream, s, cycle == 0 ? 1 : 0);
     else
-      hipLaunchKernelGGL((shared_start_kernel<false>), gd, bd, 0, stream, s, cycle == 0 ? 1 : 0);
+      hipLaunchKernelGGL((shared_start_kernel<S, false>), gd, bd, 0, stream, s, cycle == 0 ? 1 : 0);
     DGAMI_HIP_CHECK(hipGetLastError());
     for (int k = 0; k < SH_M; ++k) {
-      if (!diag) DGAMI_STEP(shared_apply<T>(s, s.V + k * vec, false, s.tile_live, stream));
-      DGAMI_STEP(shared_product(s, s.P, s.u, s.tile_live, true, stream));
+      if (!diag) DGAMI_STEP((shared_apply<T, false>(s, s.V + k * vec, s.tile_live, stream)));
+      DGAMI_STEP(shared_product(s, s.ps, s.u, s.g, s.tile_live, true, stream));
       DGAMI_STEP(diag ? shared_step<true>(s, k, stream) : shared_step<false>(s, k, stream));
     }
-    hipLaunchKernelGGL(shared_update_kernel, gd, bd, 0, stream, s, cycle, cycle == SH_CYCLES - 1 ? 1 : 0);
+    hipLaunchKernelGGL((shared_update_kernel<S>), gd, bd, 0, stream, s, cycle, cycle == SH_CYCLES - 1 ? 1 : 0);
     DGAMI_HIP_CHECK(hipGetLastError());
   }
 #undef DGAMI_STEP
@@ -578,26 +636,48 @@ bool ladder_shared_applies(const LadderArgs& a, int precision) {
 }
 
 // A batch by one launch per product and per pass over the basis: vec and st hold the vectors and the
-// columns' data of ng groups.
-static size_t large_vectors(const LadderArgs& a, size_t groups, int N) {
-  return groups * N * (static_cast<size_t>(a.n) * (SH_M + 4) + (a.v_r ? a.T : 0));
+// columns' data of ng groups. With a complex64 basis (c64) A0 X has its own vector, and P and D(q) are
+// there in complex64 too (in `narrow`, shared_narrow values).
+static size_t large_vectors(const LadderArgs& a, size_t groups, int N, bool c64) {
+  const size_t vec = static_cast<size_t>(a.n) * groups * N, sums = a.v_r ? static_cast<size_t>(a.T) * groups * N : 0;
+  return c64 ? vec * ((SH_M + 3) * sizeof(float2) + 2 * sizeof(double2)) + sums * sizeof(double2)
+             : (vec * (SH_M + 4) + sums) * sizeof(double2);
+}
+static size_t shared_narrow_size(const LadderArgs& a, size_t groups) {
+  return groups * a.n * a.n + static_cast<size_t>(a.nw) * a.T * a.T * a.nv * a.nq;
 }
 static size_t large_state(size_t groups, int N) {
   const size_t per_col = sizeof(double2) * (SH_M + SH_ROT + SH_M + 1) + sizeof(double) * (SH_M + 3) + 2 * sizeof(int);
   return groups * (N * per_col + 2 * ceil_div(N, SH_TN) * sizeof(int));
 }
 
-static int shared_large_solve(const SharedGroups& sg, double2* vec, void* st, hipStream_t stream) {
-  SharedArgs s{};
+template <typename S>
+static int shared_large_solve(const SharedGroups& sg, char* vec, void* st, float2* narrow, hipStream_t stream) {
+  SharedArgs<S> s{};
   static_cast<SharedGroups&>(s) = sg;
   const size_t cols = static_cast<size_t>(s.groups) * s.N, used = cols * s.a.n;
   s.ntile = static_cast<int>(ceil_div(s.N, SH_TN));
   s.cols = cols;
-  s.V = vec;
+  s.X = reinterpret_cast<double2*>(vec);
+  s.sums = s.X + used;
+  double2* end = s.sums + (s.a.v_r ? cols * s.a.T : 0);
+  if constexpr (std::is_same<S, float2>::value) {
+    s.ax = end;
+    end += used;
+    const size_t nn = static_cast<size_t>(s.groups) * s.a.n * s.a.n;
+    s.ds = narrow;
+    float2* p = narrow + static_cast<size_t>(s.a.nw) * s.a.T * s.a.T * s.a.nv * s.a.nq;
+    hipLaunchKernelGGL(shared_narrow_kernel, dim3(ceil_div(nn, 256)), dim3(256), 0, stream, s.P, p, nn);
+    DGAMI_HIP_CHECK(hipGetLastError());
+    s.ps = p;
+  } else {
+    s.ds = s.dd;
+    s.ps = s.P;
+  }
+  s.V = reinterpret_cast<S*>(end);
   s.u = s.V + used * (SH_M + 1);
   s.g = s.u + used;
-  s.X = s.g + used;
-  s.sums = s.X + used;
+  if constexpr (std::is_same<S, double2>::value) s.ax = s.g;
   s.rs = static_cast<double2*>(st);
   s.R = s.rs + SH_M * cols;
   s.gv = s.R + SH_ROT * cols;
@@ -611,25 +691,27 @@ static int shared_large_solve(const SharedGroups& sg, double2* vec, void* st, hi
   s.tile_live = s.tile_run + static_cast<size_t>(s.groups) * s.ntile;
   int rc = 0;
   switch (s.a.T) {
-    case 1: rc = shared_solve<1>(s, s.A0, stream); break;
-    case 4: rc = shared_solve<4>(s, s.A0, stream); break;
-    case 9: rc = shared_solve<9>(s, s.A0, stream); break;
-    default: rc = shared_solve<16>(s, s.A0, stream); break;
+    case 1: rc = shared_solve<1>(s, stream); break;
+    case 4: rc = shared_solve<4>(s, stream); break;
+    case 9: rc = shared_solve<9>(s, stream); break;
+    default: rc = shared_solve<16>(s, stream); break;
   }
   if (rc) return rc;
-  hipLaunchKernelGGL(shared_output_kernel, dim3(s.a.n, s.groups), dim3(256), 0, stream, s);
+  hipLaunchKernelGGL((shared_output_kernel<S>), dim3(s.a.n, s.groups), dim3(256), 0, stream, s);
   DGAMI_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
-int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
+int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream) {
   const int n = a.n, T = a.T, nq = a.nq, TT = T * T, N = nq * T;
   const size_t G = static_cast<size_t>(a.nchan) * a.nw, nn = static_cast<size_t>(n) * n;
   const size_t items = G * nq;
   const bool tiles = n <= SHARED_TILE_N;
+  const bool c64 = !tiles && precision != DGAMI_PLAIN_FP64;
   const size_t pk = tiles ? shared_packed(n) : 0;
   // groups per batch: matrices and, for large sizes, vectors of at most 24 GiB
-  const size_t per_group = (2 * (nn + pk) + (tiles ? 0 : large_vectors(a, 1, N))) * sizeof(double2);
+  const size_t per_group = 2 * (nn + pk) * sizeof(double2) + (tiles ? 0 : large_vectors(a, 1, N, c64)) +
+                           (c64 ? nn * sizeof(float2) : 0);
   const size_t gb = std::max<size_t>(1, std::min<size_t>({(size_t(24) << 30) / per_group, G, 65535}));
   SharedGroups s{};
   s.a = a;
@@ -639,9 +721,10 @@ int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
   const size_t rows = static_cast<size_t>(a.nw) * TT * a.nv;
   const size_t vsz = a.v_r ? static_cast<size_t>(a.nchan) * TT : 0, dvsz = vsz * nq;
   const size_t szc = rows + rows * nq + vsz + dvsz + gb * (nn + pk) * 2 + gb * n * T;
-  double2* mean = static_cast<double2*>(workspace(WS_SHARED, szc * sizeof(double2)));
-  double2* vec = static_cast<double2*>(
-      workspace(WS_SHARED_VEC, (tiles ? shared_tile_workspace(s) : large_vectors(a, gb, N)) * sizeof(double2)));
+  const size_t nsz = c64 ? shared_narrow_size(a, gb) : 0;
+  double2* mean = static_cast<double2*>(workspace(WS_SHARED, szc * sizeof(double2) + nsz * sizeof(float2)));
+  char* vec = static_cast<char*>(workspace(
+      WS_SHARED_VEC, tiles ? shared_tile_workspace(s) * sizeof(double2) : large_vectors(a, gb, N, c64)));
   const size_t ints = gb * N + NUM_XCD + items + gb + 64;
   char* st = static_cast<char*>(workspace(WS_SHARED_STATE, (tiles ? 0 : large_state(gb, N)) + ints * sizeof(int)));
   if (!mean || !vec || !st) return -2;
@@ -652,6 +735,7 @@ int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
   double2* P = A0 + gb * nn;
   double2* pack = P + gb * nn;
   double2* z0 = pack + 2 * gb * pk;
+  float2* narrow = reinterpret_cast<float2*>(z0 + gb * n * T);  // D(q), P in complex64
   s.dd = dd;
   s.dv = a.v_r ? dv : nullptr;
   s.A0 = A0;
@@ -670,6 +754,10 @@ int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL(shared_vmean_kernel, dim3(static_cast<unsigned>(vsz)), dim3(64), 0, stream, a, vmean, dv);
     DGAMI_HIP_CHECK(hipGetLastError());
   }
+  if (c64) {
+    hipLaunchKernelGGL(shared_narrow_kernel, dim3(ceil_div(rows * nq, 256)), dim3(256), 0, stream, dd, narrow, rows * nq);
+    DGAMI_HIP_CHECK(hipGetLastError());
+  }
   for (size_t g0 = 0; g0 < G; g0 += gb) {
     const int ng = static_cast<int>(std::min(gb, G - g0));
     s.group0 = static_cast<int>(g0);
@@ -686,12 +774,13 @@ int ladder_solve_shared(const LadderArgs& a, hipStream_t stream) {
     }
     if (rc) return rc;
     if (tiles) {
-      rc = shared_tile_solve(s, pack, z0, vec, next, stream);
+      rc = shared_tile_solve(s, pack, z0, reinterpret_cast<double2*>(vec), next, stream);
     } else {
       hipLaunchKernelGGL(shared_rhs_kernel, dim3(ceil_div(static_cast<size_t>(ng) * n, 4)), dim3(256), 0, stream, P, z0,
                          ng * n, n, T, a.nv);
       DGAMI_HIP_CHECK(hipGetLastError());
-      rc = shared_large_solve(s, vec, st, stream);
+      rc = c64 ? shared_large_solve<float2>(s, vec, st, narrow, stream)
+               : shared_large_solve<double2>(s, vec, st, nullptr, stream);
     }
     if (rc) return rc;
     hipLaunchKernelGGL(shared_collect_kernel, dim3(ceil_div(static_cast<size_t>(ng) * nq, 256)), dim3(256), 0, stream, s, list,

@@ -33,6 +33,10 @@ constexpr double SH_DONE_TOL = 2e-16;
 // ... provided that the cycle began at a residual below SH_TRUST of |X|: the preceding cycle then was right
 // to SH_TRUST, so P is the inverse of A0 to SH_TRUST and this cycle's error is at most that part of its start.
 constexpr double SH_TRUST = 1e-7;
+// The same with the basis, P and D(q) in complex64 (the mixed forms above SHARED_TILE_N; X, A0 and the residuals
+// stay in FP64): a cycle can gain five digits, and |X| is wanted to SH_DONE_TOL_C64, four digits beyond what the
+// refinement of the mixed LU asks for.
+constexpr double SH_CYCLE_TOL_C64 = 1e-5, SH_DONE_TOL_C64 = 1e-14, SH_TRUST_C64 = 1e-9;
 // A cycle that leaves more than this of its residual is stagnating.
 constexpr double SH_STAGNATION = 0.3;
 
@@ -53,7 +57,7 @@ struct SharedGroups {
 
 // DGAMI_LADDER_SHARED = 0 / 1: never / wherever the form can run (for comparisons and tests).
 bool ladder_shared_applies(const LadderArgs& a, int precision);
-int ladder_solve_shared(const LadderArgs& a, hipStream_t stream);
+int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream);
 
 // A batch of n <= SHARED_TILE_N, to the output and the columns' state, with z0 = P B. pack: space for two
 // packed matrices per group (shared_packed); next: NUM_XCD integers.

@@ -82,6 +82,29 @@ def test_shared_ladder_matches_oracle(K, nb, niv, niw, nq, with_v, precision):
     assert _rel(K.qf_to_ref4(out[0], nb).cpu().numpy(), ref) < (1e-10 if precision == 0 else 1e-8)
 
 
+@pytest.mark.parametrize("precision", [1, 2])
+@pytest.mark.parametrize("spread", [0.03, 0.15])
+@pytest.mark.parametrize("nb,niv,niw,nq,with_v", [
+    (1, 129, 0, 65, False),  # n = 258, one column in the second tile
+    (1, 129, 0, 65, True),
+    (2, 33, 1, 19, True),    # n = 264
+    (3, 16, 0, 17, False),   # n = 288
+    (4, 9, 0, 17, True),     # n = 288, 272 columns
+    (3, 40, 0, 16, False),   # n = 720
+])
+def test_complex64_basis_matches_the_fp64_form(K, nb, niv, niw, nq, with_v, spread, precision):
+    """The mixed forms above n = 256 iterate in complex64 on FP64 residuals: |X| to 1e-14 times the norm
+    of the inverse of 1 + P D(q), at most ten here, where both forms converge."""
+    say(f"complex64 basis nb={nb} niv={niv} nq={nq} n={nb * nb * 2 * niv} V={with_v} spread={spread}")
+    chi0_inv, gamma, u, v, beta = _case(nb, niv, niw, nq, 7 * nb + niv, spread, with_v)
+    ops = _operands(K, chi0_inv, gamma, u, v if with_v else None)
+    ref, info0 = K.ladder_solve_sum(*ops, beta)
+    out, info = K.ladder_solve_sum(*ops, beta, precision)
+    torch.cuda.synchronize()
+    assert not info.any() and not info0.any()
+    assert float((out - ref).abs().max() / ref.abs().max()) < 1e-11
+
+
 @pytest.mark.parametrize("nb,niv,nq", [(1, 40, 20), (2, 20, 18), (2, 33, 16)])  # n = 80: column kernel; 160, 264: blocked LU
 def test_unconverged_problems_take_the_lu(K, nb, niv, nq):
     """chi0^-1 that differs between the q-points by more than its mean: the iteration does not converge
