@@ -129,23 +129,6 @@ __global__ void __launch_bounds__(64) shared_vmean_kernel(LadderArgs a, double2*
   if (lane == 0) mean[blockIdx.x] = s;
 }
 
-// A0 of the groups [g0, g0 + groups): grid (ceil(n*n/256), groups).
-__global__ void __launch_bounds__(256) shared_matrix_kernel(LadderArgs a, const double2* __restrict__ mean,
-                                                            const double2* __restrict__ vmean,
-                                                            double2* __restrict__ A0, int g0) {
-  const size_t nn = static_cast<size_t>(a.n) * a.n;
-  const size_t e = blockIdx.x * static_cast<size_t>(256) + threadIdx.x;
-  if (e >= nn) return;
-  const int grp = g0 + blockIdx.y, chan = grp / a.nw, w = grp - chan * a.nw;
-  const int i = static_cast<int>(e / a.n), j = static_cast<int>(e - static_cast<size_t>(i) * a.n);
-  const int ri = i / a.nv, vi = i - ri * a.nv, cj = j / a.nv, vj = j - cj * a.nv;
-  double2 uv = a.u_r[chan * a.T * a.T + ri * a.T + cj];
-  if (vmean) uv = cadd(uv, vmean[chan * a.T * a.T + ri * a.T + cj]);
-  double2 x = cscale(csub(a.gamma[grp * nn + e], uv), a.inv_beta2);
-  if (vi == vj) x = cadd(x, mean[(static_cast<size_t>(w) * a.T * a.T + ri * a.T + cj) * a.nv + vi]);
-  A0[blockIdx.y * nn + e] = x;
-}
-
 // z0 = P B: sums of P over the frequencies of every orbital pair. One wavefront per (group, row).
 __global__ void __launch_bounds__(256) shared_rhs_kernel(const double2* __restrict__ P, double2* __restrict__ z0, int rows,
                                                          int n, int T, int nv) {
@@ -710,7 +693,7 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream) 
   const bool c64 = !tiles && precision != DGAMI_PLAIN_FP64;
   const size_t pk = tiles ? shared_packed(n) : 0;
   // groups per batch: matrices and, for large sizes, vectors of at most 24 GiB
-  const size_t per_group = 2 * (nn + pk) * sizeof(double2) + (tiles ? 0 : large_vectors(a, 1, N, c64)) +
+  const size_t per_group = (2 * (nn + pk) + shared_inverse_workspace(n)) * sizeof(double2) + (tiles ? 0 : large_vectors(a, 1, N, c64)) +
                            (c64 ? nn * sizeof(float2) : 0);
   const size_t gb = std::max<size_t>(1, std::min<size_t>({(size_t(24) << 30) / per_group, G, 65535}));
   SharedGroups s{};
@@ -720,12 +703,12 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream) 
 
   const size_t rows = static_cast<size_t>(a.nw) * TT * a.nv;
   const size_t vsz = a.v_r ? static_cast<size_t>(a.nchan) * TT : 0, dvsz = vsz * nq;
-  const size_t szc = rows + rows * nq + vsz + dvsz + gb * (nn + pk) * 2 + gb * n * T;
+  const size_t szc = rows + rows * nq + vsz + dvsz + gb * ((nn + pk) * 2 + n * T + shared_inverse_workspace(n));
   const size_t nsz = c64 ? shared_narrow_size(a, gb) : 0;
   double2* mean = static_cast<double2*>(workspace(WS_SHARED, szc * sizeof(double2) + nsz * sizeof(float2)));
   char* vec = static_cast<char*>(workspace(
       WS_SHARED_VEC, tiles ? shared_tile_workspace(s) * sizeof(double2) : large_vectors(a, gb, N, c64)));
-  const size_t ints = gb * N + NUM_XCD + items + gb + 64;
+  const size_t ints = gb * N + NUM_XCD + items + 64;
   char* st = static_cast<char*>(workspace(WS_SHARED_STATE, (tiles ? 0 : large_state(gb, N)) + ints * sizeof(int)));
   if (!mean || !vec || !st) return -2;
   double2* dd = mean + rows;
@@ -735,7 +718,8 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream) 
   double2* P = A0 + gb * nn;
   double2* pack = P + gb * nn;
   double2* z0 = pack + 2 * gb * pk;
-  float2* narrow = reinterpret_cast<float2*>(z0 + gb * n * T);  // D(q), P in complex64
+  double2* inv = z0 + gb * n * T;
+  float2* narrow = reinterpret_cast<float2*>(inv + gb * shared_inverse_workspace(n));  // D(q), P in complex64
   s.dd = dd;
   s.dv = a.v_r ? dv : nullptr;
   s.A0 = A0;
@@ -745,7 +729,6 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream) 
   int* next = s.state + gb * N;
   int* list = next + NUM_XCD;
   int* count = list + items;
-  int* pinfo = count + 1;  // [gb] of the inversions; a singular mean matrix shows in the columns
 
   hipLaunchKernelGGL(shared_mean_kernel, dim3(ceil_div(rows, 4)), dim3(256), 0, stream, a.chi0_inv, mean, dd,
                      static_cast<int>(rows), nq, count);
@@ -763,15 +746,7 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream) 
     s.group0 = static_cast<int>(g0);
     s.groups = ng;
     int rc = 0;
-    if (n <= SHARED_SMALL_N) {
-      rc = shared_invert_small(s, mean, a.v_r ? vmean : nullptr, A0, P, stream);
-    } else {
-      hipLaunchKernelGGL(shared_matrix_kernel, dim3(ceil_div(nn, 256), ng), dim3(256), 0, stream, a, mean,
-                         a.v_r ? vmean : nullptr, A0, s.group0);
-      DGAMI_HIP_CHECK(hipGetLastError());
-      rc = dgami_invert_dense(ng, n, reinterpret_cast<const dgami_c128*>(A0), reinterpret_cast<dgami_c128*>(P), pinfo,
-                              stream);
-    }
+    rc = shared_inverse(s, mean, a.v_r ? vmean : nullptr, A0, P, inv, stream);
     if (rc) return rc;
     if (tiles) {
       rc = shared_tile_solve(s, pack, z0, reinterpret_cast<double2*>(vec), next, stream);

@@ -65,9 +65,11 @@ size_t shared_packed(int n);
 size_t shared_tile_workspace(const SharedGroups& s);
 int shared_tile_solve(const SharedGroups& s, double2* pack, double2* z0, double2* vec, int* next, hipStream_t stream);
 
-// Mean matrices and their inverses for n <= SHARED_SMALL_N in one launch (vmean may be null).
+// Mean matrices of a batch and their inverses (vmean may be null; ladder_shared_inverse.hip). work: groups times
+// shared_inverse_workspace(n) values. A matrix that cannot be inverted is NaN in P.
 constexpr int SHARED_SMALL_N = 128;
-int shared_invert_small(const SharedGroups& s, const double2* mean, const double2* vmean, double2* A0, double2* P,
-                        hipStream_t stream);
+size_t shared_inverse_workspace(int n);
+int shared_inverse(const SharedGroups& s, const double2* mean, const double2* vmean, double2* A0, double2* P,
+                   double2* work, hipStream_t stream);
 
 }  // namespace dgami

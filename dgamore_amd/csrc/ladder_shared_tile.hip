@@ -5,8 +5,8 @@
 // each tile stops when its own columns have converged. The vector an iteration works on stays in LDS;
 // only the Krylov basis goes through memory, and the matrix comes from L2, where the tiles of a group on one XCD
 // share it. Bound by the reads of the basis (n = 120: matrix cores 28% busy). With a launch per product
-// and per pass, as the large sizes have it, 68442 problems of n = 120 took 7.4 ms (now 4.0) and 1872
-// problems of n = 216 4.8 ms (now 3.1), most of it gaps between about 250 launches.
+// and per pass, as the large sizes have it, 68442 problems of n = 120 took 7.4 ms (now 3.5) and 1872
+// problems of n = 216 4.8 ms (now 2.4), most of it gaps between about 250 launches.
 #include <algorithm>
 
 #include "dgami.h"
@@ -98,120 +98,6 @@ __global__ void __launch_bounds__(256) shared_pack_kernel(SharedGroups s, double
     for (int o = 32; o > 0; o >>= 1) acc = cadd(acc, make_double2(__shfl_xor(acc.x, o), __shfl_xor(acc.y, o)));
     if (lane == 0) z0[(blockIdx.y * static_cast<size_t>(n) + row) * T + t] = acc;
   }
-}
-
-// Mean matrices of the groups and their inverses for n <= 32 RA, n <= 16 CB: one workgroup per group holds the
-// matrix in registers (thread (tr, tc) the elements (tr + 32 a, tc + 16 b)) and inverts it in place by
-// Gauss-Jordan steps with partial pivoting, two barriers each: the owners of column k publish it and their
-// best candidate, every wavefront picks the pivot row p from the 32 candidates, its owners publish it.
-// Rows are not moved: row p of step k ends as row k of the inverse, column j as its column p_j. Bound by the
-// chain of n steps (0.8 us each at n = 120); the blocked LU with n right-hand sides took 0.5 ms for 122
-// matrices of n = 120 and 0.45 ms for 28 of n = 108 in about 40 launches.
-template <int RA, int CB>
-__global__ void __launch_bounds__(512) shared_invert_kernel(LadderArgs a, const double2* __restrict__ mean,
-                                                            const double2* __restrict__ vmean, double2* __restrict__ A0,
-                                                            double2* __restrict__ P, int g0) {
-  __shared__ double2 s_col[2][32 * RA];
-  __shared__ double2 s_row[2][16 * CB];
-  __shared__ unsigned s_key[2][32];
-  __shared__ int s_idx[2][32];
-  __shared__ int s_prow[16 * CB], s_krow[32 * RA];
-  const int n = a.n, T = a.T, nv = a.nv, tid = threadIdx.x, tr = tid >> 4, tc = tid & 15, lane = tid & 63;
-  const int grp = g0 + blockIdx.x, chan = grp / a.nw, w = grp - chan * a.nw;
-  const size_t mat = blockIdx.x * static_cast<size_t>(n) * n;
-  const double2* G = a.gamma + static_cast<size_t>(grp) * n * n;
-  double2 x[RA][CB];
-  unsigned used = 0;
-  bool bad = false;
-#pragma unroll
-  for (int r = 0; r < RA; ++r) {
-    const int i = tr + 32 * r, ri = i / nv, vi = i - ri * nv;
-    if (i >= n) used |= 1u << r;
-#pragma unroll
-    for (int b = 0; b < CB; ++b) {
-      const int j = tc + 16 * b, cj = j / nv, vj = j - cj * nv;
-      x[r][b] = make_double2(0.0, 0.0);
-      if (i < n && j < n) {
-        double2 uv = a.u_r[chan * T * T + ri * T + cj];
-        if (vmean) uv = cadd(uv, vmean[chan * T * T + ri * T + cj]);
-        double2 v = cscale(csub(G[static_cast<size_t>(i) * n + j], uv), a.inv_beta2);
-        if (vi == vj) v = cadd(v, mean[(static_cast<size_t>(w) * T * T + ri * T + cj) * nv + vi]);
-        x[r][b] = v;
-        A0[mat + static_cast<size_t>(i) * n + j] = v;
-      }
-    }
-  }
-#pragma unroll
-  for (int b = 0; b < CB; ++b) {
-#pragma unroll 1
-    for (int kk = 0; kk < 16; ++kk) {
-      const int k = 16 * b + kk, buf = k & 1;
-      if (k >= n) break;
-      if (tc == kk) {
-        unsigned best = 0;
-        int idx = tr;
-#pragma unroll
-        for (int r = 0; r < RA; ++r) {
-          s_col[buf][tr + 32 * r] = x[r][b];
-          const double m = cabs1(x[r][b]);
-          const unsigned key = pivot_key(m, !((used >> r) & 1u) && m <= 1.7e308);
-          if (key > best) {
-            best = key;
-            idx = tr + 32 * r;
-          }
-        }
-        s_key[buf][tr] = best;
-        s_idx[buf][tr] = idx;
-      }
-      __syncthreads();
-      const unsigned key = s_key[buf][lane & 31], wkey = wave_max_u32(key);
-      const int first = __ffsll(static_cast<long long>(__ballot(key == wkey))) - 1;
-      const int p = __builtin_amdgcn_readlane(s_idx[buf][lane & 31], first);
-      bad |= wkey == 0u;  // no finite candidate
-      if (tr == (p & 31)) {
-#pragma unroll
-        for (int r = 0; r < RA; ++r)
-          if (r == p >> 5) {
-            used |= 1u << r;
-#pragma unroll
-            for (int c = 0; c < CB; ++c) s_row[buf][tc + 16 * c] = x[r][c];
-          }
-      }
-      if (tid == 0) {
-        s_prow[k] = p;
-        s_krow[p] = k;
-      }
-      __syncthreads();
-      const double2 pinv = cinv(s_row[buf][k]);
-      double2 rv[CB];
-#pragma unroll
-      for (int c = 0; c < CB; ++c) rv[c] = tc + 16 * c == k ? pinv : cmul(s_row[buf][tc + 16 * c], pinv);
-#pragma unroll
-      for (int r = 0; r < RA; ++r) {
-        const double2 f = s_col[buf][tr + 32 * r];
-        const bool prow = tr + 32 * r == p;
-#pragma unroll
-        for (int c = 0; c < CB; ++c) {
-          const double2 old = tc + 16 * c == k ? make_double2(0.0, 0.0) : x[r][c];
-          x[r][c] = prow ? rv[c] : cfms(old, f, rv[c]);
-        }
-      }
-    }
-  }
-  __syncthreads();
-  const double nan = __longlong_as_double(0x7ff8000000000000ll);
-#pragma unroll
-  for (int r = 0; r < RA; ++r)
-#pragma unroll
-    for (int b = 0; b < CB; ++b) {
-      const int i = tr + 32 * r, j = tc + 16 * b;
-      if (i >= n || j >= n) continue;
-      // a singular or non-finite mean matrix: NaN, so that no column of the group converges
-      if (bad)
-        P[mat + static_cast<size_t>(i) * n + j] = make_double2(nan, nan);
-      else
-        P[mat + static_cast<size_t>(s_krow[i]) * n + s_prow[j]] = x[r][b];
-    }
 }
 
 // B <- A B for the tile in LDS: A packed, B [rows][NC] with zero rows up to a multiple of 4. A wavefront
@@ -639,17 +525,6 @@ static int tile_launch_t(const SharedTileArgs& ta, hipStream_t stream) {
   if (tile_pairs(ta.s)) return tile_launch<SharedShape<T, 4, 2>, 2>(ta, stream);
   if (ta.s.a.n <= 128) return tile_launch<SharedShape<T, 8, 1>, 1>(ta, stream);
   return tile_launch<SharedShape<T, 8, 2>, 1>(ta, stream);
-}
-
-int shared_invert_small(const SharedGroups& s, const double2* mean, const double2* vmean, double2* A0, double2* P,
-                        hipStream_t stream) {
-  const dim3 gd(s.groups), bd(512);
-  if (s.a.n <= 64)
-    hipLaunchKernelGGL((shared_invert_kernel<2, 4>), gd, bd, 0, stream, s.a, mean, vmean, A0, P, s.group0);
-  else
-    hipLaunchKernelGGL((shared_invert_kernel<4, 8>), gd, bd, 0, stream, s.a, mean, vmean, A0, P, s.group0);
-  DGAMI_HIP_CHECK(hipGetLastError());
-  return 0;
 }
 
 int shared_tile_solve(const SharedGroups& s, double2* pack, double2* z0, double2* vec, int* next, hipStream_t stream) {

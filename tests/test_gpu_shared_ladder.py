@@ -105,6 +105,26 @@ def test_complex64_basis_matches_the_fp64_form(K, nb, niv, niw, nq, with_v, spre
     assert float((out - ref).abs().max() / ref.abs().max()) < 1e-11
 
 
+@pytest.mark.parametrize("precision", [0, 2])
+@pytest.mark.parametrize("niv", [80, 130])  # n = 160: tiles; 260: the large form
+def test_singular_leading_block_takes_the_lu(K, niv, precision):
+    """Mean matrices that are regular but whose leading 64 x 64 block vanishes: the block-wise inversion
+    pivots inside its blocks only and has no inverse to offer."""
+    nq = 18
+    say(f"shared ladder, vanishing leading block: n={2 * niv} precision={precision}")
+    chi0_inv, gamma, u, v, beta = _case(1, niv, 0, nq, 3, 0.01, False)
+    mean = chi0_inv.mean(axis=0)[0, 0, 0, 0]  # [w, v]
+    block = u.reshape(()) * np.ones((64, 64)) - beta**2 * np.stack([np.diag(m[:64]) for m in mean])
+    gamma = gamma.copy()
+    gamma[0, 0, 0, 0, :, :64, :64] = block
+    ref = O.ladder_sum_solve(chi0_inv, gamma, u, v, beta)
+    out, info = K.ladder_solve_sum(*_operands(K, chi0_inv, gamma, u, None), beta, precision)
+    torch.cuda.synchronize()
+    assert not info.any()
+    # (no error bound below the conditioning of these matrices is known in advance)
+    assert _rel(K.qf_to_ref4(out[0], 1).cpu().numpy(), ref) < (1e-8 if precision == 0 else 1e-6)
+
+
 @pytest.mark.parametrize("nb,niv,nq", [(1, 40, 20), (2, 20, 18), (2, 33, 16)])  # n = 80: column kernel; 160, 264: blocked LU
 def test_unconverged_problems_take_the_lu(K, nb, niv, nq):
     """chi0^-1 that differs between the q-points by more than its mean: the iteration does not converge
