@@ -27,7 +27,7 @@ enum WorkspaceSlot {
   // work issued on the library's extra stream k (1..MAX_EXTRA_STREAMS) uses its own slots:
   // slot + k * WS_STREAM_STRIDE
   WS_STREAM_STRIDE = 16,
-  // slots of the shared-vertex ladder (beyond the extra streams' ranges)
+  // slots of the shared-vertex ladder (beyond the extra streams' ranges; offset by the stride there too)
   WS_SHARED = 64,       // mean matrices, their inverses and the q-dependent part
   WS_SHARED_VEC = 65,   // Krylov basis and iterates
   WS_SHARED_STATE = 66, // per-column Hessenberg factors and states, list of unconverged problems

@@ -19,6 +19,7 @@ int ladder_reg_launch(int variant, const LadderArgs& a, hipStream_t stream);
 int ladder_col_variant(int n, int nrhs);
 int ladder_col_launch(int variant, const LadderArgs& a, hipStream_t stream);
 int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream);
+int ladder_lanes();
 int ladder_reg_launch_multi(int variant, const LadderMulti& mm, hipStream_t stream);
 
 // Kernel of the plain FP64 solve. The environment variable DGAMI_LADDER_KERNEL (col, reg or
@@ -64,13 +65,15 @@ int ladder_solve_fp64(const LadderArgs& a, hipStream_t stream) {
 namespace dgami {
 
 // Models of a batch: the register-resident ones share launches in FP64 (at n <= 64 a
-// complex64 factorisation would save nothing); the others take the blocked LU in `precision`.
+// complex64 factorisation would save nothing); those for the shared matrix whose LU (for problems that do
+// not converge) needs no workspace are spread over the caller's and the extra streams, since the chains of
+// one model's inversion and tiles leave most of the chip idle; the others run one after the other.
 static int ladder_multi(int nmodels, const dgami_ladder_model* models, int precision, hipStream_t s) {
   DGAMI_ARG_CHECK(nmodels >= 0 && (nmodels == 0 || models), "ladder_multi: null model table");
   DGAMI_ARG_CHECK(precision == DGAMI_PLAIN_FP64 || precision == DGAMI_MIXED_FP32_IR ||
                       precision == DGAMI_MIXED_BF16X3_IR,
                   "ladder_multi: unknown precision mode");
-  std::vector<LadderArgs> small;
+  std::vector<LadderArgs> small, spread;
   int rc = 0;
   for (int m = 0; m < nmodels; ++m) {
     const dgami_ladder_model& md = models[m];
@@ -98,11 +101,22 @@ static int ladder_multi(int nmodels, const dgami_ladder_model* models, int preci
     DGAMI_ARG_CHECK(items < (size_t(1) << 30), "ladder_multi: too many problems in a model");
     const char* force = getenv("DGAMI_LADDER_KERNEL");
     if (!(force && *force) && ladder_shared_applies(a, precision)) {
-      if ((rc = ladder_solve_shared(a, precision, s)) != 0) return rc;
+      if (ladder_col_variant(a.n, a.T) >= 0)
+        spread.push_back(a);
+      else if ((rc = ladder_solve_shared(a, precision, s)) != 0)
+        return rc;
     } else if (fp64_reg_choice(a.n, a.T) >= 0)
       small.push_back(a);
     else if ((rc = precision == DGAMI_PLAIN_FP64 ? ladder_solve_fp64(a, s) : ladder_solve_mixed(a, precision, s)) != 0)
       return rc;
+  }
+  const int nl = std::min(ladder_lanes(), std::max(1, static_cast<int>(spread.size())));
+  hipStream_t lane[1 + MAX_EXTRA_STREAMS] = {s};
+  for (int l = 1; l < nl; ++l)
+    if ((rc = extra_stream_fork(s, l, &lane[l])) != 0) return rc;
+  for (size_t m = 0; m < spread.size(); ++m) {
+    const int l = static_cast<int>(m % nl);
+    if ((rc = ladder_solve_shared(spread[m], precision, lane[l], l * WS_STREAM_STRIDE)) != 0) return rc;
   }
   // the register-resident models, LADDER_MULTI_MAX per launch, in the largest variant of the group
   for (size_t g0 = 0; g0 < small.size(); g0 += LADDER_MULTI_MAX) {
@@ -121,6 +135,8 @@ static int ladder_multi(int nmodels, const dgami_ladder_model* models, int preci
     mm.start[mm.nmodels] = static_cast<int>(total);
     if ((rc = ladder_reg_launch_multi(variant, mm, s)) != 0) return rc;
   }
+  for (int l = 1; l < nl; ++l)
+    if ((rc = extra_stream_join(s, l)) != 0) return rc;
   return 0;
 }
 

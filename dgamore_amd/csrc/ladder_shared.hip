@@ -614,8 +614,9 @@ bool ladder_shared_applies(const LadderArgs& a, int precision) {
   if (v && *v) return std::string(v) == "1";
   if (a.nq < SHARED_MIN_NQ) return false;
   const double ratio = a.n / (3.0 * a.T) + 1.0, work = static_cast<double>(a.nchan) * a.nw * a.nq * ratio;
-  if (a.n <= SHARED_TILE_N && a.T <= 4) return work >= SHARED_MIN_WORK;
-  return ratio >= SHARED_MIN_RATIO && work >= (precision == DGAMI_MIXED_BF16X3_IR ? SHARED_MIN_WORK_BF16 : SHARED_MIN_WORK);
+  if (a.n <= 32) return work >= SHARED_MIN_WORK_N32 && a.T <= 4;
+  if (a.n <= SHARED_TILE_N && a.T <= 4) return work >= (a.T == 1 ? SHARED_MIN_WORK_1 : SHARED_MIN_WORK_4);
+  return ratio >= SHARED_MIN_RATIO && work >= (precision == DGAMI_PLAIN_FP64 ? SHARED_MIN_WORK : SHARED_MIN_WORK_MIXED);
 }
 
 // A batch by one launch per product and per pass over the basis: vec and st hold the vectors and the
@@ -685,7 +686,7 @@ static int shared_large_solve(const SharedGroups& sg, char* vec, void* st, float
   return 0;
 }
 
-int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream) {
+int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, int slot_offset) {
   const int n = a.n, T = a.T, nq = a.nq, TT = T * T, N = nq * T;
   const size_t G = static_cast<size_t>(a.nchan) * a.nw, nn = static_cast<size_t>(n) * n;
   const size_t items = G * nq;
@@ -705,11 +706,11 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream) 
   const size_t vsz = a.v_r ? static_cast<size_t>(a.nchan) * TT : 0, dvsz = vsz * nq;
   const size_t szc = rows + rows * nq + vsz + dvsz + gb * ((nn + pk) * 2 + n * T + shared_inverse_workspace(n));
   const size_t nsz = c64 ? shared_narrow_size(a, gb) : 0;
-  double2* mean = static_cast<double2*>(workspace(WS_SHARED, szc * sizeof(double2) + nsz * sizeof(float2)));
+  double2* mean = static_cast<double2*>(workspace(WS_SHARED + slot_offset, szc * sizeof(double2) + nsz * sizeof(float2)));
   char* vec = static_cast<char*>(workspace(
-      WS_SHARED_VEC, tiles ? shared_tile_workspace(s) * sizeof(double2) : large_vectors(a, gb, N, c64)));
+      WS_SHARED_VEC + slot_offset, tiles ? shared_tile_workspace(s) * sizeof(double2) : large_vectors(a, gb, N, c64)));
   const size_t ints = gb * N + NUM_XCD + items + 64;
-  char* st = static_cast<char*>(workspace(WS_SHARED_STATE, (tiles ? 0 : large_state(gb, N)) + ints * sizeof(int)));
+  char* st = static_cast<char*>(workspace(WS_SHARED_STATE + slot_offset, (tiles ? 0 : large_state(gb, N)) + ints * sizeof(int)));
   if (!mean || !vec || !st) return -2;
   double2* dd = mean + rows;
   double2* vmean = dd + rows * nq;

@@ -9,17 +9,22 @@ namespace dgami {
 
 // The rule: at least SHARED_MIN_NQ q-points share a matrix (its inversion costs three LUs), and there are
 // enough problems for the LU to be past its own latency, by how much more an LU computes per problem than a
-// product: problems x ratio >= SHARED_MIN_WORK with ratio = n / (3 T) + 1. Beyond one or two orbitals of up to
-// n = 256 the ratio itself has to reach SHARED_MIN_RATIO (the iteration's passes and D(q) blocks grow with T),
-// and the split-BF16 LU, twice as fast as the complex128 one, needs more problems to lose. Measured, LU form /
-// shared form in us, U = 2 ... 8. Complex128 below the line: n = 40, 450 problems 117 / 290; n = 120, 450 problems
-// 597 / 725; T = 9: n = 108, 588 problems 703 / 1499; n = 252, 2002 problems 5818 / 6899; n = 360, 5460 problems
-// 34644 / 39856; n = 720, 336 problems 12650 / 16370. Above: n = 40, 1890 problems 276 / 198; n = 64, 1890
-// problems 644 / 328; n = 120, 9702 problems 5095 / 1427; T = 4: n = 256, 2992 problems 8219 / 3502; n = 400, 990
-// problems 8434 / 7238. Split-BF16 below: T = 4, n = 400, 1890 problems 9407 / 10074; T = 9, n = 720, 1638
-// problems 29105 / 35937, 3822 problems 63206 / 67692; above: n = 480, 5712 problems 36712 / 23475; n = 720, 5642 problems 93079 / 86299.
+// product: problems x ratio >= a bound, with ratio = n / (3 T) + 1. With one or two orbitals up to n = 256 the
+// bound is SHARED_MIN_WORK_1 (T = 1) or SHARED_MIN_WORK_4, and SHARED_MIN_WORK_N32 up to n = 32, where the LU is
+// one small register tile; beyond, the ratio itself has to reach SHARED_MIN_RATIO
+// (the passes over the basis and the D(q) blocks grow with T) and the bound is SHARED_MIN_WORK, or
+// SHARED_MIN_WORK_MIXED for the mixed forms, whose LU is the faster one too. Measured, LU / this form in us
+// (beta = 10 ... 40, U = 3 ... 8). T = 1 below: n = 30, 1440 problems 168 / 230; n = 40, 990 problems 161 / 185; n = 96, 392 problems 444 / 563;
+// above: n = 40, 1350 problems 230 / 187; n = 64, 990 problems 384 / 229; n = 120, 450 problems 608 / 472, 68442 problems
+// 38100 / 3530. T = 4 below: n = 32,
+// 1440 problems 203 / 293; n = 48, 1440 problems 323 / 336; above: n = 64, 1440 problems 550 / 379; n = 80, 1170 problems 607 / 456; n = 120, 1440 problems 1072 / 764; n = 216, 540 problems
+// 1588 / 1300. Large, complex128, below: T = 9, n = 252, 560 problems 2207 / 2652; n = 360, 840 problems 5810 / 7940; n = 720,
+// 448 problems 16025 / 15066; above: T = 4, n = 400, 540 problems 5488 / 5309; T = 9, n = 540, 1170 problems
+// 20020 / 15003. Split-BF16 below: T = 9, n = 720, 448 problems 9858 / 10093; above: 840 problems 17125 / 14148,
+// 5642 problems 93079 / 55800; T = 4, n = 320, 840 problems 3658 / 3087.
 constexpr int SHARED_MIN_NQ = 16;
-constexpr double SHARED_MIN_WORK = 25000.0, SHARED_MIN_WORK_BF16 = 120000.0, SHARED_MIN_RATIO = 18.0;
+constexpr double SHARED_MIN_WORK_1 = 17000.0, SHARED_MIN_WORK_4 = 9000.0, SHARED_MIN_WORK_N32 = 30000.0;
+constexpr double SHARED_MIN_WORK = 16000.0, SHARED_MIN_WORK_MIXED = 20000.0, SHARED_MIN_RATIO = 18.0;
 constexpr int SHARED_TILE_N = 256;
 
 constexpr int SH_M = 10;           // Krylov vectors of a cycle
@@ -57,7 +62,8 @@ struct SharedGroups {
 
 // DGAMI_LADDER_SHARED = 0 / 1: never / wherever the form can run (for comparisons and tests).
 bool ladder_shared_applies(const LadderArgs& a, int precision);
-int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream);
+// slot_offset: of the workspaces (k WS_STREAM_STRIDE for work on extra stream k).
+int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, int slot_offset = 0);
 
 // A batch of n <= SHARED_TILE_N, to the output and the columns' state, with z0 = P B. pack: space for two
 // packed matrices per group (shared_packed); next: NUM_XCD integers.

@@ -170,3 +170,22 @@ def test_captured_shared_step_replays_match_eager(K, precision):
         assert float((out - ref).abs().max() / ref.abs().max()) < 1e-13, it
         pipe.graph_sigma.copy_(out)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("precision", [0, 2])
+def test_batch_spreads_its_models_over_streams(K, precision):
+    """Models of a batch in the shared form on the caller's and the extra streams, beside one for the LU
+    (n above the form's one-launch sizes) and one that does not converge: each as in a call of its own."""
+    say(f"batch of shared-form models, precision {precision}")
+    shapes = [(1, 20, 2, 17), (2, 8, 1, 16), (1, 36, 0, 33), (2, 20, 0, 16), (1, 10, 3, 18)]
+    models = []
+    for k, (nb, niv, niw, nq) in enumerate(shapes):
+        chi0_inv, gamma, u, _, beta = _case(nb, niv, niw, nq, 11 + k, 0.03 if k < 4 else 3.0, False)
+        models.append((*_operands(K, chi0_inv, gamma, u, None), beta))
+    for _ in range(2):
+        outs = K.ladder_solve_sum_multi(models, precision=precision)
+        torch.cuda.synchronize()
+        for m, o in zip(models, outs):
+            ref, info = K.ladder_solve_sum(*m, precision)
+            assert not info.any()
+            assert float((o[0] - ref).abs().max() / ref.abs().max()) < (1e-13 if precision == 0 else 1e-9)
