@@ -14,25 +14,49 @@
 namespace dgami {
 
 // ---------------------------------------------------------------------------
-// chi0: full/core frequency sums  (thread per (w, blk, q))
+// Sums over v of x [rows][nv][nq]: full over all, core over [v0, v0 + nvc), both times scale (either may be
+// null). 64 (row, q) per workgroup, whose four wavefronts add a quarter of the frequencies each: one thread per
+// (row, q) left a chain of nv loads (64x64, box 120: 39 us, 16x16, box 40: 15 us; now 13 and 4).
 // ---------------------------------------------------------------------------
-__global__ void chi0_sums_kernel(const double2* __restrict__ chi0, double2* full_sum, double2* core_sum, int nq,
-                                 int nb4, int nw, int nvf, int v0, int nvc, double inv_beta2) {
-  const size_t total = static_cast<size_t>(nw) * nb4 * nq;
-  for (size_t idx = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; idx < total;
-       idx += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const size_t q = idx % nq;
-    const size_t wb = idx / nq;  // w * nb4 + blk
-    const double2* src = chi0 + wb * nvf * nq + q;
-    double2 sf = make_double2(0.0, 0.0), sc = make_double2(0.0, 0.0);
-    for (int v = 0; v < nvf; ++v) {
-      const double2 x = src[static_cast<size_t>(v) * nq];
-      sf = cadd(sf, x);
-      if (v >= v0 && v < v0 + nvc) sc = cadd(sc, x);
+__global__ void __launch_bounds__(256) freq_sums_kernel(const double2* __restrict__ x, double2* __restrict__ full,
+                                                        double2* __restrict__ core, size_t total, int nq, int nv, int v0,
+                                                        int nvc, double scale) {
+  __shared__ double2 s_full[4][64], s_core[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const size_t idx = blockIdx.x * static_cast<size_t>(64) + lane;
+  double2 sf = make_double2(0.0, 0.0), sc = make_double2(0.0, 0.0);
+  if (idx < total) {
+    const size_t row = idx / nq, q = idx - row * nq;
+    const double2* src = x + row * nv * nq + q;
+    const int per = (nv + 3) / 4, v_end = min(nv, (wave + 1) * per);
+#pragma unroll 8
+    for (int v = wave * per; v < v_end; ++v) {
+      const double2 y = src[static_cast<size_t>(v) * nq];
+      sf = cadd(sf, y);
+      if (v >= v0 && v < v0 + nvc) sc = cadd(sc, y);
     }
-    if (full_sum) full_sum[idx] = cscale(sf, inv_beta2);
-    if (core_sum) core_sum[idx] = cscale(sc, inv_beta2);
   }
+  s_full[wave][lane] = sf;
+  s_core[wave][lane] = sc;
+  __syncthreads();
+  if (wave != 0 || idx >= total) return;
+#pragma unroll
+  for (int k = 1; k < 4; ++k) {
+    sf = cadd(sf, s_full[k][lane]);
+    sc = cadd(sc, s_core[k][lane]);
+  }
+  if (full) full[idx] = cscale(sf, scale);
+  if (core) core[idx] = cscale(sc, scale);
+}
+
+static int launch_freq_sums(const double2* x, double2* full, double2* core, size_t rows, int nq, int nv, int v0, int nvc,
+                            double scale, hipStream_t stream) {
+  const size_t total = rows * nq, blocks = (total + 63) / 64;
+  DGAMI_ARG_CHECK(blocks < (size_t(1) << 31), "frequency sums: too many elements");
+  hipLaunchKernelGGL(freq_sums_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, x, full, core, total,
+                     nq, nv, v0, nvc, scale);
+  DGAMI_HIP_CHECK(hipGetLastError());
+  return 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -54,51 +78,58 @@ __global__ void __launch_bounds__(256) chi0_inv_kernel(const double2* __restrict
 #pragma unroll
   for (int c = 0; c < T; ++c)
     m[c] = chi0[((static_cast<size_t>(w) * T * T + r * T + c) * nvf + v0 + v) * nq + q];
-  team_invert<T, TS>(m, lane);
+  int col[T];
+  const int row = team_invert_inplace<T, TS>(m, lane, col);
   if (active && lane < T) {
 #pragma unroll
-    for (int c = 0; c < T; ++c) inv[((static_cast<size_t>(w) * T * T + r * T + c) * nvc + v) * nq + q] = m[c];
+    for (int c = 0; c < T; ++c) inv[((static_cast<size_t>(w) * T * T + row * T + col[c]) * nvc + v) * nq + q] = m[c];
   }
 }
 
 // ---------------------------------------------------------------------------
-// vrg = beta chi0_inv . chi_aux_sum  (team per (w, v, q))
+// vrg = beta chi0_inv . chi_aux_sum, block row of the product per wavefront: lane = element (v, q), the slow
+// index along which the blocks' elements are contiguous; the other operand's block comes from the L1 that the T
+// wavefronts of a workgroup share. Bound by the reads. With a team of 16 lanes per 9 x 9 block, rows passed by
+// shuffles, three orbitals of (nw, nv, nq) = (31, 80, 91) took 0.60 ms (now 0.22) and kernel_r 1.0 ms (now 0.35).
 // ---------------------------------------------------------------------------
-template <int T, int TS>
-__global__ void __launch_bounds__(256) vrg_kernel(const double2* __restrict__ chi0_inv, const double2* __restrict__ aux,
-                                                 double2* __restrict__ vrg, int nq, int nw, int nv, double beta) {
-  const int lane = threadIdx.x % TS;
-  const size_t team = (blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x) / TS;
-  const size_t nteam = static_cast<size_t>(nw) * nv * nq;
-  const bool active = team < nteam;
-  const size_t tt = active ? team : 0;
-  const int q = static_cast<int>(tt % nq);
-  const int v = static_cast<int>((tt / nq) % nv);
-  const int w = static_cast<int>(tt / (static_cast<size_t>(nq) * nv));
-  const int r = lane < T ? lane : 0;
-  double2 a[T], b[T], o[T];
+template <int T>
+constexpr int row_lanes = T == 1 ? 256 : 64;  // elements of a workgroup
+template <int T>
+constexpr int row_count = T == 16 ? 8 : T;  // block rows of a workgroup
+template <int T>
+constexpr int row_unroll = T <= 4 ? T : T <= 9 ? 3 : 1;  // rows of the other operand in flight (registers)
+
+template <int T>
+__global__ void __launch_bounds__(row_lanes<T>* row_count<T>) vrg_kernel(const double2* __restrict__ chi0_inv,
+                                                              const double2* __restrict__ aux,
+                                                              double2* __restrict__ vrg, int nvq, int tiles, double beta) {
+  const int part = blockIdx.x % (T / row_count<T>), tile = blockIdx.x / (T / row_count<T>);
+  const int w = tile / tiles, e = (tile - w * tiles) * row_lanes<T> + threadIdx.x;
+  if (e >= nvq) return;
+  const int r = T == 1 ? 0 : part * row_count<T> + __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const size_t base = static_cast<size_t>(w) * T * T * nvq + e;
+  double2 o[T];
 #pragma unroll
-  for (int c = 0; c < T; ++c) {
-    const size_t off = ((static_cast<size_t>(w) * T * T + r * T + c) * nv + v) * nq + q;
-    a[c] = chi0_inv[off];
-    b[c] = aux[off];
-  }
-  team_matmul<T, TS>(a, b, o);
-  if (active && lane < T) {
+  for (int c = 0; c < T; ++c) o[c] = make_double2(0.0, 0.0);
+#pragma unroll(row_unroll<T>)
+  for (int k = 0; k < T; ++k) {
+    const double2 a = chi0_inv[base + static_cast<size_t>(r * T + k) * nvq];
 #pragma unroll
-    for (int c = 0; c < T; ++c)
-      vrg[((static_cast<size_t>(w) * T * T + r * T + c) * nv + v) * nq + q] = cscale(o[c], beta);
+    for (int c = 0; c < T; ++c) o[c] = cfma(o[c], a, aux[base + static_cast<size_t>(k * T + c) * nvq]);
   }
+#pragma unroll
+  for (int c = 0; c < T; ++c) vrg[base + static_cast<size_t>(r * T + c) * nvq] = cscale(o[c], beta);
 }
 
 // ---------------------------------------------------------------------------
-// chi_phys = ((sum_v aux / beta + full - core)^-1 + u_r + v_r)^-1  (team per (w, q))
+// chi_phys = ((sum_v aux / beta + full - core)^-1 + u_r + v_r)^-1  (team per (w, q)); sum_v aux / beta
+// comes in chi_phys itself
 // ---------------------------------------------------------------------------
 template <int T, int TS>
-__global__ void __launch_bounds__(256) chi_phys_kernel(const double2* __restrict__ aux, const double2* __restrict__ full,
+__global__ void __launch_bounds__(256) chi_phys_kernel(const double2* __restrict__ full,
                                                       const double2* __restrict__ core, const double2* __restrict__ u_r,
                                                       const double2* __restrict__ v_r, double2* __restrict__ chi_phys,
-                                                      int32_t* info, int nq, int nw, int nv, double inv_beta) {
+                                                      int32_t* info, int nq, int nw) {
   const int lane = threadIdx.x % TS;
   const size_t team = (blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x) / TS;
   const size_t nteam = static_cast<size_t>(nw) * nq;
@@ -111,10 +142,7 @@ __global__ void __launch_bounds__(256) chi_phys_kernel(const double2* __restrict
 #pragma unroll
   for (int c = 0; c < T; ++c) {
     const size_t blk = static_cast<size_t>(w) * T * T + r * T + c;
-    double2 s = make_double2(0.0, 0.0);
-    const double2* src = aux + blk * nv * nq + q;
-    for (int v = 0; v < nv; ++v) s = cadd(s, src[static_cast<size_t>(v) * nq]);
-    s = cscale(s, inv_beta);
+    const double2 s = chi_phys[blk * nq + q];
     m[c] = csub(cadd(s, full[blk * nq + q]), core[blk * nq + q]);
   }
   bool sing = team_invert<T, TS>(m, lane);
@@ -133,47 +161,46 @@ __global__ void __launch_bounds__(256) chi_phys_kernel(const double2* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// K_r = u . (vrg - vrg . u . chi_phys - [magn] 2/3 1)  (team per (w, v, q))
+// K_r = u . (vrg - vrg . u . chi_phys - [magn] 2/3 1), as u vrg - ((u vrg) u) chi_phys - [magn] 2/3 u: every
+// row of it is formed from that row of u alone, so no rows pass between lanes. Lanes and wavefronts as in vrg.
 // ---------------------------------------------------------------------------
-template <int T, int TS>
-__global__ void __launch_bounds__(256) kernel_r_kernel(const double2* __restrict__ vrg, const double2* __restrict__ chi_phys,
-                                                      const double2* __restrict__ u_r, const double2* __restrict__ v_r,
-                                                      double2* kernel, int nq, int nw, int nv, int magn, double weight,
-                                                      int accumulate) {
-  const int lane = threadIdx.x % TS;
-  const size_t team = (blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x) / TS;
-  const size_t nteam = static_cast<size_t>(nw) * nv * nq;
-  const bool active = team < nteam;
-  const size_t tt = active ? team : 0;
-  const int q = static_cast<int>(tt % nq);
-  const int v = static_cast<int>((tt / nq) % nv);
-  const int w = static_cast<int>(tt / (static_cast<size_t>(nq) * nv));
-  const int r = lane < T ? lane : 0;
-  double2 g[T], u[T], x[T], t1[T], t2[T];
+template <int T>
+__global__ void __launch_bounds__(row_lanes<T>* row_count<T>) kernel_r_kernel(
+    const double2* __restrict__ vrg, const double2* __restrict__ chi_phys, const double2* __restrict__ u_r,
+    const double2* __restrict__ v_r, double2* __restrict__ kernel, int nq, int nvq, int tiles, int magn,
+    double weight, int accumulate) {
+  const int part = blockIdx.x % (T / row_count<T>), tile = blockIdx.x / (T / row_count<T>);
+  const int w = tile / tiles, e = (tile - w * tiles) * row_lanes<T> + threadIdx.x;
+  if (e >= nvq) return;
+  const int q = e % nq, r = T == 1 ? 0 : part * row_count<T> + __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const size_t base = static_cast<size_t>(w) * T * T * nvq + e;
+  const double2* chi = chi_phys + static_cast<size_t>(w) * T * T * nq + q;
+  const double2* vq = v_r ? v_r + static_cast<size_t>(q) * T * T : nullptr;
+  auto u = [&](int i) { return vq ? cadd(u_r[i], vq[i]) : u_r[i]; };
+  double2 ug[T], o[T];
+#pragma unroll
+  for (int c = 0; c < T; ++c) ug[c] = o[c] = make_double2(0.0, 0.0);
+#pragma unroll(row_unroll<T>)
+  for (int k = 0; k < T; ++k) {
+    const double2 a = u(r * T + k);
+#pragma unroll
+    for (int c = 0; c < T; ++c) ug[c] = cfma(ug[c], a, vrg[base + static_cast<size_t>(k * T + c) * nvq]);
+  }
+#pragma unroll(T <= 4 ? T : 1)
+  for (int k = 0; k < T; ++k) {
+    double2 s = make_double2(0.0, 0.0);  // element k of the row of u vrg u
+#pragma unroll
+    for (int j = 0; j < T; ++j) s = cfma(s, ug[j], u(j * T + k));
+#pragma unroll
+    for (int c = 0; c < T; ++c) o[c] = cfma(o[c], s, chi[static_cast<size_t>(k * T + c) * nq]);
+  }
 #pragma unroll
   for (int c = 0; c < T; ++c) {
-    const size_t blk = static_cast<size_t>(w) * T * T + r * T + c;
-    g[c] = vrg[(blk * nv + v) * nq + q];
-    x[c] = chi_phys[blk * nq + q];
-    double2 uu = u_r[r * T + c];
-    if (v_r) uu = cadd(uu, v_r[static_cast<size_t>(q) * T * T + r * T + c]);
-    u[c] = uu;
-  }
-  team_matmul<T, TS>(g, u, t1);   // vrg . u
-  team_matmul<T, TS>(t1, x, t2);  // vrg . u . chi
-#pragma unroll
-  for (int c = 0; c < T; ++c) {
-    t2[c] = csub(g[c], t2[c]);
-    if (magn && c == r) t2[c].x -= 2.0 / 3.0;
-  }
-  team_matmul<T, TS>(u, t2, t1);  // u . kern
-  if (active && lane < T) {
-#pragma unroll
-    for (int c = 0; c < T; ++c) {
-      const size_t off = ((static_cast<size_t>(w) * T * T + r * T + c) * nv + v) * nq + q;
-      const double2 val = cscale(t1[c], weight);
-      kernel[off] = accumulate ? cadd(kernel[off], val) : val;
-    }
+    double2 x = csub(ug[c], o[c]);
+    if (magn) x = csub(x, cscale(u(r * T + c), 2.0 / 3.0));
+    x = cscale(x, weight);
+    double2* dst = kernel + base + static_cast<size_t>(r * T + c) * nvq;
+    *dst = accumulate ? cadd(*dst, x) : x;
   }
 }
 
@@ -222,11 +249,9 @@ extern "C" int dgami_chi0_prepare(int nq, int nb, int nw, int niv_full, int niv_
   const int nb4 = nb * nb * nb * nb;
   const int nvf = 2 * niv_full, nvc = 2 * niv_core, v0 = niv_full - niv_core;
   if (full_ || core_) {
-    const size_t total = static_cast<size_t>(nw) * nb4 * nq;
-    const unsigned blocks = ceil_div(total, 256) > 65536u ? 65536u : ceil_div(total, 256);
-    hipLaunchKernelGGL(chi0_sums_kernel, dim3(blocks), dim3(256), 0, stream, chi0, reinterpret_cast<double2*>(full_),
-                       reinterpret_cast<double2*>(core_), nq, nb4, nw, nvf, v0, nvc, 1.0 / (beta * beta));
-    DGAMI_HIP_CHECK(hipGetLastError());
+    const int rc = launch_freq_sums(chi0, reinterpret_cast<double2*>(full_), reinterpret_cast<double2*>(core_),
+                                    static_cast<size_t>(nw) * nb4, nq, nvf, v0, nvc, 1.0 / (beta * beta), stream);
+    if (rc) return rc;
   }
   if (chi0_inv_) {
     double2* inv = reinterpret_cast<double2*>(chi0_inv_);
@@ -250,13 +275,19 @@ extern "C" int dgami_vrg_chi_phys(int nq, int nb, int nw, int niv, double beta, 
   DGAMI_ARG_CHECK(nq >= 1 && nw >= 1 && niv >= 1 && beta > 0, "vrg_chi_phys: sizes");
   const int nv = 2 * niv;
   const double2* aux = reinterpret_cast<const double2*>(aux_);
+  const size_t nvq = static_cast<size_t>(nv) * nq;
+  DGAMI_ARG_CHECK(nvq * nw < (size_t(1) << 37), "vrg_chi_phys: too many elements");
   if (vrg_) {
     DGAMI_ARG_CHECK(chi0_inv_ != nullptr, "vrg_chi_phys: vrg needs chi0_inv");
     const double2* inv = reinterpret_cast<const double2*>(chi0_inv_);
     double2* vrg = reinterpret_cast<double2*>(vrg_);
-    const size_t nteam = static_cast<size_t>(nw) * nv * nq;
-#define LAUNCH(T, TS) \
-  hipLaunchKernelGGL((vrg_kernel<T, TS>), dim3(team_blocks<T, TS>(nteam)), dim3(256), 0, stream, inv, aux, vrg, nq, nw, nv, beta)
+#define LAUNCH(T, TS)                                                                                             \
+  {                                                                                                               \
+    const size_t tiles = ceil_div(nvq, row_lanes<T>);                                                             \
+    hipLaunchKernelGGL((vrg_kernel<T>), dim3(static_cast<unsigned>(tiles * nw * (T / row_count<T>))),    \
+                       dim3(row_lanes<T>, row_count<T>), 0, stream, \
+                       inv, aux, vrg, static_cast<int>(nvq), static_cast<int>(tiles), beta);                      \
+  }
     DGAMI_DISPATCH_NB(nb, LAUNCH)
 #undef LAUNCH
     DGAMI_HIP_CHECK(hipGetLastError());
@@ -269,9 +300,12 @@ extern "C" int dgami_vrg_chi_phys(int nq, int nb, int nw, int niv, double beta, 
     const double2* ur = reinterpret_cast<const double2*>(u_r_);
     const double2* vr = reinterpret_cast<const double2*>(v_r_);
     double2* out = reinterpret_cast<double2*>(chi_phys_);
-#define LAUNCH(T, TS)                                                                                                 \
-  hipLaunchKernelGGL((chi_phys_kernel<T, TS>), dim3(team_blocks<T, TS>(nteam)), dim3(256), 0, stream, aux, full, core, \
-                     ur, vr, out, info, nq, nw, nv, 1.0 / beta)
+    const int rc = launch_freq_sums(aux, out, nullptr, static_cast<size_t>(nw) * nb * nb * nb * nb, nq, nv, 0, 0,
+                                    1.0 / beta, stream);
+    if (rc) return rc;
+#define LAUNCH(T, TS)                                                                                            \
+  hipLaunchKernelGGL((chi_phys_kernel<T, TS>), dim3(team_blocks<T, TS>(nteam)), dim3(256), 0, stream, full, core, ur, \
+                     vr, out, info, nq, nw)
     DGAMI_DISPATCH_NB(nb, LAUNCH)
 #undef LAUNCH
     DGAMI_HIP_CHECK(hipGetLastError());
@@ -287,15 +321,21 @@ extern "C" int dgami_kernel_r(int nq, int nb, int nw, int niv, int channel, doub
   DGAMI_ARG_CHECK(channel == 0 || channel == 1, "kernel_r: channel must be 0 (dens) or 1 (magn)");
   DGAMI_ARG_CHECK(nq >= 1 && nw >= 1 && niv >= 1, "kernel_r: sizes");
   const int nv = 2 * niv;
-  const size_t nteam = static_cast<size_t>(nw) * nv * nq;
+  const size_t nvq = static_cast<size_t>(nv) * nq;
+  DGAMI_ARG_CHECK(nvq * nw < (size_t(1) << 37), "kernel_r: too many elements");
   const double2* vrg = reinterpret_cast<const double2*>(vrg_);
   const double2* chi = reinterpret_cast<const double2*>(chi_phys_);
   const double2* ur = reinterpret_cast<const double2*>(u_r_);
   const double2* vr = reinterpret_cast<const double2*>(v_r_);
   double2* ker = reinterpret_cast<double2*>(kernel_);
-#define LAUNCH(T, TS)                                                                                               \
-  hipLaunchKernelGGL((kernel_r_kernel<T, TS>), dim3(team_blocks<T, TS>(nteam)), dim3(256), 0, stream, vrg, chi, ur, \
-                     vr, ker, nq, nw, nv, channel, weight, accumulate)
+#define LAUNCH(T, TS)                                                                                              \
+  {                                                                                                                \
+    const size_t tiles = ceil_div(nvq, row_lanes<T>);                                                              \
+    hipLaunchKernelGGL((kernel_r_kernel<T>), dim3(static_cast<unsigned>(tiles * nw * (T / row_count<T>))),    \
+                       dim3(row_lanes<T>, row_count<T>), 0, stream, \
+                       vrg, chi, ur, vr, ker, nq, static_cast<int>(nvq), static_cast<int>(tiles), channel, weight, \
+                       accumulate);                                                                                \
+  }
   DGAMI_DISPATCH_NB(nb, LAUNCH)
 #undef LAUNCH
   DGAMI_HIP_CHECK(hipGetLastError());

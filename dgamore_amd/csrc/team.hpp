@@ -65,16 +65,43 @@ __device__ __forceinline__ bool team_invert(double2 (&m)[T], int r) {
   return singular;
 }
 
-// Row r of the team product A.B, lane r holding row r of both operands.
+// In-place inverse of the team's block without moving rows: on return lane r (< T) holds in m[c] the element
+// (row, col[c]) of the inverse, with the returned row. A quarter of the shuffles of team_invert (one row
+// broadcast per step; no second matrix, no interchange). A zero pivot counts as zero's inverse zero, as there; a NaN
+// is taken as the pivot, so that all lanes agree on the rows and it spreads over the block.
 template <int T, int TS>
-__device__ __forceinline__ void team_matmul(const double2 (&a)[T], const double2 (&b)[T], double2 (&out)[T]) {
+__device__ __forceinline__ int team_invert_inplace(double2 (&m)[T], int r, int (&col)[T]) {
+  bool used = r >= T;
+  int row = 0;
 #pragma unroll
-  for (int j = 0; j < T; ++j) out[j] = make_double2(0.0, 0.0);
+  for (int k = 0; k < T; ++k) {
+    const double mag = cabs1(m[k]);
+    double val = used ? -1.0 : mag == mag ? mag : __builtin_huge_val();
+    int p = r;
 #pragma unroll
-  for (int c = 0; c < T; ++c) {
+    for (int off = TS / 2; off > 0; off >>= 1) {
+      const double ov = __shfl_xor(val, off, TS);
+      const int oi = __shfl_xor(p, off, TS);
+      if (ov > val || (ov == val && oi < p)) {
+        val = ov;
+        p = oi;
+      }
+    }
+    col[k] = p;
+    const double2 f = m[k];
+    const double2 piv = shfl2(f, p, TS);
+    const double2 pinv = (val > 0.0) ? cinv(piv) : make_double2(0.0, 0.0);
 #pragma unroll
-    for (int j = 0; j < T; ++j) out[j] = cfma(out[j], a[c], shfl2(b[j], c, TS));
+    for (int j = 0; j < T; ++j) {
+      const double2 pr = j == k ? pinv : cmul(shfl2(m[j], p, TS), pinv);
+      m[j] = r == p ? pr : cfms(j == k ? make_double2(0.0, 0.0) : m[j], f, pr);
+    }
+    if (r == p) {
+      used = true;
+      row = k;
+    }
   }
+  return row;
 }
 
 }  // namespace dgami
