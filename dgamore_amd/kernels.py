@@ -194,21 +194,28 @@ def ladder_solve_sum(chi0_inv, gamma_cmp, u_r_m, v_r_m, beta, precision=_lib.PLA
     _lib.call("dgami_ladder_solve_sum", nchan, nq, nb, nw, nv // 2, float(beta), _p(chi0_inv), _p(gamma_cmp),
               _p(u_r_m), _p(v_r_m), int(precision), _p(out), _p(info, torch.int32), _stream())
     if check_info and not capturing():
-        if precision != _lib.PLAIN_FP64:
-            _resolve_fp64(out, info, chi0_inv, gamma_cmp, u_r_m, v_r_m, beta)
-        bad = torch.nonzero(info).cpu().numpy()
-        if len(bad):
-            raise np.linalg.LinAlgError(f"singular ladder matrix at (chan, w, q) = {bad[:8].tolist()}")
+        ladder_check(out, info, (chi0_inv, gamma_cmp, u_r_m, v_r_m, beta), precision)
     return out, info
 
 
-def _resolve_fp64(out, info, chi0_inv, gamma_cmp, u_r_m, v_r_m, beta):
-    """Solve the items whose mixed-precision refinement failed (info < 0) again with the plain
-    FP64 LU, one call per (channel, w) with the failed q-points, and put the results and their
-    info in place."""
-    bad = torch.nonzero(info < 0).cpu().numpy()
-    if not len(bad):
-        return
+def ladder_check(out, info, model, precision=_lib.PLAIN_FP64):
+    """The check of ladder_solve_sum on the results of a call without it: info is read once (this
+    waits for the solve); failed items of the mixed forms are solved again in place, singular
+    matrices raise. Returns whether items were solved again. model: the first five arguments."""
+    host = info.cpu().numpy()
+    again = precision != _lib.PLAIN_FP64 and bool((host < 0).any())
+    if again:
+        _resolve_fp64(out, info, *model, np.argwhere(host < 0))
+        host = info.cpu().numpy()
+    if host.any():
+        raise np.linalg.LinAlgError(f"singular ladder matrix at (chan, w, q) = {np.argwhere(host)[:8].tolist()}")
+    return again
+
+
+def _resolve_fp64(out, info, chi0_inv, gamma_cmp, u_r_m, v_r_m, beta, bad):
+    """Solve the items whose mixed-precision refinement failed (bad: their (channel, w, q)) again with
+    the plain FP64 LU, one call per (channel, w) with the failed q-points, and put the results and
+    their info in place."""
     for c, w in sorted({(int(c), int(w)) for c, w, _ in bad}):
         qs = sorted(int(q) for cc, ww, q in bad if cc == c and ww == w)
         qi = torch.tensor(qs, dtype=torch.long, device=out.device)
@@ -247,12 +254,8 @@ def ladder_solve_sum_multi(models, check_info=True, precision=_lib.PLAIN_FP64):
     else:
         _lib.call("dgami_ladder_solve_sum_multi_prec", len(models), ctypes.addressof(table), int(precision), _stream())
     if check_info and not capturing():
-        for (out, info), (chi0_inv, gamma_cmp, u_r_m, v_r_m, beta) in zip(outs, models):
-            if precision != _lib.PLAIN_FP64:
-                _resolve_fp64(out, info, chi0_inv, gamma_cmp, u_r_m, v_r_m, beta)
-            bad = torch.nonzero(info).cpu().numpy()
-            if len(bad):
-                raise np.linalg.LinAlgError(f"singular ladder matrix at (chan, w, q) = {bad[:8].tolist()}")
+        for (out, info), model in zip(outs, models):
+            ladder_check(out, info, model, precision)
     return outs
 
 

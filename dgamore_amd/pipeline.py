@@ -127,10 +127,31 @@ class SDEPipeline:
         step leaves info in self.last_info for the caller to read after a replay."""
         sigma = self.sigma_dmft if sigma is None else sigma
         front = self.front(sigma, mu)
-        aux, info = K.ladder_solve_sum(front["chi0_inv"], self.gamma, self.u_r, self.v_r, self.m.beta, self.precision,
-                                       check_info=not K.capturing())
+        aux, info = K.ladder_solve_sum(*self.ladder_model(front), self.precision, check_info=False)
+        if self.lambda_correction is not None:  # its root find on the host needs sound susceptibilities
+            K.ladder_check(aux, info, self.ladder_model(front), self.precision)
+        last = self.last
+        new = self.back(front, aux, info, sigma, sigma_old, keep)
+        # info is read when the rest of the step is queued: read before it, the GPU would wait for the
+        # host's launches (16x16, one orbital: 18 of them after the solve)
+        if self.lambda_correction is None and self.resolve([(self, front, aux, info, last)]):
+            new = self.back(self.front(sigma, mu), aux, info, sigma, sigma_old, keep)
         self.last_info = info
-        return self.back(front, aux, info, sigma, sigma_old, keep)
+        return new
+
+    @staticmethod
+    def resolve(solved):
+        """ladder_check of (pipeline, front, aux, info, last) tuples whose steps are queued already
+        (nothing under capture); on an error every pipeline's `last` is put back. Returns whether
+        items of any were solved again, so that the steps have to be formed anew."""
+        if K.capturing():
+            return False
+        try:
+            return any([K.ladder_check(aux, info, p.ladder_model(f), p.precision) for p, f, aux, info, _ in solved])
+        except np.linalg.LinAlgError:
+            for p, _, _, _, last in solved:
+                p.last = last
+            raise
 
     def front(self, sigma, mu=None):
         """G(k), the bubble, chi0^-1 with its sums and the double-counting kernel: everything the
@@ -378,10 +399,19 @@ class ModelBatch:
         mus = [None] * len(self.pipes) if mus is None else mus
         fronts = [p.front(s, mu) for p, s, mu in zip(self.pipes, sigmas, mus)]
         outs = K.ladder_solve_sum_multi([p.ladder_model(f) for p, f in zip(self.pipes, fronts)],
-                                        check_info=not K.capturing(), precision=self.precision)
+                                        check_info=False, precision=self.precision)
+
+        def backs():
+            return [p.back(f, aux, info, s, None, keep)
+                    for p, f, (aux, info), s in zip(self.pipes, fronts, outs, sigmas)]
+
+        solved = [(p, f, aux, info, p.last) for p, f, (aux, info) in zip(self.pipes, fronts, outs)]
+        news = backs()
+        if SDEPipeline.resolve(solved):
+            fronts = [p.front(s, mu) for p, s, mu in zip(self.pipes, sigmas, mus)]
+            news = backs()
         for p, (_, info) in zip(self.pipes, outs):
             p.last_info = info
-        news = [p.back(f, aux, info, s, None, keep) for p, f, (aux, info), s in zip(self.pipes, fronts, outs, sigmas)]
         if scf:
             news = [p.scf_update(n) for p, n in zip(self.pipes, news)]
         return news
