@@ -617,81 +617,90 @@ __global__ void __launch_bounds__(256) blk_gemm_kernel(BlockedState<S> st, GemmR
 // from HBM at a depth of 64. The whole factorisation at n = 720 (5642 problems) takes 199 ms with chunks of 8
 // (three workgroups per CU), 262 ms with chunks of 16 (two), and took 240 ms with 4x4-per-thread
 // vector-FMA tiles; at n = 120 (68442 problems) 34.4 against 38.3 ms.
-template <int MI, bool FUSED = false>
-__global__ void __launch_bounds__(256, MI == 2 ? 3 : 2) blk_gemm_f64_kernel(BlockedState<double2> st, GemmRange g, int nprob) {
+// LIST: of a subset whose size only the device knows; the grid covers `stride` problems and loops over the
+// rest (a grid for every problem of an empty subset of 5642 at n = 720 took 2.2 ms in workgroups that return
+// at once). Elsewhere, and in the one fused launch of a subset, stride is nprob and there is no loop, which
+// costs registers.
+constexpr int BLK_LIST_STRIDE = 64;
+template <int MI, bool FUSED = false, bool LIST = false>
+__global__ void __launch_bounds__(256, MI == 2 ? 3 : 2) blk_gemm_f64_kernel(BlockedState<double2> st, GemmRange g, int nprob,
+                                                                              int stride) {
   constexpr int TM = 32 * MI, KC = 8;
-  int b, t;
-  if (!xcd_tile(blockIdx.x, nprob, g.tiles_r * g.tiles_c, b, t)) return;
-  if (ladder_idle(st.src, st.item0 + b)) return;
-  const int tr = t / g.tiles_c, tcl = t - (t / g.tiles_c) * g.tiles_c;
-  const int ld = st.ld;
-  double2* W = st.W + static_cast<size_t>(b) * st.n * ld;
-  const int rt = g.r0 + tr * TM, ct = g.c0 + tcl * 64;
   __shared__ double2 s_a[TM][KC + 1];
   __shared__ double2 s_b[KC][65];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = 16 * MI * (wave >> 1), wn = 32 * (wave & 1);
-  constexpr int LA = TM / 32;
-  const int ar = tid / KC, ak = tid % KC, bk = tid / 64, bc = tid % 64;
-  const double2* A[LA];
+  int b, t;
+  if (!xcd_tile(blockIdx.x, stride, g.tiles_r * g.tiles_c, b, t)) return;
+  for (; b < nprob; b += stride) {
+    if (ladder_idle(st.src, st.item0 + b)) return;
+    const int tr = t / g.tiles_c, tcl = t - (t / g.tiles_c) * g.tiles_c;
+    const int ld = st.ld;
+    double2* W = st.W + static_cast<size_t>(b) * st.n * ld;
+    const int rt = g.r0 + tr * TM, ct = g.c0 + tcl * 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = 16 * MI * (wave >> 1), wn = 32 * (wave & 1);
+    constexpr int LA = TM / 32;
+    const int ar = tid / KC, ak = tid % KC, bk = tid / 64, bc = tid % 64;
+    const double2* A[LA];
 #pragma unroll
-  for (int u = 0; u < LA; ++u) A[u] = W + static_cast<size_t>(min(rt + ar + 32 * u, g.r1 - 1)) * ld + g.k0 + ak;
-  const double2* B = W + static_cast<size_t>(g.k0 + bk) * ld + min(ct + bc, g.c1 - 1);
-  double2 ra[LA], rb[2];
-  auto load = [&](int kc) {
-    if (kc + KC <= g.kw) {
+    for (int u = 0; u < LA; ++u) A[u] = W + static_cast<size_t>(min(rt + ar + 32 * u, g.r1 - 1)) * ld + g.k0 + ak;
+    const double2* B = W + static_cast<size_t>(g.k0 + bk) * ld + min(ct + bc, g.c1 - 1);
+    double2 ra[LA], rb[2];
+    auto load = [&](int kc) {
+      if (kc + KC <= g.kw) {
 #pragma unroll
-      for (int u = 0; u < LA; ++u) ra[u] = A[u][kc];
+        for (int u = 0; u < LA; ++u) ra[u] = A[u][kc];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) rb[u] = B[static_cast<size_t>(kc + 4 * u) * ld];
-    } else {
+        for (int u = 0; u < 2; ++u) rb[u] = B[static_cast<size_t>(kc + 4 * u) * ld];
+      } else {
 #pragma unroll
-      for (int u = 0; u < LA; ++u) ra[u] = kc + ak < g.kw ? A[u][kc] : make_double2(0.0, 0.0);
+        for (int u = 0; u < LA; ++u) ra[u] = kc + ak < g.kw ? A[u][kc] : make_double2(0.0, 0.0);
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-        rb[u] = kc + bk + 4 * u < g.kw ? B[static_cast<size_t>(kc + 4 * u) * ld] : make_double2(0.0, 0.0);
+        for (int u = 0; u < 2; ++u)
+          rb[u] = kc + bk + 4 * u < g.kw ? B[static_cast<size_t>(kc + 4 * u) * ld] : make_double2(0.0, 0.0);
+      }
+    };
+    load(0);
+    ZmmaAcc<MI, 2> acc;
+    LadderSrc src{};
+    if constexpr (FUSED) src = ladder_src(st.src, st.item0 + b);
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const int r = min(rt + wm + 16 * i + zmma_row(lane, r4), g.r1 - 1);
+          const int c = min(ct + wn + 16 * j + (lane & 15), g.c1 - 1);
+          double2 x;
+          if constexpr (FUSED)
+            x = gemm_c_at<double2>(st, W, g, b, r, c, src, nullptr);
+          else
+            x = W[static_cast<size_t>(r) * ld + c];
+          acc.re[i][j][r4] = x.x;
+          acc.im[i][j][r4] = x.y;
+        }
+    for (int kc = 0; kc < g.kw; kc += KC) {
+#pragma unroll
+      for (int u = 0; u < LA; ++u) s_a[ar + 32 * u][ak] = make_double2(-ra[u].x, -ra[u].y);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) s_b[bk + 4 * u][bc] = rb[u];
+      __syncthreads();
+      if (kc + KC < g.kw) load(kc + KC);
+      zmma_chunk<MI, 2, TM, 64, KC>(acc, s_a, s_b, wm, wn, lane);
+      __syncthreads();
     }
-  };
-  load(0);
-  ZmmaAcc<MI, 2> acc;
-  LadderSrc src{};
-  if constexpr (FUSED) src = ladder_src(st.src, st.item0 + b);
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const int r = min(rt + wm + 16 * i + zmma_row(lane, r4), g.r1 - 1);
-        const int c = min(ct + wn + 16 * j + (lane & 15), g.c1 - 1);
-        double2 x;
-        if constexpr (FUSED)
-          x = gemm_c_at<double2>(st, W, g, b, r, c, src, nullptr);
-        else
-          x = W[static_cast<size_t>(r) * ld + c];
-        acc.re[i][j][r4] = x.x;
-        acc.im[i][j][r4] = x.y;
-      }
-  for (int kc = 0; kc < g.kw; kc += KC) {
-#pragma unroll
-    for (int u = 0; u < LA; ++u) s_a[ar + 32 * u][ak] = make_double2(-ra[u].x, -ra[u].y);
-#pragma unroll
-    for (int u = 0; u < 2; ++u) s_b[bk + 4 * u][bc] = rb[u];
-    __syncthreads();
-    if (kc + KC < g.kw) load(kc + KC);
-    zmma_chunk<MI, 2, TM, 64, KC>(acc, s_a, s_b, wm, wn, lane);
-    __syncthreads();
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const int r = rt + wm + 16 * i + zmma_row(lane, r4), c = ct + wn + 16 * j + (lane & 15);
+          if (r < g.r1 && c < g.c1)
+            W[static_cast<size_t>(r) * ld + c] = make_double2(acc.re[i][j][r4], acc.im[i][j][r4]);
+        }
+    if constexpr (!LIST) break;
   }
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const int r = rt + wm + 16 * i + zmma_row(lane, r4), c = ct + wn + 16 * j + (lane & 15);
-        if (r < g.r1 && c < g.c1)
-          W[static_cast<size_t>(r) * ld + c] = make_double2(acc.re[i][j][r4], acc.im[i][j][r4]);
-      }
 }
 
 // Same update on the FP32 matrix cores: each wavefront owns a 32x32 quarter of the tile as
@@ -1075,9 +1084,11 @@ struct BlockedSteps {
     // tiles are 8% faster over the whole factorisation (more workgroups per CU), and at n = 120
     // a 128-row tile over the short updates is mostly empty.
     constexpr bool c128 = std::is_same<S, double2>::value;
-    const bool tall = c128 && mode == BLK_GEMM_VECTOR && r1 - r0 > 96 && st.tall_tiles;
+    const bool list = c128 && st.src.nitems && !fused;
+    const bool tall = c128 && mode == BLK_GEMM_VECTOR && r1 - r0 > 96 && st.tall_tiles && !list;
     const GemmRange g = gemm_range(r0, r1, c0, c1, k0, kw, tall ? 128 : 64, fused);
-    const size_t grid = xcd_grid(nb, static_cast<size_t>(g.tiles_r) * g.tiles_c);
+    const int stride = list ? std::min(nb, BLK_LIST_STRIDE) : nb;
+    const size_t grid = xcd_grid(stride, static_cast<size_t>(g.tiles_r) * g.tiles_c);
     DGAMI_ARG_CHECK(grid < (size_t(1) << 31), "ladder: trailing update grid too large");
     hipEvent_t start = nullptr;
     const bool prof = profile_on();
@@ -1085,16 +1096,18 @@ struct BlockedSteps {
     const dim3 gd(static_cast<unsigned>(grid));
     if (mode == BLK_GEMM_VECTOR) {
       if constexpr (c128) {
-        if (tall) {
+        if (list) {
+          hipLaunchKernelGGL((blk_gemm_f64_kernel<2, false, true>), gd, dim3(256), 0, stream, st, g, nb, stride);
+        } else if (tall) {
           if (fused)
-            hipLaunchKernelGGL((blk_gemm_f64_kernel<4, true>), gd, dim3(256), 0, stream, st, g, nb);
+            hipLaunchKernelGGL((blk_gemm_f64_kernel<4, true>), gd, dim3(256), 0, stream, st, g, nb, stride);
           else
-            hipLaunchKernelGGL((blk_gemm_f64_kernel<4>), gd, dim3(256), 0, stream, st, g, nb);
+            hipLaunchKernelGGL((blk_gemm_f64_kernel<4>), gd, dim3(256), 0, stream, st, g, nb, stride);
         } else {
           if (fused)
-            hipLaunchKernelGGL((blk_gemm_f64_kernel<2, true>), gd, dim3(256), 0, stream, st, g, nb);
+            hipLaunchKernelGGL((blk_gemm_f64_kernel<2, true>), gd, dim3(256), 0, stream, st, g, nb, stride);
           else
-            hipLaunchKernelGGL((blk_gemm_f64_kernel<2>), gd, dim3(256), 0, stream, st, g, nb);
+            hipLaunchKernelGGL((blk_gemm_f64_kernel<2>), gd, dim3(256), 0, stream, st, g, nb, stride);
         }
       } else {
         if (fused)
@@ -1258,7 +1271,8 @@ int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream) {
   DGAMI_ARG_CHECK(n <= BLK_MAX_N, "ladder: compound size above 1536 is not supported");
   const size_t items = static_cast<size_t>(a.nchan) * a.nw * a.nq;
   const size_t per = static_cast<size_t>(n) * ld * sizeof(double2);
-  const int nl = static_cast<int>(std::min<size_t>(ladder_lanes(), items));
+  // (a subset, empty as a rule, in half as many launches)
+  const int nl = a.nitems ? 1 : static_cast<int>(std::min<size_t>(ladder_lanes(), items));
   // MI355X holds 288 GB of HBM: factor up to 48 GiB of problems per pass (over all lanes)
   size_t batch = (size_t(48) << 30) / (per * nl);
   if (batch < 1) batch = 1;
