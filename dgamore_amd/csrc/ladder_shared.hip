@@ -47,6 +47,7 @@ struct SharedArgs : SharedGroups {
   int ntile;              // tiles of SH_TN columns
   size_t cols;            // columns of the batch
   const S* ps;            // P and D(q) in S (the originals where S is double2)
+  const __bf16* pb;       // P split for the BF16 matrix cores (cgemm.hpp) in place of ps, or null
   const S* ds;
   S* V;                   // [SH_M + 1][groups][n][N] Krylov basis
   S* u;                   // operand of the products [groups][n][N]
@@ -569,10 +570,24 @@ static int shared_product(const SharedGroups& s, const double2* A, const double2
   return three ? launch_zgemm<true>(g, s.groups, stream) : launch_zgemm<false>(g, s.groups, stream);
 }
 
-static int shared_product(const SharedGroups& s, const float2* A, const float2* B, float2* C, const int* tiles, bool,
-                          hipStream_t stream) {
+// g = P u.
+static int shared_precondition(const SharedArgs<double2>& s, const int* tiles, hipStream_t stream) {
+  return shared_product(s, s.ps, s.u, s.g, tiles, true, stream);
+}
+
+static int shared_precondition(const SharedArgs<float2>& s, const int* tiles, hipStream_t stream) {
   static_assert(CG_TN == SH_TN, "the tiles whose activity is tracked");
-  return launch_cgemm(shared_operands<CgemmArgs>(s, A, B, C, tiles), s.groups, stream);
+  if (!s.pb) return launch_cgemm(shared_operands<CgemmArgs>(s, s.ps, s.u, s.g, tiles), s.groups, stream);
+  CgemmBf16Args g;
+  g.A = s.pb;
+  g.B = s.u;
+  g.C = s.g;
+  g.M = g.K = s.a.n;
+  g.lda = cgemm_split_lda(s.a.n);
+  g.N = g.ldb = g.ldc = s.N;
+  g.sb = g.sc = static_cast<long long>(s.a.n) * s.N;
+  g.tile_active = tiles;
+  return launch_cgemm_bf16x3(g, s.groups, stream);
 }
 
 template <int T, typename S>
@@ -587,7 +602,7 @@ static int shared_solve(SharedArgs<S>& s, hipStream_t stream) {
     if (cycle > 0) {
       DGAMI_STEP(shared_product(s, s.A0, s.X, s.ax, s.tile_run, false, stream));
       DGAMI_STEP((shared_apply<T, true>(s, s.X, s.tile_run, stream)));
-      DGAMI_STEP(shared_product(s, s.ps, s.u, s.g, s.tile_run, true, stream));
+      DGAMI_STEP(shared_precondition(s, s.tile_run, stream));
     }
     if (diag)
       hipLaunchKernelGGL((shared_start_kernel<S, true>), gd, bd, 0, stream, s, cycle == 0 ? 1 : 0);
@@ -596,7 +611,7 @@ static int shared_solve(SharedArgs<S>& s, hipStream_t stream) {
     DGAMI_HIP_CHECK(hipGetLastError());
     for (int k = 0; k < SH_M; ++k) {
       if (!diag) DGAMI_STEP((shared_apply<T, false>(s, s.V + k * vec, s.tile_live, stream)));
-      DGAMI_STEP(shared_product(s, s.ps, s.u, s.g, s.tile_live, true, stream));
+      DGAMI_STEP(shared_precondition(s, s.tile_live, stream));
       DGAMI_STEP(diag ? shared_step<true>(s, k, stream) : shared_step<false>(s, k, stream));
     }
     hipLaunchKernelGGL((shared_update_kernel<S>), gd, bd, 0, stream, s, cycle, cycle == SH_CYCLES - 1 ? 1 : 0);
@@ -621,22 +636,24 @@ bool ladder_shared_applies(const LadderArgs& a, int precision) {
 
 // A batch by one launch per product and per pass over the basis: vec and st hold the vectors and the
 // columns' data of ng groups. With a complex64 basis (c64) A0 X has its own vector, and P and D(q) are
-// there in complex64 too (in `narrow`, shared_narrow values).
+// there in complex64 too (in `narrow`: P or its split form, then D(q)).
 static size_t large_vectors(const LadderArgs& a, size_t groups, int N, bool c64) {
   const size_t vec = static_cast<size_t>(a.n) * groups * N, sums = a.v_r ? static_cast<size_t>(a.T) * groups * N : 0;
   return c64 ? vec * ((SH_M + 3) * sizeof(float2) + 2 * sizeof(double2)) + sums * sizeof(double2)
              : (vec * (SH_M + 4) + sums) * sizeof(double2);
 }
-static size_t shared_narrow_size(const LadderArgs& a, size_t groups) {
-  return groups * a.n * a.n + static_cast<size_t>(a.nw) * a.T * a.T * a.nv * a.nq;
+static size_t shared_narrow_p(const LadderArgs& a, size_t groups) {
+  return groups * a.n * cgemm_split_lda(a.n);
 }
+
 static size_t large_state(size_t groups, int N) {
   const size_t per_col = sizeof(double2) * (SH_M + SH_ROT + SH_M + 1) + sizeof(double) * (SH_M + 3) + 2 * sizeof(int);
   return groups * (N * per_col + 2 * ceil_div(N, SH_TN) * sizeof(int));
 }
 
 template <typename S>
-static int shared_large_solve(const SharedGroups& sg, char* vec, void* st, float2* narrow, hipStream_t stream) {
+static int shared_large_solve(const SharedGroups& sg, char* vec, void* st, float2* narrow, const float2* ds, bool bf16,
+                              hipStream_t stream) {
   SharedArgs<S> s{};
   static_cast<SharedGroups&>(s) = sg;
   const size_t cols = static_cast<size_t>(s.groups) * s.N, used = cols * s.a.n;
@@ -649,11 +666,18 @@ static int shared_large_solve(const SharedGroups& sg, char* vec, void* st, float
     s.ax = end;
     end += used;
     const size_t nn = static_cast<size_t>(s.groups) * s.a.n * s.a.n;
-    s.ds = narrow;
-    float2* p = narrow + static_cast<size_t>(s.a.nw) * s.a.T * s.a.T * s.a.nv * s.a.nq;
-    hipLaunchKernelGGL(shared_narrow_kernel, dim3(ceil_div(nn, 256)), dim3(256), 0, stream, s.P, p, nn);
+    s.ds = ds;
+    if (bf16) {
+      const int ldp = cgemm_split_lda(s.a.n);
+      __bf16* p = reinterpret_cast<__bf16*>(narrow);
+      hipLaunchKernelGGL(cgemm_split_kernel, dim3(ceil_div(static_cast<size_t>(s.a.n) * ldp, 256), s.groups), dim3(256), 0,
+                         stream, s.P, p, s.a.n, ldp);
+      s.pb = p;
+    } else {
+      hipLaunchKernelGGL(shared_narrow_kernel, dim3(ceil_div(nn, 256)), dim3(256), 0, stream, s.P, narrow, nn);
+      s.ps = narrow;
+    }
     DGAMI_HIP_CHECK(hipGetLastError());
-    s.ps = p;
   } else {
     s.ds = s.dd;
     s.ps = s.P;
@@ -695,7 +719,7 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
   const size_t pk = tiles ? shared_packed(n) : 0;
   // groups per batch: matrices and, for large sizes, vectors of at most 24 GiB
   const size_t per_group = (2 * (nn + pk) + shared_inverse_workspace(n)) * sizeof(double2) + (tiles ? 0 : large_vectors(a, 1, N, c64)) +
-                           (c64 ? nn * sizeof(float2) : 0);
+                           (c64 ? shared_narrow_p(a, 1) * sizeof(float2) : 0);
   const size_t gb = std::max<size_t>(1, std::min<size_t>({(size_t(24) << 30) / per_group, G, 65535}));
   SharedGroups s{};
   s.a = a;
@@ -705,7 +729,7 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
   const size_t rows = static_cast<size_t>(a.nw) * TT * a.nv;
   const size_t vsz = a.v_r ? static_cast<size_t>(a.nchan) * TT : 0, dvsz = vsz * nq;
   const size_t szc = rows + rows * nq + vsz + dvsz + gb * ((nn + pk) * 2 + n * T + shared_inverse_workspace(n));
-  const size_t nsz = c64 ? shared_narrow_size(a, gb) : 0;
+  const size_t nsz = c64 ? shared_narrow_p(a, gb) + rows * nq : 0;
   double2* mean = static_cast<double2*>(workspace(WS_SHARED + slot_offset, szc * sizeof(double2) + nsz * sizeof(float2)));
   char* vec = static_cast<char*>(workspace(
       WS_SHARED_VEC + slot_offset, tiles ? shared_tile_workspace(s) * sizeof(double2) : large_vectors(a, gb, N, c64)));
@@ -720,7 +744,8 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
   double2* pack = P + gb * nn;
   double2* z0 = pack + 2 * gb * pk;
   double2* inv = z0 + gb * n * T;
-  float2* narrow = reinterpret_cast<float2*>(inv + gb * shared_inverse_workspace(n));  // D(q), P in complex64
+  float2* narrow = reinterpret_cast<float2*>(inv + gb * shared_inverse_workspace(n));  // P, D(q) in complex64
+  float2* ds = narrow + shared_narrow_p(a, gb);
   s.dd = dd;
   s.dv = a.v_r ? dv : nullptr;
   s.A0 = A0;
@@ -739,7 +764,7 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
     DGAMI_HIP_CHECK(hipGetLastError());
   }
   if (c64) {
-    hipLaunchKernelGGL(shared_narrow_kernel, dim3(ceil_div(rows * nq, 256)), dim3(256), 0, stream, dd, narrow, rows * nq);
+    hipLaunchKernelGGL(shared_narrow_kernel, dim3(ceil_div(rows * nq, 256)), dim3(256), 0, stream, dd, ds, rows * nq);
     DGAMI_HIP_CHECK(hipGetLastError());
   }
   for (size_t g0 = 0; g0 < G; g0 += gb) {
@@ -755,8 +780,8 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
       hipLaunchKernelGGL(shared_rhs_kernel, dim3(ceil_div(static_cast<size_t>(ng) * n, 4)), dim3(256), 0, stream, P, z0,
                          ng * n, n, T, a.nv);
       DGAMI_HIP_CHECK(hipGetLastError());
-      rc = c64 ? shared_large_solve<float2>(s, vec, st, narrow, stream)
-               : shared_large_solve<double2>(s, vec, st, nullptr, stream);
+      rc = c64 ? shared_large_solve<float2>(s, vec, st, narrow, ds, precision == DGAMI_MIXED_BF16X3_IR, stream)
+               : shared_large_solve<double2>(s, vec, st, nullptr, nullptr, false, stream);
     }
     if (rc) return rc;
     hipLaunchKernelGGL(shared_collect_kernel, dim3(ceil_div(static_cast<size_t>(ng) * nq, 256)), dim3(256), 0, stream, s, list,

@@ -39,7 +39,8 @@ constexpr double SH_DONE_TOL = 2e-16;
 // to SH_TRUST, so P is the inverse of A0 to SH_TRUST and this cycle's error is at most that part of its start.
 constexpr double SH_TRUST = 1e-7;
 // The same with the basis, P and D(q) in complex64 (the mixed forms above SHARED_TILE_N; X, A0 and the residuals
-// stay in FP64): a cycle can gain five digits, and |X| is wanted to SH_DONE_TOL_C64, four digits beyond what the
+// stay in FP64; the split-BF16 form multiplies P in split BF16, with the same number of cycles in every case
+// measured): a cycle can gain five digits, and |X| is wanted to SH_DONE_TOL_C64, four digits beyond what the
 // refinement of the mixed LU asks for.
 constexpr double SH_CYCLE_TOL_C64 = 1e-5, SH_DONE_TOL_C64 = 1e-14, SH_TRUST_C64 = 1e-9;
 // A cycle that leaves more than this of its residual is stagnating.
