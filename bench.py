@@ -10,12 +10,14 @@ in HBM. The default workload is the 3-orbital t2g model on a 24x24 k-grid
 local inputs averaged over the lattice's orbital symmetry and its kernel mapped
 to the full zone with the per-k orbital transforms.
 The JSON line reports (q, w) ladder solves per second of the whole step in
-the headline form (bf16x3: complex64 LU whose trailing updates run as three
-split-BF16 matrix-core products, refined in FP64; mixed: the same with FP32
-matrix-core updates; plain: complex128), the step wall time, the same for the
+the headline form (bf16x3: an iteration with the inverse of the matrix that the
+q-points of a (channel, w) share, in complex64 with split-BF16 matrix-core products,
+on FP64 residuals; mixed: the same with FP32 matrix-core products; plain:
+complex128 throughout; where that form does not pay, a blocked LU of every problem in
+the same precisions with FP64 refinement), the step wall time, the same for the
 plain complex128 form with the relative errors of chi*, chi and Sigma between
-the two, the roofline of the dominant kernel (the trailing-matrix update of
-the blocked LU) timed with HIP events on its launch stream, and a CPU
+the two, the roofline of the dominant kernel (the product with the shared inverse,
+or the LU's trailing-matrix update) timed with HIP events on its launch stream, and a CPU
 baseline: the NumPy restatement of the reference's per-q solve path timed on
 the host on a bounded sample of the same workload.
 """
@@ -37,6 +39,7 @@ PEAK_HBM_GBS = 8000.0
 # HBM bytes per trailing-update launch measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE
 # (scaled by the copy-kernel factors), one "precision workload GB_per_launch" line each
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "trailing_update_traffic.txt")
+SHARED_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "shared_product_traffic.txt")  # the same of a full product
 # the headline metric, as the benchmark definition names it
 METRIC = "(q,\u03c9) ladder solves/s + \u03a3 wall time: mixed vs FP64 on GPU at \u22641e-8 rel err"
 
@@ -48,8 +51,8 @@ def parse():
     ap.add_argument("--warmup", type=int, default=1)
     ap.add_argument("--config", type=int, default=2)
     ap.add_argument("--precision", default="bf16x3", choices=["plain", "mixed", "bf16x3"],
-                    help="form whose throughput is the headline value (mixed: complex64 LU on the FP32 matrix "
-                         "cores + FP64 refinement; bf16x3: the same with split-BF16 MFMA trailing updates)")
+                    help="form whose throughput is the headline value (mixed: complex64 on the FP32 matrix "
+                         "cores + FP64 residuals; bf16x3: the same with split-BF16 MFMA products)")
     ap.add_argument("--no-compare", action="store_true", help="skip the plain FP64 comparison run")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-seconds", type=float, default=10.0, help="target CPU-baseline sample time")
@@ -529,14 +532,13 @@ def time_sigma(pipe, nrep, stream):
 def dominant_kernel(pipe, stream, ms_ladder, precision_name):
     """Roofline of the dominant kernel of the ladder solve, timed with HIP events on its stream.
 
-    Compound sizes above 128 run the blocked LU, whose trailing-matrix update dominates: the
-    library brackets each of its launches with events (dgami_profile_*) and returns the
-    algorithmic flops (8 m n k per problem) and the bytes of the C tile read and written plus the
-    A and B panels read once. The ladder is matrix-core work (8/3 n^3 + 8 nb^2 n^2 flops per
-    solve against kilobytes of operands), so the bound is the matrix-core peak of the precision
-    (split-BF16: the BF16 peak / 3 products). `traffic` is the HBM bytes per launch measured with
+    Above n = 256 the library brackets with events (dgami_profile_*) the first product of a call
+    with the shared inverse matrices, of all columns (8 n^2 flops per column), or, where the blocked
+    LU runs, each trailing-matrix update (8 m n k per problem), and returns these flops and the bytes
+    of the operands and the result. Both are matrix-core work, so the bound is the matrix-core peak
+    of the precision (split-BF16: the BF16 peak / 3 products). `traffic` is the HBM bytes per launch measured with
     rocprofv3 FETCH_SIZE / WRITE_SIZE (profiles/trailing_update_traffic.txt).
-    Smaller sizes run one register-resident kernel per call, timed as the whole ladder call.
+    Smaller sizes run one kernel for the solve, timed as the whole ladder call in LU flops.
     """
     import torch
 
@@ -579,17 +581,21 @@ def dominant_kernel(pipe, stream, ms_ladder, precision_name):
     avg_ms = prof["ms"] / prof["launches"]
     tf = prof["flops"] / (prof["ms"] * 1e-3) / 1e12
     gbs = prof["bytes"] / (prof["ms"] * 1e-3) / 1e9
+    n = m.nb**2 * 2 * m.niv
+    shared = prof["launches"] and prof["flops"] == 8.0 * n * n * m.nb**2 * pipe.solves_per_step()
     traffic = None
-    if os.path.exists(TRAFFIC_FILE):
-        for line in open(TRAFFIC_FILE):
+    traffic_file = SHARED_TRAFFIC_FILE if shared else TRAFFIC_FILE
+    if os.path.exists(traffic_file):
+        for line in open(traffic_file):
             f = line.split("#", 1)[0].split()
             if len(f) == 3 and f[0] == precision_name and f[1] == m.name:
                 traffic = float(f[2]) * 1e9
-    return {"kernel": "trailing-matrix update of the blocked LU (blk_gemm_*)", "launches": prof["launches"],
+    return {"kernel": "product with the shared inverse matrices (cgemm_*, zgemm)" if shared
+            else "trailing-matrix update of the blocked LU (blk_gemm_*)", "launches": prof["launches"],
             "avg_launch_ms": avg_ms, "bound": "mfma", "achieved": tf, "peak": peak_tf, "unit": "TFLOP/s",
             "frac": tf / peak_tf, "traffic": traffic,
             "algorithmic_flops_per_launch": prof["flops"] / prof["launches"],
-            "c_tile_and_panel_bytes_per_launch": prof["bytes"] / prof["launches"],
+            "operand_and_result_bytes_per_launch": prof["bytes"] / prof["launches"],
             "hbm_GBps_of_measured_traffic": None if traffic is None else traffic / (avg_ms * 1e-3) / 1e9,
             "hbm_frac_of_measured_traffic": None if traffic is None else traffic / (avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
             "measured_with": "the ladder on one stream (DGAMI_LADDER_STREAMS=1); the timed steps use two",
@@ -707,7 +713,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": {0: "c128", 1: "c64-LU+c128-refinement", 2: "bf16x3-LU+c128-refinement"}[prec],
+        "dtype": {0: "c128", 1: "c64+c128-refinement", 2: "bf16x3+c128-refinement"}[prec],
         "data": "synthetic (seeded DMFT-like model, random-perturbation local vertex"
                 + (")" if args.no_symmetric or model.orbital_transforms is None
                    else ", orbital-symmetric, full-zone map with per-k orbital transforms)"),
@@ -721,8 +727,9 @@ def main():
         "ladder_ms": ms_ladder,
         "ladder_solves_per_s": solves / (ms_ladder * 1e-3),
         "ladder_roofline": {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
-                            "frac": achieved / peak, "flops_per_solve": pipe.ladder_flops_per_solve()},
-        "ladder_traffic": None if roof.get("traffic") is None else {
+                            "frac": achieved / peak, "flops_per_solve": pipe.ladder_flops_per_solve(),
+                            "flops_counted": "those of one LU per problem (the shared-matrix form needs fewer)"},
+        "ladder_traffic": None if roof.get("traffic") is None or "shared" in roof["kernel"] else {
             "trailing_update_GB_per_call": roof["traffic"] * roof["launches"] / 1e9,
             "algorithmic_GB_per_call": ladder_algorithmic_bytes(pipe) / 1e9,
             "ratio": roof["traffic"] * roof["launches"] / ladder_algorithmic_bytes(pipe)},

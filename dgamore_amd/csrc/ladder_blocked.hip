@@ -1091,7 +1091,7 @@ struct BlockedSteps {
     const size_t grid = xcd_grid(stride, static_cast<size_t>(g.tiles_r) * g.tiles_c);
     DGAMI_ARG_CHECK(grid < (size_t(1) << 31), "ladder: trailing update grid too large");
     hipEvent_t start = nullptr;
-    const bool prof = profile_on();
+    const bool prof = profile_on() && !st.src.nitems;
     if (prof && profile_begin(stream, &start)) return -2;
     const dim3 gd(static_cast<unsigned>(grid));
     if (mode == BLK_GEMM_VECTOR) {

@@ -611,7 +611,15 @@ static int shared_solve(SharedArgs<S>& s, hipStream_t stream) {
     DGAMI_HIP_CHECK(hipGetLastError());
     for (int k = 0; k < SH_M; ++k) {
       if (!diag) DGAMI_STEP((shared_apply<T, false>(s, s.V + k * vec, s.tile_live, stream)));
+      // the first product of a batch, of all columns, is what dgami_profile_* times here
+      hipEvent_t start = nullptr;
+      const bool prof = cycle == 0 && k == 0 && profile_on();
+      if (prof && profile_begin(stream, &start)) return -2;
       DGAMI_STEP(shared_precondition(s, s.tile_live, stream));
+      if (prof) {
+        const double nn = static_cast<double>(s.a.n) * s.a.n * s.groups;
+        if (profile_end(stream, start, (nn + 2.0 * vec) * sizeof(S), 8.0 * nn * s.N)) return -2;
+      }
       DGAMI_STEP(diag ? shared_step<true>(s, k, stream) : shared_step<false>(s, k, stream));
     }
     hipLaunchKernelGGL((shared_update_kernel<S>), gd, bd, 0, stream, s, cycle, cycle == SH_CYCLES - 1 ? 1 : 0);
@@ -631,7 +639,8 @@ bool ladder_shared_applies(const LadderArgs& a, int precision) {
   const double ratio = a.n / (3.0 * a.T) + 1.0, work = static_cast<double>(a.nchan) * a.nw * a.nq * ratio;
   if (a.n <= 32) return work >= SHARED_MIN_WORK_N32 && a.T <= 4;
   if (a.n <= SHARED_TILE_N && a.T <= 4) return work >= (a.T == 1 ? SHARED_MIN_WORK_1 : SHARED_MIN_WORK_4);
-  return ratio >= SHARED_MIN_RATIO && work >= (precision == DGAMI_PLAIN_FP64 ? SHARED_MIN_WORK : SHARED_MIN_WORK_MIXED);
+  return precision == DGAMI_PLAIN_FP64 ? ratio >= SHARED_MIN_RATIO && work >= SHARED_MIN_WORK
+                                       : ratio >= SHARED_MIN_RATIO_MIXED && work >= SHARED_MIN_WORK_MIXED;
 }
 
 // A batch by one launch per product and per pass over the basis: vec and st hold the vectors and the

@@ -12,19 +12,21 @@ namespace dgami {
 // product: problems x ratio >= a bound, with ratio = n / (3 T) + 1. With one or two orbitals up to n = 256 the
 // bound is SHARED_MIN_WORK_1 (T = 1) or SHARED_MIN_WORK_4, and SHARED_MIN_WORK_N32 up to n = 32, where the LU is
 // one small register tile; beyond, the ratio itself has to reach SHARED_MIN_RATIO
-// (the passes over the basis and the D(q) blocks grow with T) and the bound is SHARED_MIN_WORK, or
-// SHARED_MIN_WORK_MIXED for the mixed forms, whose LU is the faster one too. Measured, LU / this form in us
+// (the passes over the basis and the D(q) blocks grow with T) and the bound is SHARED_MIN_WORK, with
+// other bounds for the mixed forms (SHARED_MIN_RATIO_MIXED, SHARED_MIN_WORK_MIXED). Measured, LU / this form in us
 // (beta = 10 ... 40, U = 3 ... 8). T = 1 below: n = 30, 1440 problems 168 / 230; n = 40, 990 problems 161 / 185; n = 96, 392 problems 444 / 563;
 // above: n = 40, 1350 problems 230 / 187; n = 64, 990 problems 384 / 229; n = 120, 450 problems 608 / 472, 68442 problems
 // 38100 / 3530. T = 4 below: n = 32,
 // 1440 problems 203 / 293; n = 48, 1440 problems 323 / 336; above: n = 64, 1440 problems 550 / 379; n = 80, 1170 problems 607 / 456; n = 120, 1440 problems 1072 / 764; n = 216, 540 problems
 // 1588 / 1300. Large, complex128, below: T = 9, n = 252, 560 problems 2207 / 2652; n = 360, 840 problems 5810 / 7940; n = 720,
-// 448 problems 16025 / 15066; above: T = 4, n = 400, 540 problems 5488 / 5309; T = 9, n = 540, 1170 problems
-// 20020 / 15003. Split-BF16 below: T = 9, n = 720, 448 problems 9858 / 10093; above: 840 problems 17125 / 14148,
-// 5642 problems 93079 / 55800; T = 4, n = 320, 840 problems 3658 / 3087.
+// 448 problems 16025 / 15066 (not far above); above: T = 4, n = 400, 540 problems 5488 / 5309; T = 9, n = 540, 1170 problems
+// 20020 / 15003. Split-BF16 below: T = 9, n = 252, ratio 10; above: n = 360, 840 problems 4617 / 4407, 2790
+// problems 12119 / 8767; n = 720, 448 problems 9814 / 8481, 5642 problems 93282 / 39980; T = 4, n = 320, 448
+// problems 2795 / 2221. Complex64: n = 720, 448 problems 14209 / 9866.
 constexpr int SHARED_MIN_NQ = 16;
 constexpr double SHARED_MIN_WORK_1 = 17000.0, SHARED_MIN_WORK_4 = 9000.0, SHARED_MIN_WORK_N32 = 30000.0;
-constexpr double SHARED_MIN_WORK = 16000.0, SHARED_MIN_WORK_MIXED = 20000.0, SHARED_MIN_RATIO = 18.0;
+constexpr double SHARED_MIN_WORK = 16000.0, SHARED_MIN_WORK_MIXED = 11000.0;
+constexpr double SHARED_MIN_RATIO = 18.0, SHARED_MIN_RATIO_MIXED = 14.0;
 constexpr int SHARED_TILE_N = 256;
 
 constexpr int SH_M = 10;           // Krylov vectors of a cycle

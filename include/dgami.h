@@ -83,12 +83,12 @@ int dgami_version(void);
 int dgami_workspace_hold(void);
 int dgami_workspace_release(void);
 
-/* Kernel timing of the trailing-matrix updates of the blocked ladder LU (the dominant
- * kernel for compound sizes above 128). No counterpart in the reference: it is the
- * measurement facility behind the roofline figures. While enabled, every trailing-update
- * launch is bracketed by HIP events on its launch stream and its algorithmic work is
- * accumulated: bytes = C tile read + written + the A and B panels read once, flops =
- * 8 m n k. dgami_profile_enable(1) resets the counters; dgami_profile_read waits for the
+/* Kernel timing of the ladder's dominant kernel for compound sizes above 256. No counterpart
+ * in the reference: it is the measurement facility behind the roofline figures. While
+ * enabled, every trailing-matrix update of a blocked LU, and the first product with the
+ * inverse mean matrices of every batch of the shared-matrix form, is bracketed by HIP events
+ * on its launch stream and its algorithmic work is accumulated: bytes = C tile read + written
+ * + the A and B panels read once (the product: its operands and result once), flops = 8 m n k. dgami_profile_enable(1) resets the counters; dgami_profile_read waits for the
  * recorded events and returns the totals (time in ms). */
 int dgami_profile_enable(int on);
 int dgami_profile_read(double* ms, double* bytes, double* flops, int64_t* launches);
