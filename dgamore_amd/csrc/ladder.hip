@@ -22,7 +22,8 @@ int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream);
 int ladder_lanes();
 int ladder_reg_launch_multi(int variant, const LadderMulti& mm, hipStream_t stream);
 
-// Kernel of the plain FP64 solve. The environment variable DGAMI_LADDER_KERNEL (col, reg or
+// Kernel of the plain FP64 solve where the q-points' shared matrix does not serve it (ladder_shared.hpp has
+// that rule). The environment variable DGAMI_LADDER_KERNEL (col, reg or
 // blocked) forces one family for comparisons; otherwise an autotuned choice for (n, nrhs)
 // wins; otherwise the size rule: "reg" (2D register tiles) up to compound size 64, the
 // blocked workspace LU above it. Measured on 8192 matrices per call, the register kernel

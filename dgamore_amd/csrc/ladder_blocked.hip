@@ -1146,9 +1146,8 @@ struct BlockedSteps {
 // are updated by all earlier panels at once; after panel j its interchanges are applied to the
 // earlier panels' columns. The trailing columns then receive, panel by panel, the
 // interchanges, the row-block update and the U blocks, and the rows below the block one
-// trailing update of depth NPAN * NB. Complex128 uses two panels per block (its vector-FMA
-// trailing update is compute-bound, and the extra in-block updates of deeper blocks cost more
-// than they save); complex64 uses four, halving the trailing matrix's HBM traffic.
+// trailing update of depth NPAN * NB. Complex128 uses two panels per block (the extra in-block
+// updates of deeper blocks cost more than they save); complex64 uses four, halving the trailing matrix's HBM traffic.
 template <typename S, int NB, int RPT, int MAXTH, int NPAN>
 static int blocked_factor_nb(const LadderArgs& a, BlockedState<S>& st, int item0, int nb, hipStream_t stream) {
   static_assert(NPAN >= 1 && NPAN <= BLK_PANELS, "panels per outer block");

@@ -1,4 +1,5 @@
-// Mixed-precision ladder solves: complex64 LU factorisation, FP64 iterative refinement.
+// Mixed-precision ladder solves: complex64 LU factorisation, FP64 iterative refinement (where the q-points'
+// shared matrix, ladder_shared.hpp, does not serve them).
 //
 // Every item's matrix A is factored once in FP32 (PA = LU, batched blocked LU of
 // ladder_blocked.hip with the interchanges also applied left of each panel; trailing
@@ -385,7 +386,7 @@ __global__ void __launch_bounds__(256) mix_info_kernel(const int* __restrict__ s
 int ladder_solve_mixed(const LadderArgs& a, int precision, hipStream_t stream) {
   DGAMI_ARG_CHECK(precision == DGAMI_MIXED_FP32_IR || precision == DGAMI_MIXED_BF16X3_IR,
                   "ladder: unknown mixed-precision mode");
-  // the shared form solves in FP64 whatever the factors' form (its errors are the smaller ones)
+  // many q-points that share a matrix: on FP64 residuals too, with the smaller errors
   if (ladder_shared_applies(a, precision)) return ladder_solve_shared(a, precision, stream);
   // the split-BF16 factors carry ~2^-16 relative error per product instead of 2^-24, so
   // each refinement step gains fewer digits and more steps may be needed

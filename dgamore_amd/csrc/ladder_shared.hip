@@ -13,7 +13,9 @@
 //
 // Each cycle runs up to SH_M iterations from the residual of the current X, B - A0 X - D(q) X, formed
 // in FP64 from A0 and D(q) themselves, so the error of P only slows the convergence down; X ends as
-// an LU solution with a step of iterative refinement does. Every column has its own Hessenberg matrix and
+// an LU solution with a step of iterative refinement does. The mixed forms hold the basis, P and D(q) in
+// complex64 and multiply P on the FP32 or (split) BF16 matrix cores: 62 groups at n = 720 with 91 q-points
+// 80 ms in complex128, 40 in split BF16 (LU: 235 and 94). Every column has its own Hessenberg matrix and
 // status on the device; tiles of 64 columns (SH_TN) without an active column are skipped by the
 // products and the basis kernels, and no value is read by the host, so a call can be captured.
 // Problems with a column that does not converge (a singular or nearly singular A(q), a NaN) are

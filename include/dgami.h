@@ -53,9 +53,9 @@ typedef struct {
 
 /* Ladder precision modes (dgami_ladder_solve_sum). */
 enum {
-  DGAMI_PLAIN_FP64 = 0,    /* complex128 LU, the reference's algorithm in FP64 */
-  DGAMI_MIXED_FP32_IR = 1, /* FP32 LU + FP64 residual iterative refinement */
-  DGAMI_MIXED_BF16X3_IR = 2 /* split-BF16 (3-term) MFMA trailing updates + FP64 IR */
+  DGAMI_PLAIN_FP64 = 0,    /* complex128 throughout */
+  DGAMI_MIXED_FP32_IR = 1, /* FP32 factors or basis + FP64 residuals and solution */
+  DGAMI_MIXED_BF16X3_IR = 2 /* the same with split-BF16 (3-term) MFMA products */
 };
 
 /* Negative per-matrix codes in the `info` arrays of the mixed-precision ladder forms: the FP64
@@ -136,10 +136,12 @@ int dgami_chi0_prepare(int nq, int nb, int nw, int niv_full, int niv_core, doubl
 /* Batched ladder solves with the nu' sum, for nchan channels at once:
  *   A(c,q,w) = chi0_inv(q,w,v) delta_vv' + (gamma[c][w] - u_r[c] - v_r[c][q]) / beta^2   (CMP)
  *   chi_aux_sum[c][w][(o1,o2),(o4,o3)][v][q] = (1/beta) sum_v' [A^-1]_{(o1,o2,v),(o4,o3,v')}
- * computed as an LU solve with the nb^2 indicator right-hand sides.
+ * computed as an LU solve with the nb^2 indicator right-hand sides, or, where many q-points share
+ * the matrix of a (c, w), by an iteration with its inverse on FP64 residuals whose unconverged
+ * items take the complex128 LU (up to n = 256 in FP64 in every precision; info is the LU's).
  * chi0_inv: QF (nv = 2*niv); gamma: [nchan] x CMP; u_r: [nchan][nb^4] (M order);
  * v_r: [nchan] x QO or NULL (V = 0); chi_aux_sum: [nchan] x QF; info: [nchan][nw][nq] int32,
- * 0 or k+1 for an exactly singular pivot at elimination step k; the mixed forms also report
+ * 0 or k+1 for an exactly singular pivot at elimination step k; the mixed LU forms also report
  * DGAMI_INFO_REFINE_STALLED / DGAMI_INFO_REFINE_NONFINITE per item. Nothing is read back to the
  * host in any precision, so every form can be captured in a HIP graph.
  * precision: DGAMI_PLAIN_FP64 / DGAMI_MIXED_FP32_IR / DGAMI_MIXED_BF16X3_IR.
