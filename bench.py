@@ -311,7 +311,7 @@ def batch_graph(steps, warmup, seed, symmetric=True, precision="plain"):
         "metric": METRIC,
         "value": solves / (ms * 1e-3), "unit": "solves/s", "n_gpus": 1, "steps": steps, "warmup": warmup,
         "ms_per_step": ms, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "c128" if prec == _lib.PLAIN_FP64 else f"{precision} LU + c128 refinement (n > 64), c128 (n <= 64)",
+        "dtype": "c128" if prec == _lib.PLAIN_FP64 else f"{precision} + c128 refinement (blocked LU, or shared matrix above n = 256), c128 otherwise",
         "data": "synthetic (16 seeded DMFT-like models, random-perturbation local vertices)",
         "config": {"workload": f"batch of {len(models)} models (seed {seed}): 1-3 orbitals, beta 5-40, niv=niw="
                                f"round(1.5 beta), k-grids 16^2-32^2, compound sizes {min(sizes)}..{max(sizes)}; "
@@ -575,7 +575,7 @@ def dominant_kernel(pipe, stream, ms_ladder, precision_name):
     if prof["launches"] == 0:
         flops = pipe.solves_per_step() * pipe.ladder_flops_per_solve()
         tf = flops / (ms_ladder * 1e-3) / 1e12
-        return {"bound": "mfma", "kernel": "register-resident ladder kernel (one launch per call)",
+        return {"bound": "mfma", "kernel": "ladder kernel of one launch (register LU, or tiles of the shared-matrix form), in LU flops",
                 "achieved": tf, "peak": peak_tf, "unit": "TFLOP/s", "frac": tf / peak_tf, "traffic": None,
                 "launches": 1, "avg_launch_ms": ms_ladder}
     avg_ms = prof["ms"] / prof["launches"]

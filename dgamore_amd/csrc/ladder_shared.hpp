@@ -11,22 +11,24 @@ namespace dgami {
 // enough problems for the LU to be past its own latency, by how much more an LU computes per problem than a
 // product: problems x ratio >= a bound, with ratio = n / (3 T) + 1. With one or two orbitals up to n = 256 the
 // bound is SHARED_MIN_WORK_1 (T = 1) or SHARED_MIN_WORK_4, and SHARED_MIN_WORK_N32 up to n = 32, where the LU is
-// one small register tile; beyond, the ratio itself has to reach SHARED_MIN_RATIO
-// (the passes over the basis and the D(q) blocks grow with T) and the bound is SHARED_MIN_WORK, with
-// other bounds for the mixed forms (SHARED_MIN_RATIO_MIXED, SHARED_MIN_WORK_MIXED). Measured, LU / this form in us
-// (beta = 10 ... 40, U = 3 ... 8). T = 1 below: n = 30, 1440 problems 168 / 230; n = 40, 990 problems 161 / 185; n = 96, 392 problems 444 / 563;
-// above: n = 40, 1350 problems 230 / 187; n = 64, 990 problems 384 / 229; n = 120, 450 problems 608 / 472, 68442 problems
-// 38100 / 3530. T = 4 below: n = 32,
-// 1440 problems 203 / 293; n = 48, 1440 problems 323 / 336; above: n = 64, 1440 problems 550 / 379; n = 80, 1170 problems 607 / 456; n = 120, 1440 problems 1072 / 764; n = 216, 540 problems
-// 1588 / 1300. Large, complex128, below: T = 9, n = 252, 560 problems 2207 / 2652; n = 360, 840 problems 5810 / 7940; n = 720,
-// 448 problems 16025 / 15066 (not far above); above: T = 4, n = 400, 540 problems 5488 / 5309; T = 9, n = 540, 1170 problems
-// 20020 / 15003. Split-BF16 below: T = 9, n = 252, ratio 10; above: n = 360, 840 problems 4617 / 4407, 2790
-// problems 12119 / 8767; n = 720, 448 problems 9814 / 8481, 5642 problems 93282 / 39980; T = 4, n = 320, 448
-// problems 2795 / 2221. Complex64: n = 720, 448 problems 14209 / 9866.
+// one small register tile; beyond, the ratio itself has to reach SHARED_MIN_RATIO (the passes over the basis and the
+// D(q) blocks grow with T), with other bounds for the mixed forms, whose LU is faster too. The lines lie where
+// this form wins by a third: the iterations of a self-consistency loop grow harder than its first (n = 540, 240 and
+// 1080, eight of them, mixing 0.3: 20 -> 37, 5.7 -> 8.4 and 118 -> 212 ms; LU 27, 10.2 and 248), and the LU's time does not.
+// Measured, LU / this form in us (beta = 10 ... 40, U = 3 ... 8). T = 1 below: n = 30, 1440 problems 168 / 230; n = 40,
+// 990 problems 161 / 185, 1350 230 / 187; n = 96, 392 problems 444 / 563; n = 120, 450 problems 608 / 472; above: n = 40,
+// 1890 problems 276 / 184; n = 64, 990 problems 384 / 229; n = 120, 810 problems 765 / 482, 68442 problems 38100 / 3530.
+// T = 4 below: n = 32, 1440 problems 203 / 293; n = 48, 1440 problems 323 / 336; above: n = 64, 1440 problems 550 / 379;
+// n = 120, 1440 problems 1072 / 764; n = 216, 540 problems 1588 / 1300; n = 256, 540 problems 2101 / 1422. Large,
+// complex128, below: T = 9, n = 252, 560 problems 2207 / 2652; n = 360, 2790 problems 18169 / 17032; n = 720, 448
+// problems 16025 / 15066; T = 4, n = 400, 540 problems 5488 / 5309; above: 630 problems 5756 / 3839; T = 9, n = 540, 1170
+// problems 20020 / 15003; n = 720, 5642 problems 239700 / 82000. Split-BF16 below: T = 9, n = 360, 2790 problems 12119 /
+// 8767; n = 540, 2700 problems 26600 / 20050; n = 720, 448 problems 9814 / 8481; T = 4, n = 400, 540 problems 4681 / 3416;
+// above: n = 720, 5642 problems 93282 / 39980. Complex64: n = 720, 720 problems 20929 / 13331.
 constexpr int SHARED_MIN_NQ = 16;
-constexpr double SHARED_MIN_WORK_1 = 17000.0, SHARED_MIN_WORK_4 = 9000.0, SHARED_MIN_WORK_N32 = 30000.0;
-constexpr double SHARED_MIN_WORK = 16000.0, SHARED_MIN_WORK_MIXED = 11000.0;
-constexpr double SHARED_MIN_RATIO = 18.0, SHARED_MIN_RATIO_MIXED = 14.0;
+constexpr double SHARED_MIN_WORK_1 = 20000.0, SHARED_MIN_WORK_4 = 9000.0, SHARED_MIN_WORK_N32 = 30000.0;
+constexpr double SHARED_MIN_WORK = 20000.0, SHARED_MIN_WORK_MIXED = 25000.0;
+constexpr double SHARED_MIN_RATIO = 18.0, SHARED_MIN_RATIO_MIXED = 24.0;
 constexpr int SHARED_TILE_N = 256;
 
 constexpr int SH_M = 10;           // Krylov vectors of a cycle
