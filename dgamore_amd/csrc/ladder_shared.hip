@@ -75,10 +75,12 @@ struct SharedArgs : SharedGroups {
 template <typename S>
 struct SharedTol {
   static constexpr double cycle = SH_CYCLE_TOL, done = SH_DONE_TOL, trust = SH_TRUST;
+  static constexpr double lowest = SH_NORM_MIN, highest = SH_NORM_MAX;
 };
 template <>
 struct SharedTol<float2> {
   static constexpr double cycle = SH_CYCLE_TOL_C64, done = SH_DONE_TOL_C64, trust = SH_TRUST_C64;
+  static constexpr double lowest = SH_NORM_MIN_C64, highest = SH_NORM_MAX_C64;
 };
 
 __device__ __forceinline__ double2 sh_wide(double2 x) { return x; }
@@ -225,6 +227,7 @@ __global__ void __launch_bounds__(256) shared_start_kernel(SharedArgs<S> s, int 
     int st = first ? SH_RUN : s.state[x.col];
     const double xn = first ? nrm : s.xnorm[x.col];
     if (!(nrm <= 1e300)) st = SH_FAIL;  // infinite or NaN
+    if (first && !(nrm >= SharedTol<S>::lowest && nrm <= SharedTol<S>::highest)) st = SH_FAIL;
     if (st == SH_RUN && nrm <= SharedTol<S>::done * xn) st = SH_DONE;
     if (st == SH_RUN && !first && nrm > SH_STAGNATION * xn) st = SH_FAIL;  // P is no inverse
     const int live = x.in && st == SH_RUN;

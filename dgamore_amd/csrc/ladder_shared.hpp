@@ -49,6 +49,11 @@ constexpr double SH_TRUST = 1e-7;
 constexpr double SH_CYCLE_TOL_C64 = 1e-5, SH_DONE_TOL_C64 = 1e-14, SH_TRUST_C64 = 1e-9;
 // A cycle that leaves more than this of its residual is stagnating.
 constexpr double SH_STAGNATION = 0.3;
+// Columns whose first vector P B lies outside these bounds are left to the LU: its square, or that of a residual
+// 2^-53 of it, would leave the range of double (or P and its products that of float), and a column of zeros
+// pass for a converged one.
+constexpr double SH_NORM_MIN = 1e-130, SH_NORM_MAX = 1e130;
+constexpr double SH_NORM_MIN_C64 = 1e-20, SH_NORM_MAX_C64 = 1e20;
 
 enum SharedState { SH_RUN = 0, SH_DONE = 1, SH_FAIL = 2 };
 

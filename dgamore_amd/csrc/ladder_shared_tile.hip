@@ -433,6 +433,7 @@ __device__ __forceinline__ void shared_tile(const SharedTileArgs& ta, SharedLds<
     }
     if (cycle == 0) xn = beta0;
     if (!(beta0 <= 1e300)) state = SH_FAIL;  // infinite or NaN
+    if (cycle == 0 && !(beta0 >= SH_NORM_MIN && beta0 <= SH_NORM_MAX)) state = SH_FAIL;
     if (state == SH_RUN && beta0 <= SH_DONE_TOL * xn) state = SH_DONE;
     if (state == SH_RUN && cycle > 0 && beta0 > SH_STAGNATION * xn) state = SH_FAIL;  // P is no inverse
     const double target = fmax(SH_CYCLE_TOL * beta0, SH_DONE_TOL * xn);
