@@ -284,6 +284,7 @@ __global__ void __launch_bounds__(256) shared_step_kernel(SharedArgs<S> s, int k
     if (j > k) h[j] = make_double2(0.0, 0.0);
     left -= h[j].x * h[j].x + h[j].y * h[j].y;
   }
+  if constexpr (std::is_same<S, float2>::value) left = fmax(left, SH_LOSS_C64 * nrm);
   const double hn = sqrt(fmax(left, 0.0));
   const double inv = hn > 1e-150 ? 1.0 / hn : 0.0;
   const double2* dd = shared_diag(s, x);
@@ -351,7 +352,9 @@ __global__ void __launch_bounds__(256) shared_step_kernel(SharedArgs<S> s, int k
   }
 }
 
-// End of a cycle: X (+)= sum_j y_j V_j with the y of the column's triangular factor, and its state.
+// End of a cycle: X (+)= sum_j y_j V_j with the y of the column's triangular factor, and its state. With a
+// complex64 basis the residual sum_j rho_j V_j is formed in the same pass (rho: the rotated residual turned
+// back; one more vector is read).
 template <typename S>
 __global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs<S> s, int cycle, int last) {
   const int tile_id = blockIdx.x;
@@ -375,6 +378,27 @@ __global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs<S> s, int
       y[j] = cmul(r, cinv(s.R[(static_cast<size_t>(j) * (j + 1) / 2 + j) * cols + col]));
     }
   }
+  constexpr bool C64 = std::is_same<S, float2>::value;
+  double2 rho[C64 ? SH_M : 1], end = make_double2(0.0, 0.0);  // end: of V_kd
+  double ynrm = 0.0;
+  if constexpr (C64) {
+    double2 cur = kd > 0 ? s.gv[static_cast<size_t>(kd) * cols + col] : end;
+#pragma unroll
+    for (int j = SH_M; j > 0; --j) {
+      if (j < SH_M) rho[j] = make_double2(0.0, 0.0);
+      if (j <= kd) {
+        const double2 e = cscale(cur, s.rc[(j - 1) * cols + col]);
+        if (j < SH_M) rho[j] = e;
+        if (j == kd) end = e;
+        const double2 sn = s.rs[(j - 1) * cols + col];
+        cur = cmul(make_double2(-sn.x, -sn.y), cur);
+      }
+    }
+    rho[0] = cur;
+#pragma unroll
+    for (int j = 0; j < SH_M; ++j) ynrm = fma(y[j].x, y[j].x, fma(y[j].y, y[j].y, ynrm));
+    ynrm = sqrt(ynrm);
+  }
   if (x.wave == 0) {
     int km = kd;
     for (int o = 32; o > 0; o >>= 1) km = max(km, __shfl_xor(km, o));
@@ -382,7 +406,7 @@ __global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs<S> s, int
   }
   __syncthreads();
   const int kmax = s_kmax;
-  double nrm = 0.0;
+  double nrm = 0.0, left = 0.0;  // |X|^2 and, with a complex64 basis, the residual's square
   auto pass = [&](auto kc_tag) {
     constexpr int KC = decltype(kc_tag)::value;
 #pragma unroll 2
@@ -392,6 +416,14 @@ __global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs<S> s, int
 #pragma unroll
       for (int j = 0; j < KC; ++j) p[j] = s.V[static_cast<size_t>(j < kmax ? j : 0) * vec + o];
       double2 acc = cycle > 0 ? s.X[o] : make_double2(0.0, 0.0);
+      if constexpr (C64) {
+        const double2 v = sh_wide(s.V[static_cast<size_t>(kmax) * vec + o]);
+        double2 r = kd == kmax ? cmul(end, v) : make_double2(0.0, 0.0);
+#pragma unroll
+        for (int j = 0; j < KC; ++j)
+          if (j <= kd && j < kmax) r = cfma(r, rho[j], sh_wide(p[j]));
+        left = fma(r.x, r.x, fma(r.y, r.y, left));
+      }
 #pragma unroll
       for (int j = 0; j < KC; ++j)
         if (j < kd) acc = cfma(acc, y[j], sh_wide(p[j]));
@@ -407,15 +439,16 @@ __global__ void __launch_bounds__(256) shared_update_kernel(SharedArgs<S> s, int
     case 4: pass(std::integral_constant<int, 8>{}); break;
     default: pass(std::integral_constant<int, SH_M>{}); break;
   }
-  const double xn = sqrt(wave_sum(sh, make_double2(nrm, 0.0), x).x);
+  const double2 norms = wave_sum(sh, make_double2(nrm, left), x);
+  const double xn = sqrt(norms.x);
   if (x.wave == 0) {
     int st = s.state[col];
     if (run) {
       const double2 g = s.gv[static_cast<size_t>(kd) * cols + col];
-      const double res = hypot(g.x, g.y), b0 = s.beta0[col];
+      const double b0 = s.beta0[col], res = C64 ? sqrt(norms.y) : hypot(g.x, g.y);
       if (!(xn <= 1e300) || !(res <= 1e300))
         st = SH_FAIL;
-      else if (cycle > 0 && res <= 2.0 * SharedTol<S>::done * xn && b0 <= SharedTol<S>::trust * xn)
+      else if (cycle > 0 && res <= 2.0 * SharedTol<S>::done * xn && fmax(b0, ynrm) <= SharedTol<S>::trust * xn)
         st = SH_DONE;
       else if (last || !(res <= SH_STAGNATION * b0))
         st = SH_FAIL;

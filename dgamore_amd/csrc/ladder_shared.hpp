@@ -44,9 +44,14 @@ constexpr double SH_DONE_TOL = 2e-16;
 constexpr double SH_TRUST = 1e-7;
 // The same with the basis, P and D(q) in complex64 (the mixed forms above SHARED_TILE_N; X, A0 and the residuals
 // stay in FP64; the split-BF16 form multiplies P in split BF16, with the same number of cycles in every case
-// measured): a cycle can gain five digits, and |X| is wanted to SH_DONE_TOL_C64, four digits beyond what the
-// refinement of the mixed LU asks for.
+// measured): a cycle can gain five digits, and the residual P (B - A X) is wanted below SH_DONE_TOL_C64 of |X|, four
+// digits beyond what the refinement of the mixed LU asks for.
 constexpr double SH_CYCLE_TOL_C64 = 1e-5, SH_DONE_TOL_C64 = 1e-14, SH_TRUST_C64 = 1e-9;
+// The norms and the orthogonality of a complex64 basis hold to about 2^-23 only, so |w|^2 - sum |h|^2 says nothing
+// about a remainder below SH_LOSS_C64 |w|^2 (where D(q) is close to a multiple of A0 it came out as zero, and columns
+// ended at 5e-12). The remainder is taken as no smaller; and whether a column is done decides the norm of the
+// residual as the stored vectors give it, formed with the update of X, not the Hessenberg matrix's estimate.
+constexpr double SH_LOSS_C64 = 2.4e-7;
 // A cycle that leaves more than this of its residual is stagnating.
 constexpr double SH_STAGNATION = 0.3;
 // Columns whose first vector P B lies outside these bounds are left to the LU: its square, or that of a residual
