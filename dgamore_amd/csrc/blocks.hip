@@ -99,12 +99,22 @@ constexpr int row_count = T == 16 ? 8 : T;  // block rows of a workgroup
 template <int T>
 constexpr int row_unroll = T <= 4 ? T : T <= 9 ? 3 : 1;  // rows of the other operand in flight (registers)
 
+// A launch holds fewer than 2^32 work-items per dimension, and the elements (v, q) of a w are counted in 32 bits.
+template <int T>
+static bool row_launch_fits(size_t nvq, size_t nw) {
+  const size_t tiles = (nvq + row_lanes<T> - 1) / row_lanes<T>;
+  return nvq < (size_t(1) << 32) && tiles * nw < (size_t(1) << 31) &&
+         tiles * nw * (T / row_count<T>) * row_lanes<T> < (size_t(1) << 32);
+}
+
 template <int T>
 __global__ void __launch_bounds__(row_lanes<T>* row_count<T>) vrg_kernel(const double2* __restrict__ chi0_inv,
                                                               const double2* __restrict__ aux,
-                                                              double2* __restrict__ vrg, int nvq, int tiles, double beta) {
+                                                              double2* __restrict__ vrg, unsigned nvq, int tiles,
+                                                              double beta) {
   const int part = blockIdx.x % (T / row_count<T>), tile = blockIdx.x / (T / row_count<T>);
-  const int w = tile / tiles, e = (tile - w * tiles) * row_lanes<T> + threadIdx.x;
+  const int w = tile / tiles;
+  const unsigned e = static_cast<unsigned>(tile - w * tiles) * row_lanes<T> + threadIdx.x;
   if (e >= nvq) return;
   const int r = T == 1 ? 0 : part * row_count<T> + __builtin_amdgcn_readfirstlane(threadIdx.y);
   const size_t base = static_cast<size_t>(w) * T * T * nvq + e;
@@ -167,12 +177,14 @@ __global__ void __launch_bounds__(256) chi_phys_kernel(const double2* __restrict
 template <int T>
 __global__ void __launch_bounds__(row_lanes<T>* row_count<T>) kernel_r_kernel(
     const double2* __restrict__ vrg, const double2* __restrict__ chi_phys, const double2* __restrict__ u_r,
-    const double2* __restrict__ v_r, double2* __restrict__ kernel, int nq, int nvq, int tiles, int magn,
+    const double2* __restrict__ v_r, double2* __restrict__ kernel, unsigned nq, unsigned nvq, int tiles, int magn,
     double weight, int accumulate) {
   const int part = blockIdx.x % (T / row_count<T>), tile = blockIdx.x / (T / row_count<T>);
-  const int w = tile / tiles, e = (tile - w * tiles) * row_lanes<T> + threadIdx.x;
+  const int w = tile / tiles;
+  const unsigned e = static_cast<unsigned>(tile - w * tiles) * row_lanes<T> + threadIdx.x;
   if (e >= nvq) return;
-  const int q = e % nq, r = T == 1 ? 0 : part * row_count<T> + __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const unsigned q = e % nq;
+  const int r = T == 1 ? 0 : part * row_count<T> + __builtin_amdgcn_readfirstlane(threadIdx.y);
   const size_t base = static_cast<size_t>(w) * T * T * nvq + e;
   const double2* chi = chi_phys + static_cast<size_t>(w) * T * T * nq + q;
   const double2* vq = v_r ? v_r + static_cast<size_t>(q) * T * T : nullptr;
@@ -276,17 +288,17 @@ extern "C" int dgami_vrg_chi_phys(int nq, int nb, int nw, int niv, double beta, 
   const int nv = 2 * niv;
   const double2* aux = reinterpret_cast<const double2*>(aux_);
   const size_t nvq = static_cast<size_t>(nv) * nq;
-  DGAMI_ARG_CHECK(nvq * nw < (size_t(1) << 37), "vrg_chi_phys: too many elements");
   if (vrg_) {
     DGAMI_ARG_CHECK(chi0_inv_ != nullptr, "vrg_chi_phys: vrg needs chi0_inv");
     const double2* inv = reinterpret_cast<const double2*>(chi0_inv_);
     double2* vrg = reinterpret_cast<double2*>(vrg_);
 #define LAUNCH(T, TS)                                                                                             \
   {                                                                                                               \
-    const size_t tiles = ceil_div(nvq, row_lanes<T>);                                                             \
-    hipLaunchKernelGGL((vrg_kernel<T>), dim3(static_cast<unsigned>(tiles * nw * (T / row_count<T>))),    \
-                       dim3(row_lanes<T>, row_count<T>), 0, stream, \
-                       inv, aux, vrg, static_cast<int>(nvq), static_cast<int>(tiles), beta);                      \
+    const size_t tiles = (nvq + row_lanes<T> - 1) / row_lanes<T>;                                                 \
+    DGAMI_ARG_CHECK(row_launch_fits<T>(nvq, nw), "vrg_chi_phys: too many elements");                              \
+    hipLaunchKernelGGL((vrg_kernel<T>), dim3(static_cast<unsigned>(tiles * nw * (T / row_count<T>))),             \
+                       dim3(row_lanes<T>, row_count<T>), 0, stream, inv, aux, vrg, static_cast<unsigned>(nvq),    \
+                       static_cast<int>(tiles), beta);                                                            \
   }
     DGAMI_DISPATCH_NB(nb, LAUNCH)
 #undef LAUNCH
@@ -322,7 +334,6 @@ extern "C" int dgami_kernel_r(int nq, int nb, int nw, int niv, int channel, doub
   DGAMI_ARG_CHECK(nq >= 1 && nw >= 1 && niv >= 1, "kernel_r: sizes");
   const int nv = 2 * niv;
   const size_t nvq = static_cast<size_t>(nv) * nq;
-  DGAMI_ARG_CHECK(nvq * nw < (size_t(1) << 37), "kernel_r: too many elements");
   const double2* vrg = reinterpret_cast<const double2*>(vrg_);
   const double2* chi = reinterpret_cast<const double2*>(chi_phys_);
   const double2* ur = reinterpret_cast<const double2*>(u_r_);
@@ -330,11 +341,12 @@ extern "C" int dgami_kernel_r(int nq, int nb, int nw, int niv, int channel, doub
   double2* ker = reinterpret_cast<double2*>(kernel_);
 #define LAUNCH(T, TS)                                                                                              \
   {                                                                                                                \
-    const size_t tiles = ceil_div(nvq, row_lanes<T>);                                                              \
-    hipLaunchKernelGGL((kernel_r_kernel<T>), dim3(static_cast<unsigned>(tiles * nw * (T / row_count<T>))),    \
-                       dim3(row_lanes<T>, row_count<T>), 0, stream, \
-                       vrg, chi, ur, vr, ker, nq, static_cast<int>(nvq), static_cast<int>(tiles), channel, weight, \
-                       accumulate);                                                                                \
+    const size_t tiles = (nvq + row_lanes<T> - 1) / row_lanes<T>;                                                  \
+    DGAMI_ARG_CHECK(row_launch_fits<T>(nvq, nw), "kernel_r: too many elements");                                   \
+    hipLaunchKernelGGL((kernel_r_kernel<T>), dim3(static_cast<unsigned>(tiles * nw * (T / row_count<T>))),         \
+                       dim3(row_lanes<T>, row_count<T>), 0, stream, vrg, chi, ur, vr, ker,                         \
+                       static_cast<unsigned>(nq), static_cast<unsigned>(nvq), static_cast<int>(tiles), channel,    \
+                       weight, accumulate);                                                                        \
   }
   DGAMI_DISPATCH_NB(nb, LAUNCH)
 #undef LAUNCH
