@@ -6,6 +6,8 @@
 // izamax); rows move between lanes with wavefront shuffles, so no LDS and no
 // barriers are needed. Blocks are in M order: element (r, c) of the
 // compound block [(o1,o2),(o4,o3)] sits at r*T + c.
+#include <algorithm>
+
 #include "dgami.h"
 #include "dgami_internal.hpp"
 #include "dgami_launch.hpp"
@@ -16,43 +18,47 @@ namespace dgami {
 // ---------------------------------------------------------------------------
 // Sums over v of x [rows][nv][nq]: full over all, core over [v0, v0 + nvc), both times scale (either may be
 // null). 64 (row, q) per workgroup, whose four wavefronts add a quarter of the frequencies each: one thread per
-// (row, q) left a chain of nv loads (64x64, box 120: 39 us, 16x16, box 40: 15 us; now 13 and 4).
+// (row, q) left a chain of nv loads (64x64, box 120: 39 us, 16x16, box 40: 15 us; now 13 and 4). A workgroup goes
+// on to further elements where a launch of 2^32 work-items would not hold them.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) freq_sums_kernel(const double2* __restrict__ x, double2* __restrict__ full,
                                                         double2* __restrict__ core, size_t total, int nq, int nv, int v0,
                                                         int nvc, double scale) {
   __shared__ double2 s_full[4][64], s_core[4][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const size_t idx = blockIdx.x * static_cast<size_t>(64) + lane;
-  double2 sf = make_double2(0.0, 0.0), sc = make_double2(0.0, 0.0);
-  if (idx < total) {
-    const size_t row = idx / nq, q = idx - row * nq;
-    const double2* src = x + row * nv * nq + q;
-    const int per = (nv + 3) / 4, v_end = min(nv, (wave + 1) * per);
+  for (size_t idx0 = blockIdx.x * static_cast<size_t>(64); idx0 < total; idx0 += gridDim.x * static_cast<size_t>(64)) {
+    const size_t idx = idx0 + lane;
+    double2 sf = make_double2(0.0, 0.0), sc = make_double2(0.0, 0.0);
+    if (idx < total) {
+      const size_t row = idx / nq, q = idx - row * nq;
+      const double2* src = x + row * nv * nq + q;
+      const int per = (nv + 3) / 4, v_end = min(nv, (wave + 1) * per);
 #pragma unroll 8
-    for (int v = wave * per; v < v_end; ++v) {
-      const double2 y = src[static_cast<size_t>(v) * nq];
-      sf = cadd(sf, y);
-      if (v >= v0 && v < v0 + nvc) sc = cadd(sc, y);
+      for (int v = wave * per; v < v_end; ++v) {
+        const double2 y = src[static_cast<size_t>(v) * nq];
+        sf = cadd(sf, y);
+        if (v >= v0 && v < v0 + nvc) sc = cadd(sc, y);
+      }
     }
-  }
-  s_full[wave][lane] = sf;
-  s_core[wave][lane] = sc;
-  __syncthreads();
-  if (wave != 0 || idx >= total) return;
+    s_full[wave][lane] = sf;
+    s_core[wave][lane] = sc;
+    __syncthreads();
+    if (wave == 0 && idx < total) {
 #pragma unroll
-  for (int k = 1; k < 4; ++k) {
-    sf = cadd(sf, s_full[k][lane]);
-    sc = cadd(sc, s_core[k][lane]);
+      for (int k = 1; k < 4; ++k) {
+        sf = cadd(sf, s_full[k][lane]);
+        sc = cadd(sc, s_core[k][lane]);
+      }
+      if (full) full[idx] = cscale(sf, scale);
+      if (core) core[idx] = cscale(sc, scale);
+    }
+    __syncthreads();
   }
-  if (full) full[idx] = cscale(sf, scale);
-  if (core) core[idx] = cscale(sc, scale);
 }
 
 static int launch_freq_sums(const double2* x, double2* full, double2* core, size_t rows, int nq, int nv, int v0, int nvc,
                             double scale, hipStream_t stream) {
-  const size_t total = rows * nq, blocks = (total + 63) / 64;
-  DGAMI_ARG_CHECK(blocks < (size_t(1) << 31), "frequency sums: too many elements");
+  const size_t total = rows * nq, blocks = std::min<size_t>((total + 63) / 64, size_t(1) << 22);
   hipLaunchKernelGGL(freq_sums_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, x, full, core, total,
                      nq, nv, v0, nvc, scale);
   DGAMI_HIP_CHECK(hipGetLastError());

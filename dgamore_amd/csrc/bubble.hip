@@ -43,12 +43,13 @@ __global__ void __launch_bounds__(FFT_MAX_THREADS) bubble_kernel(const double2* 
   double2* tw = smem + plan.nlds;
   const int nb4 = nb * nb * nb * nb;
   const int nv = 2 * niv;
-  // blockIdx.x -> (w, blk, v), v fastest; blk in M order ((a*nb+b)*nb+d)*nb+c
-  int idx = blockIdx.x;
+  // workgroup -> (w, blk, v), v fastest; blk in M order ((a*nb+b)*nb+d)*nb+c
+  unsigned idx = flat_block();
   const int v = idx % nv;
   idx /= nv;
   const int blk = idx % nb4;
   const int w = idx / nb4;
+  if (w > niw) return;
   const int c = blk % nb;
   const int d = (blk / nb) % nb;
   const int b = (blk / (nb * nb)) % nb;
@@ -116,7 +117,7 @@ int bubble_run(const BubbleShape& sh, int nx, int ny, int nz, int nb, int niv_g,
   DGAMI_ARG_CHECK(nblocks < (size_t(1) << 31), "bubble: too many slices");
   const double scale = -beta / (static_cast<double>(nk) * nk);
   allow_lds(bubble_kernel, lds);
-  hipLaunchKernelGGL(bubble_kernel, dim3(static_cast<unsigned>(nblocks)), dim3(threads), lds, stream, gr, irrk_ind,
+  hipLaunchKernelGGL(bubble_kernel, flat_grid(nblocks), dim3(threads), lds, stream, gr, irrk_ind,
                      reinterpret_cast<double2*>(chi0), plan, nb, niw, niv, nvg, nq_irr, scale);
   DGAMI_HIP_CHECK(hipGetLastError());
   return 0;

@@ -176,6 +176,14 @@ void* workspace(int slot, size_t bytes);
 
 inline unsigned ceil_div(size_t a, size_t b) { return static_cast<unsigned>((a + b - 1) / b); }
 
+// A grid of `blocks` workgroups in two dimensions (a launch holds fewer than 2^32 work-items in one):
+// workgroup flat_block() of it, those from `blocks` on are padding.
+inline dim3 flat_grid(size_t blocks) {
+  const size_t x = blocks < (size_t(1) << 20) ? blocks : size_t(1) << 20;
+  return dim3(static_cast<unsigned>(x), static_cast<unsigned>((blocks + x - 1) / x));
+}
+__device__ __forceinline__ unsigned flat_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
+
 // Allow a kernel to use more than the default 64 KiB of dynamic LDS (gfx950 has 160 KiB per CU).
 template <typename K>
 inline void allow_lds(K kernel, size_t bytes) {

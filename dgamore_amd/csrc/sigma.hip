@@ -127,8 +127,9 @@ __global__ void __launch_bounds__(FFT_MAX_THREADS) sigma_final_kernel(const doub
   double2* buf = smem + plan.ntw;
   double2* sum = buf;  // [groups][N]; the transform has read it before it writes
   const int T = nb * nb;
-  const int v = blockIdx.x % niv_core;
-  const int ij = blockIdx.x / niv_core;
+  const int v = flat_block() % niv_core;
+  const int ij = flat_block() / niv_core;
+  if (ij >= T) return;
   fft_twiddles<true>(tw, plan);
   const int per = (nchunk + groups - 1) / groups;
   const size_t cstride = static_cast<size_t>(T) * niv_core * N;
@@ -280,7 +281,7 @@ extern "C" int dgami_sigma_from_kernel(int nx, int ny, int nz, int nb, int niw, 
   const int groups = std::max(1, FFT_MAX_THREADS / N);
   const size_t lds2 = (plan.ntw + std::max<size_t>(plan.nlds, static_cast<size_t>(groups) * N)) * sizeof(double2);
   allow_lds(sigma_final_kernel, lds2);
-  hipLaunchKernelGGL(sigma_final_kernel, dim3(base), dim3(FFT_MAX_THREADS), lds2, stream, part,
+  hipLaunchKernelGGL(sigma_final_kernel, flat_grid(base), dim3(FFT_MAX_THREADS), lds2, stream, part,
                      reinterpret_cast<double2*>(sigma), plan, nb, niv_core, nchunk, groups, -0.5 / beta / N);
   DGAMI_HIP_CHECK(hipGetLastError());
   return 0;

@@ -54,3 +54,35 @@ def test_vrg_and_kernel_beyond_2_31_elements(K):
     total = fv.sum() * fq / 2.0
     ref = total / (1.0 + 0.25 * total)
     assert float((chi[0, 0] - ref).abs().max() / ref.abs().max()) < 1e-12
+
+
+def test_frequency_sums_of_2_30_momenta(K):
+    nq = (1 << 30) + 5
+    print(f"[gpu-case] frequency sums over {nq} momenta", flush=True)
+    x = torch.empty((1, 1, 2, nq), dtype=C128, device="cuda")
+    x[0, 0, 0] = 1.5 + 0.25j
+    x[0, 0, 1] = -0.5 + 1.0j
+    marks = [0, 63, 64, (1 << 28) - 1, 1 << 28, (1 << 28) + 64, 1 << 30, nq - 1]
+    for i, q in enumerate(marks):
+        x[0, 0, 0, q] = 10.0 + i
+    inv, full, core = K.chi0_prepare(x, 1, 1, 2.0)
+    torch.cuda.synchronize()
+    del inv, core
+    want = torch.full((nq,), (1.0 + 1.25j) / 4.0, dtype=C128, device="cuda")
+    for i, q in enumerate(marks):
+        want[q] = (9.5 + i + 1.0j) / 4.0
+    assert torch.equal(full[0, 0], want)
+
+
+def test_bubble_of_2_23_slabs_of_4096_points(K):
+    nk, niw, niv, beta = (64, 64, 1), 2047, 2048, 2.0
+    print("[gpu-case] bubble of 2^23 slabs of 64x64", flush=True)
+    ng = niw + niv
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    g = torch.view_as_complex(torch.randn((4096, 2 * ng, 2), dtype=torch.float64, device="cuda", generator=gen))
+    chi = K.bubble_irrq(g.reshape(nk + (1, 1, 2 * ng)), nk, niw, niv, beta, K.to_dev(np.zeros(1), torch.int32))
+    torch.cuda.synchronize()
+    prod = (-beta / 4096) * (g.T.contiguous() @ g)  # q = 0: -beta / N sum_k G(k, v) G(k, v - w)
+    for w in (0, 1, 1023, niw):
+        ref = torch.diagonal(prod, -w)[ng - niv - w:ng + niv - w]  # elements (v, v - w)
+        assert float((chi[w, 0, :, 0] - ref).abs().max()) < 1e-12 * float(prod.abs().max()), w
