@@ -89,6 +89,7 @@ void* workspace(int slot, size_t bytes) {
   size_t want = bytes < 256 ? 256 : bytes;
   if (hipMalloc(&s.ptr, want) != hipSuccess) {
     s.ptr = nullptr;
+    (void)hipGetLastError();  // reported here; left pending, the next launch would seem to have failed
     set_error("workspace: hipMalloc of " + std::to_string(want) + " bytes failed");
     return nullptr;
   }
