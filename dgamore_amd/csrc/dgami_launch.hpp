@@ -41,6 +41,34 @@ constexpr int MAX_EXTRA_STREAMS = 3;
 int extra_stream_fork(hipStream_t caller, int k, hipStream_t* out);
 int extra_stream_join(hipStream_t caller, int k);
 
+// The extra streams of one call: 1, 2, ... forked one after the other, and all joined by join() or,
+// where the call ends in an error, by the destructor: what they still do on the caller's arrays is
+// then ordered before whatever the caller puts on its stream next.
+class ExtraStreamSet {
+ public:
+  explicit ExtraStreamSet(hipStream_t caller) : caller_(caller) {}
+  ExtraStreamSet(const ExtraStreamSet&) = delete;
+  ExtraStreamSet& operator=(const ExtraStreamSet&) = delete;
+  ~ExtraStreamSet() { (void)join(); }
+  int fork(hipStream_t* out) {
+    const int rc = extra_stream_fork(caller_, count_ + 1, out);
+    if (rc == 0) ++count_;
+    return rc;
+  }
+  int join() {
+    int rc = 0;
+    for (; count_ > 0; --count_) {
+      const int r = extra_stream_join(caller_, count_);
+      if (rc == 0) rc = r;
+    }
+    return rc;
+  }
+
+ private:
+  hipStream_t caller_;
+  int count_ = 0;
+};
+
 int launch_fft_grid(const double2* in, double2* out, int64_t batch, int nx, int ny, int nz, int sign, double scale,
                     hipStream_t stream);
 int launch_ref2_to_gk(const double2* in, double2* out, int nk, int nb, int nv_in, int v0, int nv, hipStream_t stream);

@@ -113,8 +113,9 @@ static int ladder_multi(int nmodels, const dgami_ladder_model* models, int preci
   }
   const int nl = std::min(ladder_lanes(), std::max(1, static_cast<int>(spread.size())));
   hipStream_t lane[1 + MAX_EXTRA_STREAMS] = {s};
+  ExtraStreamSet extra(s);
   for (int l = 1; l < nl; ++l)
-    if ((rc = extra_stream_fork(s, l, &lane[l])) != 0) return rc;
+    if ((rc = extra.fork(&lane[l])) != 0) return rc;
   for (size_t m = 0; m < spread.size(); ++m) {
     const int l = static_cast<int>(m % nl);
     if ((rc = ladder_solve_shared(spread[m], precision, lane[l], l * WS_STREAM_STRIDE)) != 0) return rc;
@@ -136,9 +137,7 @@ static int ladder_multi(int nmodels, const dgami_ladder_model* models, int preci
     mm.start[mm.nmodels] = static_cast<int>(total);
     if ((rc = ladder_reg_launch_multi(variant, mm, s)) != 0) return rc;
   }
-  for (int l = 1; l < nl; ++l)
-    if ((rc = extra_stream_join(s, l)) != 0) return rc;
-  return 0;
+  return extra.join();
 }
 
 }  // namespace dgami

@@ -1284,6 +1284,7 @@ int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream) {
     hipStream_t s;
   };
   Lane lanes[1 + MAX_EXTRA_STREAMS];
+  ExtraStreamSet extra(stream);
   for (int l = 0; l < nl; ++l) {
     Lane& L = lanes[l];
     if (!blocked_alloc(L.st, n, ld, ncol, batch, WS_LADDER + l * WS_STREAM_STRIDE)) return -2;
@@ -1293,7 +1294,7 @@ int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream) {
     if (!L.tri) return -2;
     L.s = stream;
     if (l > 0) {
-      const int rc = extra_stream_fork(stream, l, &L.s);
+      const int rc = extra.fork(&L.s);
       if (rc) return rc;
     }
   }
@@ -1315,11 +1316,7 @@ int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream) {
     rc = blocked_copy_info(a, L.st.info, static_cast<int>(item0), nb, L.s);
     if (rc) return rc;
   }
-  for (int l = 1; l < nl; ++l) {
-    const int rc = extra_stream_join(stream, l);
-    if (rc) return rc;
-  }
-  return 0;
+  return extra.join();
 }
 
 }  // namespace dgami

@@ -540,17 +540,16 @@ int ladder_solve_mixed(const LadderArgs& a, int precision, hipStream_t stream) {
   Lane lanes[1 + MAX_EXTRA_STREAMS];
   int rc = setup(lanes[0], 0, stream);
   if (rc) return rc;
+  ExtraStreamSet extra(stream);
   for (int l = 1; l < nl; ++l) {
     hipStream_t sx = nullptr;
-    if ((rc = extra_stream_fork(stream, l, &sx)) != 0) return rc;
+    if ((rc = extra.fork(&sx)) != 0) return rc;
     if ((rc = setup(lanes[l], l * WS_STREAM_STRIDE, sx)) != 0) return rc;
   }
   int k = 0;
   for (size_t g0 = 0; g0 < groups; g0 += gb, k = (k + 1) % nl)
     if ((rc = run(lanes[k], g0)) != 0) return rc;
-  for (int l = 1; l < nl; ++l)
-    if ((rc = extra_stream_join(stream, l)) != 0) return rc;
-  return 0;
+  return extra.join();
 }
 
 }  // namespace dgami

@@ -281,6 +281,7 @@ static int vertex_solve_t(LadderArgs a, int what, const VertexArgs& o_in, int ge
     hipStream_t s;
   };
   Lane lanes[1 + MAX_EXTRA_STREAMS];
+  ExtraStreamSet extra(stream);
   for (int l = 0; l < nl; ++l) {
     Lane& L = lanes[l];
     if (!blocked_alloc(L.st, n, ld, ncol, batch, WS_LADDER + l * WS_STREAM_STRIDE)) return -2;
@@ -289,7 +290,7 @@ static int vertex_solve_t(LadderArgs a, int what, const VertexArgs& o_in, int ge
     if (!L.tri) return -2;
     L.s = stream;
     if (l > 0) {
-      const int rc = extra_stream_fork(stream, l, &L.s);
+      const int rc = extra.fork(&L.s);
       if (rc) return rc;
     }
   }
@@ -338,11 +339,7 @@ static int vertex_solve_t(LadderArgs a, int what, const VertexArgs& o_in, int ge
     rc = blocked_copy_info(a, st.info, static_cast<int>(item0), nb, stream);
     if (rc) return rc;
   }
-  for (int l = 1; l < nl; ++l) {
-    const int rc = extra_stream_join(stream, l);
-    if (rc) return rc;
-  }
-  return 0;
+  return extra.join();
 }
 
 // precision: DGAMI_PLAIN_FP64 (complex128 LU), or a complex64 LU with FP32 (DGAMI_MIXED_FP32_IR) or
