@@ -1,18 +1,21 @@
 """Autotuner of the batched ladder solves.
 
-The library can run one ladder shape -- compound size n = nb^2 * 2 niv, nrhs = nb^2 right-hand
+The library can run the LU of one ladder shape -- compound size n = nb^2 * 2 niv, nrhs = nb^2 right-hand
 sides, a precision mode -- with several kernels: register-tile variants and column-cyclic
 variants for small n (plain FP64 only), and blocked-LU panel shapes (panel width 32 or 16,
 rows per panel thread) for any n up to 1536. tune_ladder() times every candidate on a
 synthetic, well-conditioned batch of the caller's shape, drops any whose result differs from
-the library's default kernel, stores the fastest in the library's process-wide table (which
-every later ladder call of that shape reads) and records it in a JSON cache keyed by the GPU
-name, so that a later process loads the choice without timing again.
+the library's default LU kernel, stores the fastest in the library's process-wide table (which
+every later LU of that shape reads) and records it in a JSON cache keyed by the GPU name, so
+that a later process loads the choice without timing again. Calls that the library solves
+through the matrix their q-points share are no LU: while the tuner times, its thread's calls
+take the LU in any case, and the table does not decide where that form runs.
 
 The reference has no counterpart: NumPy's inverse and solve pick their LAPACK kernels
 themselves (four_point.py:620-684).
 """
 
+import contextlib
 import ctypes
 import json
 import os
@@ -84,8 +87,8 @@ def _device_key():
 
 def _key(n, nrhs, precision, nitems):
     # problems per call enter as a power-of-two bucket: a full GPU and a nearly empty one may prefer
-    # different kernels
-    return f"{n}:{nrhs}:{PRECISION_NAMES[precision]}:{1 << max(0, int(nitems) - 1).bit_length()}"
+    # different kernels ("lu": the LU was timed, whatever form a call of that size takes)
+    return f"lu:{n}:{nrhs}:{PRECISION_NAMES[precision]}:{1 << max(0, int(nitems) - 1).bit_length()}"
 
 
 def _read_cache(path):
@@ -165,6 +168,33 @@ def tune_ladder(nb, niv, nq, nw, nchan=2, precision=_lib.PLAIN_FP64, reps=3, use
     flops = 8.0 / 3.0 * n**3 + 8.0 * nrhs * n**2
     nq_t = int(max(1, min(nq, TUNE_FLOPS // max(flops * nchan * nw, 1.0))))
     inv, gamma, u_r = _problem(nb, niv, nq_t, nw, nchan)
+    with _lu_only():
+        times = _time_candidates(cands, inv, gamma, u_r, n, nrhs, precision, reps, verbose)
+    best = min(times, key=times.get)
+    set_choice(n, nrhs, precision, best)
+    entry = dict(choice=best, name=kernel_name(best), times_ms={kernel_name(k): round(v, 4) for k, v in times.items()},
+                 problems_timed=nchan * nw * nq_t, tuned_at=time.strftime("%Y-%m-%d %H:%M:%S"))
+    if use_cache:
+        data = _read_cache(path)
+        data.setdefault(_device_key(), {})[key] = entry
+        _write_cache(path, data)
+    return dict(entry, n=n, nrhs=nrhs, source="timed")
+
+
+@contextlib.contextmanager
+def _lu_only():
+    """Ladder calls of this thread take the LU."""
+    lib = _lib.load()
+    lib.dgami_ladder_tune_lu(1)
+    try:
+        yield
+    finally:
+        lib.dgami_ladder_tune_lu(0)
+
+
+def _time_candidates(cands, inv, gamma, u_r, n, nrhs, precision, reps, verbose):
+    """Times in ms of the candidates whose results agree with the default LU kernel's."""
+    problems = gamma.shape[0] * inv.shape[0] * inv.shape[-1]
     set_choice(n, nrhs, precision, None)
     ref, _ = K.ladder_solve_sum(inv, gamma, u_r, None, 1.0, precision, check_info=False)
     tol = 1e-9 if precision == _lib.PLAIN_FP64 else 1e-7
@@ -183,18 +213,10 @@ def tune_ladder(nb, niv, nq, nw, nchan=2, precision=_lib.PLAIN_FP64, reps=3, use
                               reps)
         if verbose:
             print(f"[tune] n={n} nrhs={nrhs} {PRECISION_NAMES[precision]} {kernel_name(kid)}: "
-                  f"{times[kid]:.3f} ms ({nchan * nw * nq_t} problems)", file=sys.stderr, flush=True)
+                  f"{times[kid]:.3f} ms ({problems} problems)", file=sys.stderr, flush=True)
     if not times:
         raise RuntimeError(f"every ladder kernel candidate failed for n={n}")
-    best = min(times, key=times.get)
-    set_choice(n, nrhs, precision, best)
-    entry = dict(choice=best, name=kernel_name(best), times_ms={kernel_name(k): round(v, 4) for k, v in times.items()},
-                 problems_timed=nchan * nw * nq_t, tuned_at=time.strftime("%Y-%m-%d %H:%M:%S"))
-    if use_cache:
-        data = _read_cache(path)
-        data.setdefault(_device_key(), {})[key] = entry
-        _write_cache(path, data)
-    return dict(entry, n=n, nrhs=nrhs, source="timed")
+    return times
 
 
 def tune_models(models, nchan=2, precision=_lib.PLAIN_FP64, **kw):

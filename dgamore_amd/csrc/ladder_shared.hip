@@ -30,6 +30,7 @@
 #include "dgami_launch.hpp"
 #include "ladder_common.hpp"
 #include "ladder_shared.hpp"
+#include "ladder_tune.hpp"
 #include "cgemm.hpp"
 #include "zgemm.hpp"
 
@@ -670,7 +671,7 @@ static int shared_solve(SharedArgs<S>& s, hipStream_t stream) {
 bool ladder_shared_applies(const LadderArgs& a, int precision) {
   if (a.dense || a.rhs_mode != LADDER_RHS_INDICATOR || a.items) return false;
   if (a.T != 1 && a.T != 4 && a.T != 9 && a.T != 16) return false;
-  if (a.n > 1536 || a.nq < 2) return false;
+  if (a.n > 1536 || a.nq < 2 || ladder_tune_lu_only()) return false;
   const char* v = getenv("DGAMI_LADDER_SHARED");
   if (v && *v) return std::string(v) == "1";
   if (a.nq < SHARED_MIN_NQ) return false;

@@ -51,6 +51,12 @@ int ladder_tuned_kernel(int n, int nrhs, int precision) {
   return -1;
 }
 
+namespace {
+thread_local bool t_lu_only = false;
+}  // namespace
+
+bool ladder_tune_lu_only() { return t_lu_only; }
+
 }  // namespace dgami
 
 using namespace dgami;
@@ -96,5 +102,10 @@ extern "C" int dgami_ladder_tune_get(int n, int nrhs, int precision) {
 extern "C" int dgami_ladder_tune_clear(void) {
   std::lock_guard<std::mutex> lock(g_tune_mutex);
   g_tune.clear();
+  return 0;
+}
+
+extern "C" int dgami_ladder_tune_lu(int on) {
+  t_lu_only = on != 0;
   return 0;
 }

@@ -2,7 +2,7 @@
 //
 // A kernel id is family * 256 + variant. The host-side autotuner times the candidates of a
 // shape and stores the fastest in a process-wide table; the solve entry points read it on
-// every call and fall back to the built-in size rule when the shape has no entry.
+// every call that takes an LU and fall back to the built-in size rule when the shape has no entry.
 #pragma once
 
 namespace dgami {
@@ -25,6 +25,9 @@ bool blocked_variant_fits(bool complex64, int variant, int n);
 
 // Tuned kernel id of (n, nrhs, precision), or -1 when the autotuner has not set one.
 int ladder_tuned_kernel(int n, int nrhs, int precision);
+
+// True while this host thread tunes (dgami_ladder_tune_lu): its ladder calls take the LU in any case.
+bool ladder_tune_lu_only();
 
 // Register and column-cyclic variant limits (defined with their kernels).
 int ladder_reg_variant_count();

@@ -184,14 +184,17 @@ int dgami_ladder_solve_sum_multi_prec(int nmodels, const dgami_ladder_model* mod
  * tiles, 2 = column-cyclic, 3 = blocked LU (variant: panel shape). candidates() writes up to `cap`
  * ids that can run a compound size n with nrhs right-hand sides in `precision` and returns how many
  * there are; set() stores the choice for (n, nrhs, precision) in a process-wide table that every
- * later ladder call reads (kernel_id -1 removes it); get() returns the stored id or -1; clear()
- * empties the table. The environment variable DGAMI_LADDER_KERNEL still overrides the table. No
+ * later ladder call that takes an LU reads (kernel_id -1 removes it); get() returns the stored id or
+ * -1; clear() empties the table. lu(1) makes the calling host thread's ladder calls take the LU
+ * also where the q-points' shared matrix would serve them, until lu(0): what the tuner times are
+ * the kernels of the table. The environment variable DGAMI_LADDER_KERNEL still overrides the table. No
  * counterpart in the reference (NumPy picks its LAPACK kernels itself); the host-side autotuner
  * times the candidates and fills the table. */
 int dgami_ladder_tune_candidates(int n, int nrhs, int precision, int* ids, int cap);
 int dgami_ladder_tune_set(int n, int nrhs, int precision, int kernel_id);
 int dgami_ladder_tune_get(int n, int nrhs, int precision);
 int dgami_ladder_tune_clear(void);
+int dgami_ladder_tune_lu(int on);
 
 /* Dense-matrix variant of the ladder solve: a_cmp holds nmat assembled compound matrices
  * [nmat][n][n] (n = nb^2 * 2*niv); out[nmat][n][nb^2] = (1/beta) sum_v' [A^-1]_{(o1,o2,v),(o4,o3,v')}
