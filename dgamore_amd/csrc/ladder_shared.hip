@@ -677,7 +677,8 @@ bool ladder_shared_applies(const LadderArgs& a, int precision) {
   if (a.nq < SHARED_MIN_NQ) return false;
   const double ratio = a.n / (3.0 * a.T) + 1.0, work = static_cast<double>(a.nchan) * a.nw * a.nq * ratio;
   if (a.n <= 32) return work >= SHARED_MIN_WORK_N32 && a.T <= 4;
-  if (a.n <= SHARED_TILE_N && a.T <= 4) return work >= (a.T == 1 ? SHARED_MIN_WORK_1 : SHARED_MIN_WORK_4);
+  if (a.n <= SHARED_TILE_N && a.T <= 4)
+    return work >= (a.T == 1 ? SHARED_MIN_WORK_1 : SHARED_MIN_WORK_4)[a.n <= 64 ? 0 : a.n <= 128 ? 1 : 2];
   return precision == DGAMI_PLAIN_FP64 ? ratio >= SHARED_MIN_RATIO && work >= SHARED_MIN_WORK
                                        : ratio >= SHARED_MIN_RATIO_MIXED && work >= SHARED_MIN_WORK_MIXED;
 }

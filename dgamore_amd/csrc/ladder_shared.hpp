@@ -9,25 +9,32 @@ namespace dgami {
 
 // The rule: at least SHARED_MIN_NQ q-points share a matrix (its inversion costs three LUs), and there are
 // enough problems for the LU to be past its own latency, by how much more an LU computes per problem than a
-// product: problems x ratio >= a bound, with ratio = n / (3 T) + 1. With one or two orbitals up to n = 256 the
-// bound is SHARED_MIN_WORK_1 (T = 1) or SHARED_MIN_WORK_4, and SHARED_MIN_WORK_N32 up to n = 32, where the LU is
-// one small register tile; beyond, the ratio itself has to reach SHARED_MIN_RATIO (the passes over the basis and the
-// D(q) blocks grow with T), with other bounds for the mixed forms, whose LU is faster too. The lines lie where
-// this form wins by a third: the iterations of a self-consistency loop grow harder than its first (n = 540, 240 and
-// 1080, eight of them, mixing 0.3: 20 -> 37, 5.7 -> 8.4 and 118 -> 212 ms; LU 27, 10.2 and 248), and the LU's time does not.
-// Measured, LU / this form in us (beta = 10 ... 40, U = 3 ... 8). T = 1 below: n = 30, 1440 problems 168 / 230; n = 40,
-// 990 problems 161 / 185, 1350 230 / 187; n = 96, 392 problems 444 / 563; n = 120, 450 problems 608 / 472; above: n = 40,
-// 1890 problems 276 / 184; n = 64, 990 problems 384 / 229; n = 120, 810 problems 765 / 482, 68442 problems 38100 / 3530.
-// T = 4 below: n = 32, 1440 problems 203 / 293; n = 48, 1440 problems 323 / 336; above: n = 64, 1440 problems 550 / 379;
-// n = 120, 1440 problems 1072 / 764; n = 216, 540 problems 1588 / 1300; n = 256, 540 problems 2101 / 1422. Large,
-// complex128, below: T = 9, n = 252, 560 problems 2207 / 2652; n = 360, 2790 problems 18169 / 17032; n = 720, 448
-// problems 16025 / 15066; T = 4, n = 400, 540 problems 5488 / 5309; above: 630 problems 5756 / 3839; T = 9, n = 540, 1170
-// problems 20020 / 15003; n = 720, 5642 problems 239700 / 82000. Split-BF16 below: T = 9, n = 360, 2790 problems 12119 /
-// 8767; n = 540, 2700 problems 26600 / 20050; n = 720, 448 problems 9814 / 8481; T = 4, n = 400, 540 problems 4681 / 3416;
-// above: n = 720, 5642 problems 93282 / 39980. Complex64: n = 720, 720 problems 20929 / 13331.
+// product: work = problems x ratio reaches a bound, with ratio = n / (3 T) + 1. The LU's time does not depend on the
+// data, this form's does: the matrices of a self-consistency loop are harder than those of its first iteration, 10 ... 18
+// iterations per column there, 14 ... 35 at the eighth. The lines lie where the first eight iterations of a loop
+// (mixing 0.3) take this form no longer than the LU, in the geometric mean over a strong and a weak interaction,
+// within 3%. That leaves the last of them slower near a line (by up to 1.9 times) and faster from about twice the
+// bound on; a single first iteration gains 1.2 ... 3 times everywhere above.
+// Measured: problems, work: LU / mean of the eight, and LU / the first and the last, strong and weak interaction.
+// T = 1, n = 30: 1890, 20790: 0.82; 2790, 30690: 1.07 (1.59 0.96, 1.24 0.82). n = 40: 1440, 20640: 0.81;
+// 1890, 27090: 0.97 (1.49 0.81, 1.18 0.73); 3822, 54782: 1.64 (2.49 1.36, 1.99 1.24). n = 64: 990, 22110: 0.99; 1350, 30150:
+// 1.28. n = 80: 1188, 32868: 1.06. n = 96: 990, 32670: 0.96. n = 120: 810, 33210: 0.98; 1170, 47970: 1.18 (2.02 0.61, 1.64 0.83);
+// 2790, 114390: 1.88. n = 150: 990, 50490: 0.92. n = 200: 630, 42630: 1.01; 1530, 103530: 1.61. n = 240: 810, 65610: 1.21.
+// T = 4, n = 32: 3690, 13530: 0.96. n = 48: 1890, 9450: 1.04. n = 64: 1440, 9120: 1.23 (1.61 1.24, 1.34 0.94). n = 96: 1440, 12960:
+// 0.97. n = 120: 990, 10890: 1.01; 1440, 15840: 1.11; 2912, 32032: 1.21. n = 160: 1584, 22704: 0.89; 2730, 39130: 1.06.
+// n = 216: 540, 10260: 0.81; 1080, 20520: 1.05; 2184, 41496: 1.37 (1.97 1.19, 1.60 0.86). n = 256: 540, 12060: 0.91; 2002, 44711: 1.52.
+// Large, complex128: T = 4, n = 320: 1890, 52290: 0.87; n = 400: 1452, 49852: 0.88; 3822, 131222: 1.51 (2.79 0.96, 2.05 1.04);
+// n = 720: 630, 38430: 0.97; 1350, 82350: 1.55. T = 9, n = 360: 2912, 41739: 0.80; n = 540: 2366, 49686: 0.90; 5642, 118482:
+// 1.30; n = 720: 1638, 45318: 0.92; 2366, 65459: 1.12; 5642, 156095: 1.59 (2.38 1.29, 1.91 1.18); n = 1080: 1274, 52234: 1.30.
+// Complex64 and split BF16: T = 4, n = 320: 1890: 1.11, 1.04; n = 400: 630, 21630: 0.83, 0.75; 1452: 1.19, 1.05; T = 9,
+// n = 540: 1170, 24570: 0.85, 0.78; n = 720: 728, 20141: 0.91, 0.80; 1638: 1.14, 1.02; 5642: 2.01, 1.66.
 constexpr int SHARED_MIN_NQ = 16;
-constexpr double SHARED_MIN_WORK_1 = 20000.0, SHARED_MIN_WORK_4 = 9000.0, SHARED_MIN_WORK_N32 = 30000.0;
-constexpr double SHARED_MIN_WORK = 20000.0, SHARED_MIN_WORK_MIXED = 25000.0;
+constexpr double SHARED_MIN_WORK_N32 = 30000.0;  // n <= 32, where the LU is one small register tile (T <= 4)
+// up to n = 64 (the inverse in the small register tile), 128 and 256, one (T = 1) and two (T = 4) orbitals
+constexpr double SHARED_MIN_WORK_1[3] = {27000.0, 35000.0, 60000.0};
+constexpr double SHARED_MIN_WORK_4[3] = {9000.0, 13500.0, 30000.0};
+// the large form: with a small ratio the passes over the basis and the D(q) blocks, which grow with T, weigh more
+constexpr double SHARED_MIN_WORK = 65000.0, SHARED_MIN_WORK_MIXED = 45000.0;
 constexpr double SHARED_MIN_RATIO = 18.0, SHARED_MIN_RATIO_MIXED = 24.0;
 constexpr int SHARED_TILE_N = 256;
 
