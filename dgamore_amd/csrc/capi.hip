@@ -98,6 +98,14 @@ void* workspace(int slot, size_t bytes) {
   return s.ptr;
 }
 
+size_t workspace_bytes(int slot) {
+  std::lock_guard<std::mutex> lock(g_ws_mutex);
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || slot >= static_cast<int>(g_slots.size())) return 0;
+  const Slot& s = g_slots[slot];
+  return s.ptr != nullptr && s.device == dev ? s.bytes : 0;
+}
+
 namespace {
 struct ExtraStreams {
   hipStream_t stream[MAX_EXTRA_STREAMS] = {};

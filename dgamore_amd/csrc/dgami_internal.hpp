@@ -173,6 +173,8 @@ int profile_end(hipStream_t stream, hipEvent_t start, double bytes, double flops
 // Grow-only device scratch owned by the library, one slot per purpose id.
 // Returns nullptr (and sets the error) when the allocation fails.
 void* workspace(int slot, size_t bytes);
+// Bytes the slot holds on the current device now.
+size_t workspace_bytes(int slot);
 
 inline unsigned ceil_div(size_t a, size_t b) { return static_cast<unsigned>((a + b - 1) / b); }
 

@@ -28,8 +28,8 @@ enum WorkspaceSlot {
   // slot + k * WS_STREAM_STRIDE
   WS_STREAM_STRIDE = 16,
   // slots of the shared-vertex ladder (beyond the extra streams' ranges; offset by the stride there too)
-  WS_SHARED = 64,       // mean matrices, their inverses and the q-dependent part
-  WS_SHARED_VEC = 65,   // Krylov basis and iterates
+  WS_SHARED_VEC = 64,   // Krylov basis and iterates; then the matrices of the problems left to the LU
+  WS_SHARED = 65,       // mean matrices, their inverses and the q-dependent part; then those LUs' pivots
   WS_SHARED_STATE = 66, // per-column Hessenberg factors and states, list of unconverged problems
 };
 constexpr int MAX_EXTRA_STREAMS = 3;

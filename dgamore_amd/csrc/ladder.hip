@@ -47,7 +47,10 @@ int ladder_solve_fp64(const LadderArgs& a, hipStream_t stream) {
     const int v = ladder_col_variant(a.n, a.T);
     if (v >= 0) return ladder_col_launch(v, a, stream);
   }
-  if (f.empty() && ladder_shared_applies(a, DGAMI_PLAIN_FP64)) return ladder_solve_shared(a, DGAMI_PLAIN_FP64, stream);
+  if (f.empty() && ladder_shared_applies(a, DGAMI_PLAIN_FP64)) {
+    const int rc = ladder_solve_shared(a, DGAMI_PLAIN_FP64, stream);
+    if (rc != SHARED_NO_SPACE) return rc;
+  }
   if (f.empty()) {
     const int tuned = ladder_tuned_kernel(a.n, a.T, DGAMI_PLAIN_FP64);
     if (tuned >= 0) {
@@ -74,8 +77,13 @@ static int ladder_multi(int nmodels, const dgami_ladder_model* models, int preci
   DGAMI_ARG_CHECK(precision == DGAMI_PLAIN_FP64 || precision == DGAMI_MIXED_FP32_IR ||
                       precision == DGAMI_MIXED_BF16X3_IR,
                   "ladder_multi: unknown precision mode");
-  std::vector<LadderArgs> small, spread;
+  std::vector<LadderArgs> small, spread, late;
   int rc = 0;
+  // one model on the caller's stream, in the form its size and precision take
+  auto solve = [&](const LadderArgs& a) {
+    return precision == DGAMI_PLAIN_FP64 || fp64_reg_choice(a.n, a.T) >= 0 ? ladder_solve_fp64(a, s)
+                                                                           : ladder_solve_mixed(a, precision, s);
+  };
   for (int m = 0; m < nmodels; ++m) {
     const dgami_ladder_model& md = models[m];
     DGAMI_ARG_CHECK(md.chi0_inv && md.gamma && md.u_r && md.chi_aux_sum, "ladder_multi: null pointer in a model");
@@ -104,11 +112,11 @@ static int ladder_multi(int nmodels, const dgami_ladder_model* models, int preci
     if (!(force && *force) && ladder_shared_applies(a, precision)) {
       if (ladder_col_variant(a.n, a.T) >= 0)
         spread.push_back(a);
-      else if ((rc = ladder_solve_shared(a, precision, s)) != 0)
+      else if ((rc = solve(a)) != 0)
         return rc;
     } else if (fp64_reg_choice(a.n, a.T) >= 0)
       small.push_back(a);
-    else if ((rc = precision == DGAMI_PLAIN_FP64 ? ladder_solve_fp64(a, s) : ladder_solve_mixed(a, precision, s)) != 0)
+    else if ((rc = solve(a)) != 0)
       return rc;
   }
   const int nl = std::min(ladder_lanes(), std::max(1, static_cast<int>(spread.size())));
@@ -118,7 +126,11 @@ static int ladder_multi(int nmodels, const dgami_ladder_model* models, int preci
     if ((rc = extra.fork(&lane[l])) != 0) return rc;
   for (size_t m = 0; m < spread.size(); ++m) {
     const int l = static_cast<int>(m % nl);
-    if ((rc = ladder_solve_shared(spread[m], precision, lane[l], l * WS_STREAM_STRIDE)) != 0) return rc;
+    rc = ladder_solve_shared(spread[m], precision, lane[l], l * WS_STREAM_STRIDE);
+    if (rc == SHARED_NO_SPACE)
+      late.push_back(spread[m]);
+    else if (rc != 0)
+      return rc;
   }
   // the register-resident models, LADDER_MULTI_MAX per launch, in the largest variant of the group
   for (size_t g0 = 0; g0 < small.size(); g0 += LADDER_MULTI_MAX) {
@@ -137,7 +149,10 @@ static int ladder_multi(int nmodels, const dgami_ladder_model* models, int preci
     mm.start[mm.nmodels] = static_cast<int>(total);
     if ((rc = ladder_reg_launch_multi(variant, mm, s)) != 0) return rc;
   }
-  return extra.join();
+  if ((rc = extra.join()) != 0) return rc;
+  for (const LadderArgs& a : late)
+    if ((rc = solve(a)) != 0) return rc;
+  return 0;
 }
 
 }  // namespace dgami

@@ -1263,6 +1263,24 @@ int ladder_lanes() {
   return s >= 1 && s <= 1 + MAX_EXTRA_STREAMS ? s : 2;
 }
 
+// Problems of a subset per pass. The matrices lie in the slot the shared form's vectors are done with, which grows for
+// them to at most a quarter of the device memory that is free: the subset is empty as a rule, and memory taken for
+// it is missing elsewhere (5642 problems of n = 720: 47 GB where the card is empty, beside 4 ... 12 GB of the shared
+// form; an empty pass over them takes 0.9 ms). Under capture the slot stays as the warm-up left it.
+static size_t subset_batch(size_t items, size_t per, hipStream_t stream) {
+  const size_t have = workspace_bytes(WS_SHARED_VEC), all = items * per;
+  size_t bytes = have;
+  if (have < all) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    size_t avail = 0, total = 0;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture == hipStreamCaptureStatusNone) {
+      if (hipMemGetInfo(&avail, &total) == hipSuccess) bytes = std::max(have, std::min(all, (avail + have) / 4));
+      (void)hipGetLastError();
+    }
+  }
+  return std::max<size_t>(1, std::min(items, bytes / per));
+}
+
 int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream) {
   const int n = a.n, ncol = n + a.T;
   // rows start on 128-byte boundaries (8 complex128 values)
@@ -1276,6 +1294,7 @@ int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream) {
   size_t batch = (size_t(48) << 30) / (per * nl);
   if (batch < 1) batch = 1;
   if (batch > (items + nl - 1) / nl) batch = (items + nl - 1) / nl;
+  if (a.nitems) batch = std::min(batch, subset_batch(items, per, stream));
   if (batch > 65535) batch = 65535;
   const int nblk = static_cast<int>(ceil_div(n, TRI_B));
   struct Lane {
@@ -1287,11 +1306,17 @@ int ladder_blocked_fp64(const LadderArgs& a, int variant, hipStream_t stream) {
   ExtraStreamSet extra(stream);
   for (int l = 0; l < nl; ++l) {
     Lane& L = lanes[l];
-    if (!blocked_alloc(L.st, n, ld, ncol, batch, WS_LADDER + l * WS_STREAM_STRIDE)) return -2;
+    auto alloc = [&]() {
+      if (!blocked_alloc(L.st, n, ld, ncol, batch, (a.nitems ? WS_SHARED_VEC : WS_LADDER) + l * WS_STREAM_STRIDE)) return false;
+      L.tri = static_cast<double2*>(
+          workspace(WS_TRI + l * WS_STREAM_STRIDE, batch * nblk * 2 * TRI_B * TRI_B * sizeof(double2)));
+      return L.tri != nullptr;
+    };
+    while (!alloc()) {
+      if (!a.nitems || batch == 1) return -2;
+      batch = (batch + 1) / 2;
+    }
     L.st.variant = variant;
-    L.tri = static_cast<double2*>(
-        workspace(WS_TRI + l * WS_STREAM_STRIDE, batch * nblk * 2 * TRI_B * TRI_B * sizeof(double2)));
-    if (!L.tri) return -2;
     L.s = stream;
     if (l > 0) {
       const int rc = extra.fork(&L.s);

@@ -387,7 +387,10 @@ int ladder_solve_mixed(const LadderArgs& a, int precision, hipStream_t stream) {
   DGAMI_ARG_CHECK(precision == DGAMI_MIXED_FP32_IR || precision == DGAMI_MIXED_BF16X3_IR,
                   "ladder: unknown mixed-precision mode");
   // many q-points that share a matrix: on FP64 residuals too, with the smaller errors
-  if (ladder_shared_applies(a, precision)) return ladder_solve_shared(a, precision, stream);
+  if (ladder_shared_applies(a, precision)) {
+    const int rc = ladder_solve_shared(a, precision, stream);
+    if (rc != SHARED_NO_SPACE) return rc;
+  }
   // the split-BF16 factors carry ~2^-16 relative error per product instead of 2^-24, so
   // each refinement step gains fewer digits and more steps may be needed
   const int max_solves = precision == DGAMI_MIXED_BF16X3_IR ? MIXED_MAX_SOLVES_BF16 : MIXED_MAX_SOLVES_FP32;

@@ -766,25 +766,29 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
   const bool tiles = n <= SHARED_TILE_N;
   const bool c64 = !tiles && precision != DGAMI_PLAIN_FP64;
   const size_t pk = tiles ? shared_packed(n) : 0;
-  // groups per batch: matrices and, for large sizes, vectors of at most 24 GiB
+  // groups per batch: matrices and, for large sizes, vectors of at most 24 GiB, fewer where the device holds less
   const size_t per_group = (2 * (nn + pk) + shared_inverse_workspace(n)) * sizeof(double2) + (tiles ? 0 : large_vectors(a, 1, N, c64)) +
                            (c64 ? shared_narrow_p(a, 1) * sizeof(float2) : 0);
-  const size_t gb = std::max<size_t>(1, std::min<size_t>({(size_t(24) << 30) / per_group, G, 65535}));
+  size_t gb = std::max<size_t>(1, std::min<size_t>({(size_t(24) << 30) / per_group, G, 65535}));
   SharedGroups s{};
   s.a = a;
   s.N = N;
-  s.groups = static_cast<int>(gb);
-
   const size_t rows = static_cast<size_t>(a.nw) * TT * a.nv;
   const size_t vsz = a.v_r ? static_cast<size_t>(a.nchan) * TT : 0, dvsz = vsz * nq;
-  const size_t szc = rows + rows * nq + vsz + dvsz + gb * ((nn + pk) * 2 + n * T + shared_inverse_workspace(n));
-  const size_t nsz = c64 ? shared_narrow_p(a, gb) + rows * nq : 0;
-  double2* mean = static_cast<double2*>(workspace(WS_SHARED + slot_offset, szc * sizeof(double2) + nsz * sizeof(float2)));
-  char* vec = static_cast<char*>(workspace(
-      WS_SHARED_VEC + slot_offset, tiles ? shared_tile_workspace(s) * sizeof(double2) : large_vectors(a, gb, N, c64)));
-  const size_t ints = gb * N + NUM_XCD + items + 64;
-  char* st = static_cast<char*>(workspace(WS_SHARED_STATE + slot_offset, (tiles ? 0 : large_state(gb, N)) + ints * sizeof(int)));
-  if (!mean || !vec || !st) return -2;
+  double2* mean = nullptr;
+  char *vec = nullptr, *st = nullptr;
+  for (;; gb = (gb + 1) / 2) {
+    s.groups = static_cast<int>(gb);
+    const size_t szc = rows + rows * nq + vsz + dvsz + gb * ((nn + pk) * 2 + n * T + shared_inverse_workspace(n));
+    const size_t nsz = c64 ? shared_narrow_p(a, gb) + rows * nq : 0;
+    const size_t ints = gb * N + NUM_XCD + items + 64;
+    mean = static_cast<double2*>(workspace(WS_SHARED + slot_offset, szc * sizeof(double2) + nsz * sizeof(float2)));
+    vec = static_cast<char*>(workspace(
+        WS_SHARED_VEC + slot_offset, tiles ? shared_tile_workspace(s) * sizeof(double2) : large_vectors(a, gb, N, c64)));
+    st = static_cast<char*>(workspace(WS_SHARED_STATE + slot_offset, (tiles ? 0 : large_state(gb, N)) + ints * sizeof(int)));
+    if (mean && vec && st) break;
+    if (gb == 1) return SHARED_NO_SPACE;
+  }
   double2* dd = mean + rows;
   double2* vmean = dd + rows * nq;
   double2* dv = vmean + vsz;

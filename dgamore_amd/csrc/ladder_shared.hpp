@@ -84,7 +84,9 @@ struct SharedGroups {
 
 // DGAMI_LADDER_SHARED = 0 / 1: never / wherever the form can run (for comparisons and tests).
 bool ladder_shared_applies(const LadderArgs& a, int precision);
-// slot_offset: of the workspaces (k WS_STREAM_STRIDE for work on extra stream k).
+// slot_offset: of the workspaces (k WS_STREAM_STRIDE for work on extra stream k). SHARED_NO_SPACE: the device
+// memory holds not even one group of it, and nothing was launched (the caller takes the LU, which may need less).
+constexpr int SHARED_NO_SPACE = -3;
 int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, int slot_offset = 0);
 
 // A batch of n <= SHARED_TILE_N, to the output and the columns' state, with z0 = P B. pack: space for two

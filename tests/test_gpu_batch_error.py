@@ -33,24 +33,24 @@ def test_streams_are_joined_when_a_model_fails(monkeypatch):
     from dgamore_amd import kernels as K
 
     monkeypatch.setenv("DGAMI_LADDER_SHARED", "1")
-    monkeypatch.setenv("DGAMI_LADDER_STREAMS", "3")
-    print("[gpu-case] batch of shared-form models, the last beyond the device's memory", flush=True)
+    monkeypatch.setenv("DGAMI_LADDER_STREAMS", "2")
+    print("[gpu-case] batch of two shared-form models and three that are refused", flush=True)
     nb, niv, nw, nq = 1, 60, 61, 900
     chi0_inv, gamma, u, _, beta = ladder_case(nb, niv, nw - 1, 6, seed=2, with_v=False)
     ci = K.ref4_to_qf(K.to_dev(chi0_inv)).repeat(1, 1, 1, nq // 6).contiguous()
     g, um = K.vertex_to_cmp(K.to_dev(gamma))[None].contiguous(), K.orb_to_m(K.to_dev(u))[None].contiguous()
     ref, _ = K.ladder_solve_sum(ci, g, um, None, beta)
-    # one model per stream; the workspace of the last (2^29 q-points of n = 120) is refused by the allocator before
-    # anything of it is launched, and the caller's stream copies the others' results next
+    # one shared-form model per stream; three more, register-kernel models of 2^30 - 1 problems each, are refused
+    # together after that, before any of them is launched; the caller's stream copies the others' results next
     outs = [torch.zeros_like(ref) for _ in range(2)]
     infos = [torch.zeros((1, nw, nq), dtype=torch.int32, device="cuda") for _ in range(2)]
-    table = (_lib.LadderModel * 3)()
-    for m in range(3):
-        k, q, w = min(m, 1), (1 << 29 if m == 2 else nq), (1 if m == 2 else nw)
-        table[m] = _lib.LadderModel(1, q, nb, w, niv, beta, K._p(ci), K._p(g), K._p(um), None, K._p(outs[k]),
-                                    K._p(infos[k], torch.int32))
-    with pytest.raises(RuntimeError):
-        _lib.call("dgami_ladder_solve_sum_multi", 3, ctypes.addressof(table), K._stream())
+    table = (_lib.LadderModel * 5)()
+    for m in range(5):
+        k, big = min(m, 1), m >= 2
+        table[m] = _lib.LadderModel(1, 1 if big else nq, nb, (1 << 30) - 1 if big else nw, 1 if big else niv, beta,
+                                    K._p(ci), K._p(g), K._p(um), None, K._p(outs[k]), K._p(infos[k], torch.int32))
+    with pytest.raises(ValueError, match="too many problems in one launch"):
+        _lib.call("dgami_ladder_solve_sum_multi", 5, ctypes.addressof(table), K._stream())
     copies = [o.clone() for o in outs]
     torch.cuda.current_stream().synchronize()
     for c in copies:
