@@ -530,9 +530,10 @@ __global__ void __launch_bounds__(256) blk_vertex32_kernel(LadderArgs a, float2*
   }
 }
 
-template <typename S, int KC, int TM = 64>
+template <typename S, int KC>
 __device__ __forceinline__ void gemm_stage(const S* W, int ld, const GemmRange& g, int rt, int ct, int kc, int kn,
-                                           S (&s_a)[TM][KC + 1], S (&s_b)[KC][65]) {
+                                           S (&s_a)[64][KC + 1], S (&s_b)[KC][65]) {
+  constexpr int TM = 64;
   for (int e = threadIdx.x; e < TM * KC; e += 256) {
     const int r = e / KC, s = e - (e / KC) * KC;
     s_a[r][s] = (rt + r < g.r1 && s < kn) ? W[static_cast<size_t>(rt + r) * ld + g.k0 + kc + s] : czero<S>();
@@ -543,15 +544,14 @@ __device__ __forceinline__ void gemm_stage(const S* W, int ld, const GemmRange& 
   }
 }
 
-// Thread (ty, tx) of the 16x16 layout owns rows ty + 16 i (i < RI) and columns tx + 16 j
-// (j < 4) of a (16 RI) x 64 tile; RI = 8 gives 12 LDS reads per 32 complex FMAs, enough
-// to keep the FP64 pipes busy.
-template <typename S, int KC, int RI, bool FUSED = false>
-__global__ void __launch_bounds__(256) blk_gemm_kernel(BlockedState<S> st, GemmRange g, int nprob) {
-  constexpr int TM = 16 * RI;
+// The complex64 update on the vector units (DGAMI_BLOCKED_GEMM=vector): thread (ty, tx) of the 16x16 layout
+// owns rows ty + 16 i and columns tx + 16 j of a 64 x 64 tile.
+template <int KC, bool FUSED = false>
+__global__ void __launch_bounds__(256) blk_gemm_kernel(BlockedState<float2> st, GemmRange g, int nprob) {
+  typedef float2 S;
+  constexpr int RI = 4, TM = 16 * RI;
   int b, t;
   if (!xcd_tile(blockIdx.x, nprob, g.tiles_r * g.tiles_c, b, t)) return;
-  if (ladder_idle(st.src, st.item0 + b)) return;
   const int tr = t / g.tiles_c, tcl = t - (t / g.tiles_c) * g.tiles_c;
   const int ld = st.ld;
   S* W = st.W + static_cast<size_t>(b) * st.n * ld;
@@ -584,7 +584,7 @@ __global__ void __launch_bounds__(256) blk_gemm_kernel(BlockedState<S> st, GemmR
   for (int kc = 0; kc < g.kw; kc += KC) {
     const int kn = min(KC, g.kw - kc);
     if (kc > 0) __syncthreads();
-    gemm_stage<S, KC, TM>(W, ld, g, rt, ct, kc, kn, s_a, s_b);
+    gemm_stage<S, KC>(W, ld, g, rt, ct, kc, kn, s_a, s_b);
     __syncthreads();
 #pragma unroll 2
     for (int s2 = 0; s2 < KC; ++s2) {
@@ -714,7 +714,6 @@ __global__ void __launch_bounds__(256) blk_gemm_mfma_kernel(BlockedState<float2>
   typedef float V4 __attribute__((ext_vector_type(4)));
   int b, t;
   if (!xcd_tile(blockIdx.x, nprob, g.tiles_r * g.tiles_c, b, t)) return;
-  if (ladder_idle(st.src, st.item0 + b)) return;
   const int tr = t / g.tiles_c, tcl = t - (t / g.tiles_c) * g.tiles_c;
   const int ld = st.ld;
   float2* W = st.W + static_cast<size_t>(b) * st.n * ld;
@@ -824,7 +823,6 @@ __global__ void __launch_bounds__(256) blk_gemm_bf16x3_kernel(BlockedState<float
   constexpr int KR = 2 * KC + 8;  // bf16 per staged row (interleaved re/im, padded)
   int b, t;
   if (!xcd_tile(blockIdx.x, nprob, g.tiles_r * g.tiles_c, b, t)) return;
-  if (ladder_idle(st.src, st.item0 + b)) return;
   const int tr = t / g.tiles_c, tcl = t - (t / g.tiles_c) * g.tiles_c;
   const int ld = st.ld;
   float2* W = st.W + static_cast<size_t>(b) * st.n * ld;
@@ -1111,9 +1109,9 @@ struct BlockedSteps {
         }
       } else {
         if (fused)
-          hipLaunchKernelGGL((blk_gemm_kernel<S, 32, 4, true>), gd, dim3(256), 0, stream, st, g, nb);
+          hipLaunchKernelGGL((blk_gemm_kernel<32, true>), gd, dim3(256), 0, stream, st, g, nb);
         else
-          hipLaunchKernelGGL((blk_gemm_kernel<S, 32, 4>), gd, dim3(256), 0, stream, st, g, nb);
+          hipLaunchKernelGGL((blk_gemm_kernel<32>), gd, dim3(256), 0, stream, st, g, nb);
       }
     } else if constexpr (std::is_same<S, float2>::value) {
       if (mode == BLK_GEMM_BF16X3) {

@@ -23,8 +23,9 @@ struct LadderArgs {
   // CHI0INV / VERTEX right-hand sides restricted to the columns (c, v') with v' in
   // [rhs_vlo, rhs_vlo + rhs_w) for every orbital pair c (rhs_w = 0: every column)
   int rhs_vlo = 0, rhs_w = 0;
-  // LU of a subset: work index k < *nitems stands for problem items[k]; kernels launched for more
-  // problems than the device count return at once (null: every problem, k itself)
+  // LU of a subset (column kernel and complex128 blocked LU): work index k < *nitems stands for problem
+  // items[k]; kernels launched for more problems than the device count return at once (null: every problem,
+  // k itself)
   const int* items = nullptr;
   const int* nitems = nullptr;
 };

@@ -278,8 +278,7 @@ __device__ __forceinline__ void ladder_reg_solve(const LadderArgs& a, int item) 
 
 template <int TR, int TC, int RPT, int CPT>
 __global__ void __launch_bounds__(TR* TC) ladder_reg_kernel(LadderArgs a) {
-  if (ladder_idle(a, blockIdx.x)) return;
-  ladder_reg_solve<TR, TC, RPT, CPT>(a, ladder_item(a, blockIdx.x));
+  ladder_reg_solve<TR, TC, RPT, CPT>(a, blockIdx.x);
 }
 
 // Several models in one launch: workgroup b solves item b - start[m] of the model m with

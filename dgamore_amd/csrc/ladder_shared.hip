@@ -676,8 +676,8 @@ bool ladder_shared_applies(const LadderArgs& a, int precision) {
   if (v && *v) return std::string(v) == "1";
   if (a.nq < SHARED_MIN_NQ) return false;
   const double ratio = a.n / (3.0 * a.T) + 1.0, work = static_cast<double>(a.nchan) * a.nw * a.nq * ratio;
-  if (a.n <= 32) return work >= SHARED_MIN_WORK_N32 && a.T <= 4;
-  if (a.n <= SHARED_TILE_N && a.T <= 4)
+  if (a.n <= 32) return work >= SHARED_MIN_WORK_N32 && a.T <= SHARED_TILE_T;
+  if (a.n <= SHARED_TILE_N && a.T <= SHARED_TILE_T)
     return work >= (a.T == 1 ? SHARED_MIN_WORK_1 : SHARED_MIN_WORK_4)[a.n <= 64 ? 0 : a.n <= 128 ? 1 : 2];
   return precision == DGAMI_PLAIN_FP64 ? ratio >= SHARED_MIN_RATIO && work >= SHARED_MIN_WORK
                                        : ratio >= SHARED_MIN_RATIO_MIXED && work >= SHARED_MIN_WORK_MIXED;
@@ -763,7 +763,7 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
   const int n = a.n, T = a.T, nq = a.nq, TT = T * T, N = nq * T;
   const size_t G = static_cast<size_t>(a.nchan) * a.nw, nn = static_cast<size_t>(n) * n;
   const size_t items = G * nq;
-  const bool tiles = n <= SHARED_TILE_N;
+  const bool tiles = n <= SHARED_TILE_N && T <= SHARED_TILE_T;
   const bool c64 = !tiles && precision != DGAMI_PLAIN_FP64;
   const size_t pk = tiles ? shared_packed(n) : 0;
   // groups per batch: matrices and, for large sizes, vectors of at most 24 GiB, fewer where the device holds less

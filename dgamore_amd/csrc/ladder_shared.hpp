@@ -36,7 +36,7 @@ constexpr double SHARED_MIN_WORK_4[3] = {9000.0, 13500.0, 30000.0};
 // the large form: with a small ratio the passes over the basis and the D(q) blocks, which grow with T, weigh more
 constexpr double SHARED_MIN_WORK = 65000.0, SHARED_MIN_WORK_MIXED = 45000.0;
 constexpr double SHARED_MIN_RATIO = 18.0, SHARED_MIN_RATIO_MIXED = 24.0;
-constexpr int SHARED_TILE_N = 256;
+constexpr int SHARED_TILE_N = 256, SHARED_TILE_T = 4;  // of the form in tiles
 
 constexpr int SH_M = 10;           // Krylov vectors of a cycle
 constexpr int SH_ROT = SH_M * (SH_M + 1) / 2;
@@ -89,7 +89,7 @@ bool ladder_shared_applies(const LadderArgs& a, int precision);
 constexpr int SHARED_NO_SPACE = -3;
 int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, int slot_offset = 0);
 
-// A batch of n <= SHARED_TILE_N, to the output and the columns' state, with z0 = P B. pack: space for two
+// A batch of n <= SHARED_TILE_N and T <= SHARED_TILE_T, to the output and the columns' state, with z0 = P B. pack: space for two
 // packed matrices per group (shared_packed); next: NUM_XCD integers.
 size_t shared_packed(int n);
 size_t shared_tile_workspace(const SharedGroups& s);

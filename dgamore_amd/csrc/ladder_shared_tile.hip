@@ -1,4 +1,5 @@
-// Ladder sums through the groups' shared matrix (ladder_shared.hip) for compound sizes up to 256.
+// Ladder sums through the groups' shared matrix (ladder_shared.hip) for compound sizes up to 256 of one
+// and two orbitals (the LU is faster for more of them at these sizes).
 //
 // Columns are independent, so one workgroup takes a tile of 16 columns of a group through the whole
 // solution (products, orthogonalisation, cycles, output) without any other workgroup: one launch, and
@@ -197,7 +198,7 @@ __device__ __forceinline__ void shared_apply(const SharedGroups& s, SharedLds<H>
     for (int c = 0; c < T; ++c) y[c] = v[(c * nv + vi) * NC + x.c];
     const double2* d = x.dd + static_cast<size_t>(vi) * nq;
     const size_t blk = static_cast<size_t>(nv) * nq;
-    constexpr int RU = T == 9 ? 3 : T == 4 ? 4 : 1;
+    constexpr int RU = T == 4 ? 4 : 1;
 #pragma unroll RU
     for (int r = 0; r < T; ++r) {
       double2 acc = make_double2(0.0, 0.0);
@@ -535,12 +536,7 @@ int shared_tile_solve(const SharedGroups& s, double2* pack, double2* z0, double2
                      pack, z0, next);
   DGAMI_HIP_CHECK(hipGetLastError());
   const SharedTileArgs ta{s, pack, pack + pk * s.groups, static_cast<int>(ceil_div(s.N, 16)), vec, next};
-  switch (s.a.T) {
-    case 1: return tile_launch_t<1>(ta, stream);
-    case 4: return tile_launch_t<4>(ta, stream);
-    case 9: return tile_launch_t<9>(ta, stream);
-    default: return tile_launch_t<16>(ta, stream);
-  }
+  return s.a.T == 1 ? tile_launch_t<1>(ta, stream) : tile_launch_t<4>(ta, stream);
 }
 
 }  // namespace dgami
