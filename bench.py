@@ -538,7 +538,8 @@ def dominant_kernel(pipe, stream, ms_ladder, precision_name):
     of the operands and the result. Both are matrix-core work, so the bound is the matrix-core peak
     of the precision (split-BF16: the BF16 peak / 3 products). `traffic` is the HBM bytes per launch measured with
     rocprofv3 FETCH_SIZE / WRITE_SIZE (profiles/trailing_update_traffic.txt).
-    Smaller sizes run one kernel for the solve, timed as the whole ladder call in LU flops.
+    Smaller sizes run one kernel for the solve, timed as the whole ladder call: the register LU in its flops, the
+    tiles of the shared-matrix form as a time alone.
     """
     import torch
 
@@ -573,11 +574,13 @@ def dominant_kernel(pipe, stream, ms_ladder, precision_name):
     # and, unless the whole run is on one stream, the launches as the default two lanes run them
     prof2 = None if os.environ.get("DGAMI_LADDER_STREAMS") == "1" else profiled(2)
     if prof["launches"] == 0:
+        if takes_shared_form(pipe):  # its operations depend on the data: no rate to hold against a peak
+            return {"bound": "mfma", "kernel": "tiles of the shared-matrix form", "achieved": None, "peak": peak_tf,
+                    "unit": "TFLOP/s", "frac": None, "traffic": None, "launches": 1, "avg_launch_ms": ms_ladder}
         flops = pipe.solves_per_step() * pipe.ladder_flops_per_solve()
         tf = flops / (ms_ladder * 1e-3) / 1e12
-        return {"bound": "mfma", "kernel": "ladder kernel of one launch (register LU, or tiles of the shared-matrix form), in LU flops",
-                "achieved": tf, "peak": peak_tf, "unit": "TFLOP/s", "frac": tf / peak_tf, "traffic": None,
-                "launches": 1, "avg_launch_ms": ms_ladder}
+        return {"bound": "mfma", "kernel": "register LU", "achieved": tf, "peak": peak_tf, "unit": "TFLOP/s",
+                "frac": tf / peak_tf, "traffic": None, "launches": 1, "avg_launch_ms": ms_ladder}
     avg_ms = prof["ms"] / prof["launches"]
     tf = prof["flops"] / (prof["ms"] * 1e-3) / 1e12
     gbs = prof["bytes"] / (prof["ms"] * 1e-3) / 1e9
@@ -601,6 +604,28 @@ def dominant_kernel(pipe, stream, ms_ladder, precision_name):
             "measured_with": "the ladder on one stream (DGAMI_LADDER_STREAMS=1); the timed steps use two",
             "two_lanes": None if prof2 is None else {"launches": prof2["launches"],
                                                      "avg_launch_ms": prof2["ms"] / max(1, prof2["launches"])}}
+
+
+def takes_shared_form(pipe):
+    """Whether the ladder call goes through the q-points' shared matrix: its last bits then differ from the LU's."""
+    import torch
+
+    from dgamore_amd import kernels as K
+
+    def solve():
+        return K.ladder_solve_sum(pipe.last["chi0_inv"], pipe.gamma, pipe.u_r, pipe.v_r, pipe.m.beta, pipe.precision,
+                                  check_info=False)[0]
+
+    old = os.environ.get("DGAMI_LADDER_SHARED")
+    own = solve()
+    os.environ["DGAMI_LADDER_SHARED"] = "0"
+    try:
+        return not torch.equal(own, solve())
+    finally:
+        if old is None:
+            os.environ.pop("DGAMI_LADDER_SHARED", None)
+        else:
+            os.environ["DGAMI_LADDER_SHARED"] = old
 
 
 def ladder_algorithmic_bytes(pipe):
@@ -672,7 +697,8 @@ def main():
     ms_sigma = time_sigma(pipe, max(2, args.steps), stream)
     roof = dominant_kernel(pipe, stream, ms_ladder, args.precision)
     print(f"[bench] {args.precision}: Sigma sum {ms_sigma:.3f} ms; dominant kernel {roof['kernel']}: "
-          f"{roof['launches']} launches, {roof['avg_launch_ms']:.3f} ms avg, {roof['frac']:.3f} of {roof['bound']} peak",
+          f"{roof['launches']} launches, {roof['avg_launch_ms']:.3f} ms avg"
+          + ("" if roof["frac"] is None else f", {roof['frac']:.3f} of {roof['bound']} peak"),
           file=sys.stderr, flush=True)
 
     compare = None
@@ -727,8 +753,9 @@ def main():
         "ladder_ms": ms_ladder,
         "ladder_solves_per_s": solves / (ms_ladder * 1e-3),
         "ladder_roofline": {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
-                            "frac": achieved / peak, "flops_per_solve": pipe.ladder_flops_per_solve(),
-                            "flops_counted": "those of one LU per problem (the shared-matrix form needs fewer)"},
+                            "frac": None if takes_shared_form(pipe) else achieved / peak,
+                            "flops_per_solve": pipe.ladder_flops_per_solve(),
+                            "flops_counted": "those of one LU per problem (the shared-matrix form needs fewer: no frac)"},
         "ladder_traffic": None if roof.get("traffic") is None or "shared" in roof["kernel"] else {
             "trailing_update_GB_per_call": roof["traffic"] * roof["launches"] / 1e9,
             "algorithmic_GB_per_call": ladder_algorithmic_bytes(pipe) / 1e9,
