@@ -18,7 +18,8 @@
 // 80 ms in complex128, 40 in split BF16 (LU: 235 and 94). Every column has its own Hessenberg matrix and
 // status on the device; tiles of 64 columns (SH_TN) without an active column are skipped by the
 // products and the basis kernels, and no value is read by the host, so a call can be captured.
-// Problems with a column that does not converge (a singular or nearly singular A(q), a NaN) are
+// Problems with a column that does not converge (a singular or nearly singular A(q), a NaN), and those of a
+// group whose matrices may be singular in a way that the right-hand sides do not show (shared_equal_rows), are
 // collected on the device and solved by the LU with partial pivoting, whose info they report.
 #include <algorithm>
 #include <cstdlib>
@@ -104,20 +105,31 @@ __global__ void __launch_bounds__(256) shared_narrow_kernel(const double2* __res
 }
 
 // ---------------------------------------------------------------------------
-// D(q) = chi0^-1(q) - mean over q and the mean, one wavefront per (w, block, v).
+// D(q) = chi0^-1(q) - mean over q and the mean, one wavefront per (w, block, v); zero [nw][T][nv]: whether an element
+// of a diagonal block vanishes.
 __global__ void __launch_bounds__(256) shared_mean_kernel(const double2* __restrict__ ci, double2* __restrict__ mean,
-                                                          double2* __restrict__ dd, int rows, int nq,
-                                                          int* __restrict__ count) {
+                                                          double2* __restrict__ dd, int rows, int nq, int T, int nv,
+                                                          int* __restrict__ zero, int* __restrict__ count) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // of the unconverged problems
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= rows) return;
   const double2* src = ci + static_cast<size_t>(row) * nq;
   double2 s = make_double2(0.0, 0.0);
-  for (int q = lane; q < nq; q += 64) s = cadd(s, src[q]);
+  bool none = false;
+  for (int q = lane; q < nq; q += 64) {
+    const double2 x = src[q];
+    s = cadd(s, x);
+    none |= x.x == 0.0 && x.y == 0.0;
+  }
   for (int o = 32; o > 0; o >>= 1) s = cadd(s, make_double2(__shfl_xor(s.x, o), __shfl_xor(s.y, o)));
   s = cscale(s, 1.0 / nq);
   for (int q = lane; q < nq; q += 64) dd[static_cast<size_t>(row) * nq + q] = csub(src[q], s);
-  if (lane == 0) mean[row] = s;
+  const bool any = __any(none);
+  if (lane == 0) {
+    mean[row] = s;
+    const int blk = row / nv % (T * T), c = blk / T;
+    if (blk == c * T + c) zero[(row / nv / (T * T) * T + c) * nv + row % nv] = any;
+  }
 }
 
 // The same for V_r [nchan][nq][T*T]: one wavefront per (chan, block); dv is scaled by 1 / beta^2.
@@ -135,9 +147,17 @@ __global__ void __launch_bounds__(64) shared_vmean_kernel(LadderArgs a, double2*
   if (lane == 0) mean[blockIdx.x] = s;
 }
 
-// z0 = P B: sums of P over the frequencies of every orbital pair. One wavefront per (group, row).
-__global__ void __launch_bounds__(256) shared_rhs_kernel(const double2* __restrict__ P, double2* __restrict__ z0, int rows,
-                                                         int n, int T, int nv) {
+// z0 = P B: sums of P over the frequencies of every orbital pair. One wavefront per (group, row); in the last
+// s.groups workgroups the look for equal rows of the groups (n uint4 of LDS).
+__global__ void __launch_bounds__(256) shared_rhs_kernel(SharedGroups s, double2* __restrict__ z0) {
+  const int n = s.a.n, T = s.a.T, nv = s.a.nv, rows = s.groups * n, grp = blockIdx.x - (gridDim.x - s.groups);
+  if (grp >= 0) {
+    extern __shared__ uint4 s_hash[];
+    const bool equal = shared_equal_rows(s, grp, s_hash);
+    if (threadIdx.x == 0) s.equal[grp] = equal;
+    return;
+  }
+  const double2* P = s.P;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= rows) return;
   for (int t = 0; t < T; ++t) {
@@ -550,6 +570,7 @@ __global__ void __launch_bounds__(256) shared_collect_kernel(SharedGroups s, int
   if (i >= s.groups * s.a.nq) return;
   bool bad = false;
   for (int t = 0; t < T; ++t) bad |= s.state[static_cast<size_t>(i) * T + t] != SH_DONE;
+  bad |= s.equal[i / s.a.nq] != 0;
   const int item = s.group0 * s.a.nq + i;
   if (bad)
     list[atomicAdd(count, 1)] = item;
@@ -781,7 +802,7 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
     s.groups = static_cast<int>(gb);
     const size_t szc = rows + rows * nq + vsz + dvsz + gb * ((nn + pk) * 2 + n * T + shared_inverse_workspace(n));
     const size_t nsz = c64 ? shared_narrow_p(a, gb) + rows * nq : 0;
-    const size_t ints = gb * N + NUM_XCD + items + 64;
+    const size_t ints = gb * N + NUM_XCD + items + 1 + gb + static_cast<size_t>(a.nw) * n;
     mean = static_cast<double2*>(workspace(WS_SHARED + slot_offset, szc * sizeof(double2) + nsz * sizeof(float2)));
     vec = static_cast<char*>(workspace(
         WS_SHARED_VEC + slot_offset, tiles ? shared_tile_workspace(s) * sizeof(double2) : large_vectors(a, gb, N, c64)));
@@ -808,9 +829,12 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
   int* next = s.state + gb * N;
   int* list = next + NUM_XCD;
   int* count = list + items;
+  s.equal = count + 1;
+  int* zero = s.equal + gb;
+  s.zero = zero;
 
   hipLaunchKernelGGL(shared_mean_kernel, dim3(ceil_div(rows, 4)), dim3(256), 0, stream, a.chi0_inv, mean, dd,
-                     static_cast<int>(rows), nq, count);
+                     static_cast<int>(rows), nq, T, a.nv, zero, count);
   DGAMI_HIP_CHECK(hipGetLastError());
   if (a.v_r) {
     hipLaunchKernelGGL(shared_vmean_kernel, dim3(static_cast<unsigned>(vsz)), dim3(64), 0, stream, a, vmean, dv);
@@ -830,8 +854,8 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
     if (tiles) {
       rc = shared_tile_solve(s, pack, z0, reinterpret_cast<double2*>(vec), next, stream);
     } else {
-      hipLaunchKernelGGL(shared_rhs_kernel, dim3(ceil_div(static_cast<size_t>(ng) * n, 4)), dim3(256), 0, stream, P, z0,
-                         ng * n, n, T, a.nv);
+      hipLaunchKernelGGL(shared_rhs_kernel, dim3(ceil_div(static_cast<size_t>(ng) * n, 4) + ng), dim3(256),
+                         n * sizeof(uint4), stream, s, z0);
       DGAMI_HIP_CHECK(hipGetLastError());
       rc = c64 ? shared_large_solve<float2>(s, vec, st, narrow, ds, precision == DGAMI_MIXED_BF16X3_IR, stream)
                : shared_large_solve<double2>(s, vec, st, nullptr, nullptr, false, stream);

@@ -80,7 +80,45 @@ struct SharedGroups {
   const double2* dv;      // (V_r(q) - mean V_r) / beta^2: [nchan][nq][T*T], or null
   const double2* z0;      // P B [groups][n][T]
   int* state;             // [groups][N] SharedState
+  const int* zero;        // [nw][T][nv] whether chi0^-1 vanishes on the block's diagonal for some q
+  int* equal;             // [groups] whether a matrix of the group may have two equal rows
 };
+
+// Whether some A(q) of a group may have two equal rows of one orbital pair: such a matrix is singular, but its
+// right-hand sides are equal there too, so the iteration would solve it where the LU reports the zero pivot
+// (collected problems go to the LU). Rows (c, a) and (c, b) can only be equal if those of the vertex are in every
+// column but those of the frequencies a and b; four columns are compared (as hashes in LDS, [n][4]), which
+// tells any two rows of a real vertex apart. Where they and the columns a and b of the pair agree (a vertex
+// that is constant there), A(q) has equal rows if chi0^-1 vanishes in both; otherwise it has them if chi0^-1 makes
+// up for the difference, which is left to the LU to find out. All 256 threads of a workgroup call it; it runs
+// beside the packing (4 us at n = 40, with or without it).
+__device__ inline bool shared_equal_rows(const SharedGroups& s, int grp, uint4* hash) {
+  const int n = s.a.n, T = s.a.T, nv = s.a.nv;
+  const double2* G = s.a.gamma + static_cast<size_t>(s.group0 + grp) * n * n;
+  const int* zero = s.zero + static_cast<size_t>((s.group0 + grp) % s.a.nw) * n;
+  unsigned* words = reinterpret_cast<unsigned*>(hash);
+  for (int e = threadIdx.x; e < 4 * n; e += 256) {
+    const int row = e >> 2, col = row / nv * nv + (e & 3) * nv / 4;
+    const double2 x = G[static_cast<size_t>(row) * n + col];
+    const unsigned long long re = __double_as_longlong(x.x + 0.0), im = __double_as_longlong(x.y + 0.0);  // -0 = 0
+    words[e] = static_cast<unsigned>(re ^ (re >> 32)) * 0x9e3779b1u + static_cast<unsigned>(im ^ (im >> 32)) * 0x85ebca77u;
+  }
+  __syncthreads();
+  int found = 0;
+  for (int e = threadIdx.x; e < T * nv * nv; e += 256) {
+    const int ra = e / nv, b = e - ra * nv, c = ra / nv, a = ra - c * nv, rb = c * nv + b;
+    if (a >= b) continue;
+    const uint4 ha = hash[ra], hb = hash[rb];
+    auto same = [&](unsigned x, unsigned y, int v) { return x == y || v == a || v == b; };
+    if (!(same(ha.x, hb.x, 0) && same(ha.y, hb.y, nv / 4) && same(ha.z, hb.z, nv / 2) && same(ha.w, hb.w, 3 * nv / 4)))
+      continue;
+    const double2* A = G + static_cast<size_t>(ra) * n + c * nv;
+    const double2* B = G + static_cast<size_t>(rb) * n + c * nv;
+    const bool constant = A[a].x == B[a].x && A[a].y == B[a].y && A[b].x == B[b].x && A[b].y == B[b].y;
+    found |= !constant || (zero[ra] && zero[rb]);
+  }
+  return __syncthreads_or(found) != 0;
+}
 
 // DGAMI_LADDER_SHARED = 0 / 1: never / wherever the form can run (for comparisons and tests).
 bool ladder_shared_applies(const LadderArgs& a, int precision);

@@ -69,8 +69,8 @@ __host__ __device__ inline int shared_blocks(int n) { return 2 * ((n + 31) / 32)
 __host__ __device__ inline int shared_steps(int n) { return (n + 3) / 4; }
 size_t shared_packed(int n) { return static_cast<size_t>(shared_blocks(n)) * shared_steps(n) * 64; }
 
-// Both matrices packed, z0 = P B (sums of P over the frequencies of every orbital pair), and the tile
-// counters cleared. grid (2 ceil(packed / 256) + ceil(n / 4), groups).
+// Both matrices packed, z0 = P B (sums of P over the frequencies of every orbital pair), the tile counters
+// cleared, and the look for equal rows. grid (2 ceil(packed / 256) + ceil(n / 4) + 1, groups), n uint4 of LDS.
 __global__ void __launch_bounds__(256) shared_pack_kernel(SharedGroups s, double2* __restrict__ out, double2* __restrict__ z0,
                                                           int* __restrict__ next) {
   const int n = s.a.n, T = s.a.T, nv = s.a.nv, nk = shared_steps(n);
@@ -79,6 +79,12 @@ __global__ void __launch_bounds__(256) shared_pack_kernel(SharedGroups s, double
   const size_t mat = blockIdx.y * static_cast<size_t>(n) * n;
   const int lane = threadIdx.x & 63;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < NUM_XCD) next[threadIdx.x] = 0;
+  if (blockIdx.x == gridDim.x - 1) {
+    extern __shared__ uint4 s_hash[];
+    const bool equal = shared_equal_rows(s, blockIdx.y, s_hash);
+    if (threadIdx.x == 0) s.equal[blockIdx.y] = equal;
+    return;
+  }
   if (blockIdx.x < 2 * nb) {
     const bool inv = blockIdx.x >= nb;
     const size_t e = (blockIdx.x - (inv ? nb : 0)) * static_cast<size_t>(256) + threadIdx.x;
@@ -532,8 +538,8 @@ static int tile_launch_t(const SharedTileArgs& ta, hipStream_t stream) {
 int shared_tile_solve(const SharedGroups& s, double2* pack, double2* z0, double2* vec, int* next, hipStream_t stream) {
   const int n = s.a.n;
   const size_t pk = shared_packed(n);
-  hipLaunchKernelGGL(shared_pack_kernel, dim3(2 * ceil_div(pk, 256) + ceil_div(n, 4), s.groups), dim3(256), 0, stream, s,
-                     pack, z0, next);
+  hipLaunchKernelGGL(shared_pack_kernel, dim3(2 * ceil_div(pk, 256) + ceil_div(n, 4) + 1, s.groups), dim3(256),
+                     n * sizeof(uint4), stream, s, pack, z0, next);
   DGAMI_HIP_CHECK(hipGetLastError());
   const SharedTileArgs ta{s, pack, pack + pk * s.groups, static_cast<int>(ceil_div(s.N, 16)), vec, next};
   return s.a.T == 1 ? tile_launch_t<1>(ta, stream) : tile_launch_t<4>(ta, stream);
