@@ -865,8 +865,10 @@ int ladder_solve_shared(const LadderArgs& a, int precision, hipStream_t stream, 
                        count);
     DGAMI_HIP_CHECK(hipGetLastError());
   }
-  // the problems that did not converge, by the LU: its kernels are launched for every problem and
-  // return at once beyond the device count
+  // The problems that did not converge, by the LU: its kernels are launched for every problem and return at once
+  // beyond the device count. Up to n = 128 the column kernel, whose one launch costs 4 us where the list is empty
+  // (the blocked LU's twenty about 90), though it is slower where all problems fail: with the cycles before it
+  // 1890 problems of n = 40 take 0.93 ms (LU alone 0.29; with the register kernel 0.86), 6426 of n = 120 10.9 (3.8).
   LadderArgs f = a;
   f.items = list;
   f.nitems = count;

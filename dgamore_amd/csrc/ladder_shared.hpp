@@ -13,7 +13,7 @@ namespace dgami {
 // data, this form's does: the matrices of a self-consistency loop are harder than those of its first iteration, 10 ... 18
 // iterations per column there, 14 ... 35 at the eighth. The lines lie where the first eight iterations of a loop
 // (mixing 0.3) take this form no longer than the LU, in the geometric mean over a strong and a weak interaction,
-// within 3%. That leaves the last of them slower near a line (by up to 1.9 times) and faster from about twice the
+// within 3%. That leaves the last of them slower near a line (by up to 1.7 times) and faster from about twice the
 // bound on; a single first iteration gains 1.2 ... 3 times everywhere above.
 // Measured: problems, work: LU / mean of the eight, and LU / the first and the last, strong and weak interaction.
 // T = 1, n = 30: 1890, 20790: 0.82; 2790, 30690: 1.07 (1.59 0.96, 1.24 0.82). n = 40: 1440, 20640: 0.81;
@@ -88,10 +88,10 @@ struct SharedGroups {
 // right-hand sides are equal there too, so the iteration would solve it where the LU reports the zero pivot
 // (collected problems go to the LU). Rows (c, a) and (c, b) can only be equal if those of the vertex are in every
 // column but those of the frequencies a and b; four columns are compared (as hashes in LDS, [n][4]), which
-// tells any two rows of a real vertex apart. Where they and the columns a and b of the pair agree (a vertex
+// tells any two rows of an actual vertex apart. Where they and the columns a and b of the pair agree (a vertex
 // that is constant there), A(q) has equal rows if chi0^-1 vanishes in both; otherwise it has them if chi0^-1 makes
 // up for the difference, which is left to the LU to find out. All 256 threads of a workgroup call it; it runs
-// beside the packing (4 us at n = 40, with or without it).
+// beside the packing (calls of n = 40, 120, 216 and 720 take the same time with and without it).
 __device__ inline bool shared_equal_rows(const SharedGroups& s, int grp, uint4* hash) {
   const int n = s.a.n, T = s.a.T, nv = s.a.nv;
   const double2* G = s.a.gamma + static_cast<size_t>(s.group0 + grp) * n * n;
